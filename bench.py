@@ -59,8 +59,9 @@ METRIC = "cell-updates/s vs plain FP64 GPU path; p50/p99 job latency at L1 err<1
 #                                  24) + the timestep share of the 429 B timestep/limiter/reset/kick1 part
 #                                  that k_limit does not carry (349)
 #                   48 / act face  CSR 8 + gradient-phase geometry re-read 40
-#   wakeup          16 / act face  CSR 8 + limiter neighbour ids 8
 #   limit_kick      80 / act cell  reset of the extrapolations and kick1
+#                   16 / act face  CSR 8 + limiter neighbour ids 8
+#   wakeup          (the minimum bin of sync_all simulations; none in the model)
 # Sum: 192 N + 1247 N_act + 248 F_act.  FP32-flux contexts store gradients, extrapolations and face
 # records as floats: the same terms at 4-byte widths for those fields (gradients 120 -> 60,
 # extrapolations 40 -> 20, records 56 -> 28), i.e. 116 N + 1087 N_act + 192 F_act (+8 F_act periodic).
@@ -69,8 +70,8 @@ ALGO = {
     "flux": lambda n_act, f_act, n_all: 329 * n_act + 120 * f_act,
     "apply_c2p": lambda n_act, f_act, n_all: 281 * n_act + 64 * f_act,
     "grad_timestep": lambda n_act, f_act, n_all: 557 * n_act + 48 * f_act,
-    "wakeup": lambda n_act, f_act, n_all: 16 * f_act,
-    "limit_kick": lambda n_act, f_act, n_all: 80 * n_act,
+    "wakeup": lambda n_act, f_act, n_all: 0,
+    "limit_kick": lambda n_act, f_act, n_all: 80 * n_act + 16 * f_act,
 }
 ALGO_FP32 = {
     "mask_predict": lambda n_act, f_act, n_all: 116 * n_all,
@@ -78,7 +79,7 @@ ALGO_FP32 = {
     "apply_c2p": lambda n_act, f_act, n_all: 281 * n_act + 36 * f_act,
     "grad_timestep": lambda n_act, f_act, n_all: 497 * n_act + 48 * f_act,
     "wakeup": ALGO["wakeup"],
-    "limit_kick": lambda n_act, f_act, n_all: 60 * n_act,
+    "limit_kick": lambda n_act, f_act, n_all: 60 * n_act + 16 * f_act,
 }
 PERIODIC_SHIFT = 8  # bytes per active face of a periodic mesh (the flux phase's shift read)
 
@@ -238,8 +239,8 @@ def flux_kernel_name(fp32, solver, static_geometry=True, fpt=1):
             f"{'true' if static_geometry else 'false'}, {fpt or 1}>(hfv::Batch)")
 
 
-SLOT_KERNELS = {"apply_c2p": ["hfv::k_apply(hfv::Batch, int)"], "mask_predict": ["hfv::k_mask(hfv::Batch, int)"],
-                "wakeup": ["hfv::k_wakeup(hfv::Batch, int)"], "limit_kick": ["hfv::k_limit(hfv::Batch, int)"]}
+SLOT_KERNELS = {"apply_c2p": ["hfv::k_apply(hfv::Batch, int)"], "mask_predict": ["void hfv::k_mask<false>(hfv::Batch, int)"],
+                "wakeup": ["hfv::k_sync_min(hfv::Batch)"], "limit_kick": ["hfv::k_limit(hfv::Batch, int)"]}
 
 
 def slot_kernels(slot, fp32, solver, tuning, fpt=1):

@@ -126,13 +126,11 @@ SimEngine fresh_engine(const hfv_params& p) {
   E.t_current = 0.;
   uint64_t between = p.dt_snap > 0. ? sat_u64(p.dt_snap * E.time_base_inv) : HFV_MAX_NR_TIMESTEPS;
   E.between = between ? between : HFV_MAX_NR_TIMESTEPS;
-  E.ti_min = ~0ull;
-  E.min_bin = 127;
   E.chk = 1;  // the first predict checks the primitives the host writes
   return E;
 }
 
-enum { KS_PREDICT = 0, KS_MESH, KS_FLUX, KS_APPLY, KS_GRAD, KS_WAKEUP, KS_LIMIT, KS_DRIFT };
+enum { KS_PREDICT = 0, KS_MESH, KS_FLUX, KS_APPLY, KS_GRAD, KS_SYNC, KS_LIMIT };
 
 // Device memory of hfv_riemann_batch_noalloc, reserved with the code object on every GPU the library
 // runs on (held until the process ends): the Riemann kernel's counters in the first 256 bytes, then the
@@ -206,6 +204,7 @@ struct hfv_ctx {
   bool any_static = false, any_dynamic = false, any_static_grad = false, any_dynamic_grad = false;
   SimDesc* ddesc = nullptr;
   SimEngine* deng = nullptr;
+  SimStep* dst = nullptr;
   SimEngine* heng = nullptr;  // pinned mirror
   DevCounters* dcnt = nullptr;
   DevCounters* hcnt = nullptr;  // pinned
@@ -217,6 +216,7 @@ struct hfv_ctx {
   bool any_vmesh2 = false;  // ... a 2D one
   bool any_vmesh3 = false;  // ... a 3D one
   bool any_moving = false;
+  bool any_sync = false;    // a sync_all simulation
   hipGraph_t graph{};
   hipGraphExec_t gexec{};
   bool graph_ok = false;
@@ -241,6 +241,7 @@ struct hfv_ctx {
     B.F = F;
     B.sims = ddesc;
     B.eng = deng;
+    B.st = dst;
     B.nsims = nslots;
     B.cjobs = dcjobs;
     B.fjobs = dfjobs;
@@ -449,7 +450,7 @@ int alloc_batch(hfv_ctx* c) {
   C.tex = dalloc<double>(c, 5 * n);
   C.tiex = dalloc<uint64_t>(c, n);
   C.bin = dalloc<int8_t>(c, n);
-  C.wake = dalloc<int8_t>(c, n);
+  C.nbin = dalloc<int8_t>(c, n);
   C.act = dalloc<uint8_t>(c, n);
   Faces& F = c->F;
   F.nf = nf;
@@ -507,9 +508,11 @@ int alloc_batch(hfv_ctx* c) {
   c->tune_gstage.assign(S, -1);
   c->ddesc = dalloc<SimDesc>(c, S);
   c->deng = dalloc<SimEngine>(c, S);
+  c->dst = dalloc<SimStep>(c, S);
   for (void* p : c->bufs)
     if (!p) return set_err(HFV_ERR_HIP, "hipMalloc failed");
   hipStream_t st = c->stream;
+  HIP_OK(hipMemsetAsync(c->dst, 0, sizeof(SimStep) * S, st));
   const size_t sd = sizeof(double) * (size_t)n;
   double* dbl[] = {C.prim, C.grad, C.gc, C.extrap, C.cons, C.facc, C.vol, C.loc, C.cen, C.v, C.vrel, C.maor, C.msv, C.dt, C.srad, C.tex};
   int mult[] = {5, 15, 3, HFV_EX_W, 5, 5, 1, 3, 3, 3, 3, 1, 1, 1, 1, 5};
@@ -521,7 +524,7 @@ int alloc_batch(hfv_ctx* c) {
   HIP_OK(hipMemsetAsync(F.floc, 0, 2 * (size_t)std::max<int64_t>(nf, 1), st));
   HIP_OK(hipMemsetAsync(F.gcnt, 0, sizeof(uint16_t) * (size_t)std::max<int64_t>(ncc, 1), st));
   HIP_OK(hipMemsetAsync(C.bin, 0, (size_t)n, st));
-  HIP_OK(hipMemsetAsync(C.wake, 0, (size_t)n, st));
+  HIP_OK(hipMemsetAsync(C.nbin, HFV_NO_BIN, (size_t)n, st));
   HIP_OK(hipMemsetAsync(C.act, 0, (size_t)n, st));
   HIP_OK(hipMemsetAsync(F.cur, 0, (size_t)nf, st));
   HIP_OK(hipMemsetAsync(c->P.act, 0, sizeof(uint32_t) * (size_t)ncc, st));
@@ -591,6 +594,7 @@ void recompute_uniforms(hfv_ctx* c) {
   c->any_vmesh2 = false;
   c->any_vmesh3 = false;
   c->any_moving = false;
+  c->any_sync = false;
   int prec = -1;
   for (int s = 0; s < c->nslots; ++s) {
     if (!c->loaded[s]) continue;
@@ -602,6 +606,7 @@ void recompute_uniforms(hfv_ctx* c) {
     if (p.dim == 2 && p.motion != HFV_FIXED) c->any_vmesh2 = true;
     if (p.dim == 3 && p.motion != HFV_FIXED) c->any_vmesh3 = true;
     if (p.motion != HFV_FIXED) c->any_moving = true;
+    if (p.sync_all) c->any_sync = true;
     if (prec < 0) prec = p.precision;
   }
   c->solver = sol < 0 ? -1 : sol;
@@ -620,16 +625,16 @@ void recompute_uniforms(hfv_ctx* c) {
 struct LaunchSet {
   int solver;
   int precision;
-  bool moving1d, vmesh, vmesh2, vmesh3, moving, st, dyn, sgrad, dgrad;
+  bool moving1d, vmesh, vmesh2, vmesh3, moving, sync, st, dyn, sgrad, dgrad;
   bool operator==(const LaunchSet& o) const {
     return solver == o.solver && precision == o.precision && moving1d == o.moving1d && vmesh == o.vmesh &&
            vmesh2 == o.vmesh2 && vmesh3 == o.vmesh3 &&
-           moving == o.moving &&
+           moving == o.moving && sync == o.sync &&
            st == o.st && dyn == o.dyn && sgrad == o.sgrad && dgrad == o.dgrad;
   }
 };
 LaunchSet launch_set(const hfv_ctx* c) {
-  return LaunchSet{c->solver, c->precision, c->any_moving1d, c->any_vmesh, c->any_vmesh2, c->any_vmesh3, c->any_moving, c->any_static,
+  return LaunchSet{c->solver, c->precision, c->any_moving1d, c->any_vmesh, c->any_vmesh2, c->any_vmesh3, c->any_moving, c->any_sync, c->any_static,
                    c->any_dynamic, c->any_static_grad, c->any_dynamic_grad};
 }
 
@@ -889,7 +894,8 @@ int reset_slot(hfv_ctx* c, int s) {
   for (int k = 0; k < 15; ++k) HIP_OK(hipMemsetAsync((char*)C.grad + es * (k * N + cb), 0, es * cap, st));
   HIP_OK(hipMemsetAsync(C.tiex + cb, 0, sizeof(uint64_t) * cap, st));  // = the fresh engine's ti_pred
   HIP_OK(hipMemsetAsync(C.bin + cb, 0, cap, st));
-  HIP_OK(hipMemsetAsync(C.wake + cb, 0, cap, st));
+  HIP_OK(hipMemsetAsync(C.nbin + cb, HFV_NO_BIN, cap, st));
+  HIP_OK(hipMemsetAsync(c->dst + s, 0, sizeof(SimStep), st));
   HIP_OK(hipMemsetAsync(C.act + cb, 0, cap, st));
   (void)n;
   c->v_zero[s] = 1;
@@ -1053,7 +1059,21 @@ void launch_grad(hfv_ctx* c, const Batch& B, int do_grad, int do_ts) {
   if (c->any_dynamic_grad) hipLaunchKernelGGL(k_grad<false>, g, b, 0, c->stream, B, do_grad, do_ts);
 }
 
-// The kernels of one batch step (k_begin .. k_end).  Timing events only outside graph capture.
+void launch_mask(hfv_ctx* c, const Batch& B, int mode) {
+  const dim3 g((unsigned)c->ncg), b(BLOCK);
+  if (c->any_moving) hipLaunchKernelGGL(k_mask<true>, g, b, 0, c->stream, B, mode);
+  else hipLaunchKernelGGL(k_mask<false>, g, b, 0, c->stream, B, mode);
+}
+
+void launch_sync_min(hfv_ctx* c, const Batch& B) {
+  hipLaunchKernelGGL(k_sync_min, dim3((unsigned)c->ncg), dim3(BLOCK), 0, c->stream, B);
+}
+
+// The limiter of every cell and the end of every slot's step.
+void launch_limit(hfv_ctx* c, const Batch& B, int phase) {
+  hipLaunchKernelGGL(k_limit, dim3((unsigned)(c->nslots + c->ncg)), dim3(BLOCK), 0, c->stream, B, phase);
+}
+
 // Space::volume_calculation on the device for the moving meshes being stepped (1D, 2D and 3D).
 void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
   hipStream_t st = c->stream;
@@ -1091,21 +1111,13 @@ void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
   }
 }
 
+// The kernels of one batch step (k_mask .. k_limit).  Timing events only outside graph capture.
 void enqueue_step(hfv_ctx* c, bool timed) {
   Batch B = c->batch_args();
-  hipStream_t st = c->stream;
-  const unsigned gs = (unsigned)std::max(1, (c->nslots + 63) / 64);
-  const dim3 gc((unsigned)c->ncg), gf((unsigned)c->nfg), gb(BLOCK);
   const bool t = timed && c->prof;
   if (t) prof_next(c);
-  hipLaunchKernelGGL(k_begin, dim3(gs), dim3(64), 0, st, B);
-  if (c->any_moving) {
-    if (t) prof_begin(c, KS_DRIFT);
-    hipLaunchKernelGGL(k_drift, gc, gb, 0, st, B);
-    if (t) prof_end(c, KS_DRIFT);
-  }
   if (t) prof_begin(c, KS_PREDICT);
-  hipLaunchKernelGGL(k_mask, gc, gb, 0, st, B, 0);
+  launch_mask(c, B, 0);
   if (t) prof_end(c, KS_PREDICT);
   if (c->any_moving1d || c->any_vmesh) {
     if (t) prof_begin(c, KS_MESH);
@@ -1116,18 +1128,19 @@ void enqueue_step(hfv_ctx* c, bool timed) {
   launch_flux(c, B);
   if (t) prof_end(c, KS_FLUX);
   if (t) prof_begin(c, KS_APPLY);
-  hipLaunchKernelGGL(k_apply, gc, gb, 0, st, B, 7);
+  hipLaunchKernelGGL(k_apply, dim3((unsigned)c->ncg), dim3(BLOCK), 0, c->stream, B, 7);
   if (t) prof_end(c, KS_APPLY);
   if (t) prof_begin(c, KS_GRAD);
   launch_grad(c, B, 1, 1);
   if (t) prof_end(c, KS_GRAD);
-  if (t) prof_begin(c, KS_WAKEUP);
-  hipLaunchKernelGGL(k_wakeup, gc, gb, 0, st, B, 1);
-  if (t) prof_end(c, KS_WAKEUP);
+  if (c->any_sync) {
+    if (t) prof_begin(c, KS_SYNC);
+    launch_sync_min(c, B);
+    if (t) prof_end(c, KS_SYNC);
+  }
   if (t) prof_begin(c, KS_LIMIT);
-  hipLaunchKernelGGL(k_limit, gc, gb, 0, st, B, 0);
+  launch_limit(c, B, 0);
   if (t) prof_end(c, KS_LIMIT);
-  hipLaunchKernelGGL(k_end, dim3((unsigned)c->nslots), dim3(HFV_END_BLOCK), 0, st, B);
 }
 
 // Rebuild the kept time-extrapolation rates (and the staged simulations' flux records) when the host or a
@@ -1479,7 +1492,7 @@ int hfv_predict(hfv_ctx* c, double dt) {
   E.dt_pred = dt;
   HIP_OK(hipMemcpyAsync(c->deng, &E, sizeof(SimEngine), hipMemcpyHostToDevice, c->stream));
   pack_fr_if_dirty(c);  // predict reads the kept time-extrapolation rates
-  hipLaunchKernelGGL(k_mask, dim3((unsigned)c->ncg), dim3(BLOCK), 0, c->stream, c->batch_args(), 1);
+  launch_mask(c, c->batch_args(), 1);
   HIP_OK(hipGetLastError());
   c->fr_dirty = true;
   return sync_counters(c);
@@ -1491,8 +1504,7 @@ int hfv_compute_fluxes(hfv_ctx* c, const hfv_timestep_info* info) {
   c->last_info = *info;
   TRY(begin_phase_step(c, info, false));
   Batch B = c->batch_args();
-  hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, c->stream, B);
-  hipLaunchKernelGGL(k_mask, dim3((unsigned)c->ncg), dim3(BLOCK), 0, c->stream, B, 2);
+  launch_mask(c, B, 2);
   c->fr_dirty = true;
   pack_fr_if_dirty(c);
   launch_flux(c, B);
@@ -1563,9 +1575,8 @@ int hfv_timesteps(hfv_ctx* c, uint64_t* ti_next) {
   settle(c, -1);
   Batch B = c->batch_args();
   launch_grad(c, B, 0, 1);
-  hipLaunchKernelGGL(k_wakeup, dim3((unsigned)c->ncg), dim3(BLOCK), 0, c->stream, B, 0);
-  hipLaunchKernelGGL(k_limit, dim3((unsigned)c->ncg), dim3(BLOCK), 0, c->stream, B, 1);
-  hipLaunchKernelGGL(k_end, dim3((unsigned)c->nslots), dim3(HFV_END_BLOCK), 0, c->stream, B);
+  if (c->any_sync) launch_sync_min(c, B);
+  launch_limit(c, B, 1);
   HIP_OK(hipGetLastError());
   c->fr_dirty = true;
   TRY(sync_counters(c));
@@ -1600,9 +1611,8 @@ int hfv_apply_timesteps(hfv_ctx* c, const double* dt, uint64_t* ti_next) {
   HIP_OK(hipMemcpyAsync(c->C.dtq + cb, dt, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
   Batch B = c->batch_args();
   hipLaunchKernelGGL(k_ts_apply, dim3((unsigned)c->ncg), dim3(BLOCK), 0, c->stream, B);
-  hipLaunchKernelGGL(k_wakeup, dim3((unsigned)c->ncg), dim3(BLOCK), 0, c->stream, B, 0);
-  hipLaunchKernelGGL(k_limit, dim3((unsigned)c->ncg), dim3(BLOCK), 0, c->stream, B, 1);
-  hipLaunchKernelGGL(k_end, dim3((unsigned)c->nslots), dim3(HFV_END_BLOCK), 0, c->stream, B);
+  if (c->any_sync) launch_sync_min(c, B);
+  launch_limit(c, B, 1);
   HIP_OK(hipGetLastError());
   c->fr_dirty = true;
   TRY(sync_counters(c));
@@ -1718,7 +1728,7 @@ int hfv_step(hfv_ctx* c, const hfv_timestep_info* info, uint64_t* ti_next) {
 }
 
 // ---- engine (src/engine.rs:152-268), device-resident
-// The device engine loops drift generators (k_drift) and rebuild moving meshes in every dimension.
+// The device engine loops drift generators (k_mask) and rebuild moving meshes in every dimension.
 
 int hfv_run(hfv_ctx* c, int64_t max_steps, int64_t* steps_done) {
   TRY(require_mesh(c));
@@ -1820,6 +1830,7 @@ int hfv_batch_unload(hfv_ctx* c, int s) {
   c->heng[s].done = 1;
   c->heng[s].force = 0;
   HIP_OK(hipMemcpyAsync(c->deng + s, c->heng + s, sizeof(SimEngine), hipMemcpyHostToDevice, c->stream));
+  HIP_OK(hipMemsetAsync(c->dst + s, 0, sizeof(SimStep), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   const LaunchSet prev = launch_set(c);
   recompute_uniforms(c);

@@ -6,7 +6,7 @@
 //
 // HBM layout (cells/faces of all simulations concatenated, indices global):
 //   cells, component-major SoA (field[c * N + i]): prim[5], grad[15], gc[3], cons[5], facc[5] (pending
-//     flux accumulator), vol, loc[3], cen[3], v[3], vrel[3], maor, msv, dt, srad, bin (int8), wake
+//     flux accumulator), vol, loc[3], cen[3], v[3], vrel[3], maor, msv, dt, srad, bin (int8), nbin
 //     (int8), act (uint8), tex[5] (time-extrapolation rate of prim, grad and v_rel, written by k_grad
 //     when they change); extrap[N][5] (AoS: read and written whole by predict, staged whole by the flux
 //     kernel)
@@ -25,11 +25,11 @@
 //     kernels.  A block only holds items of one simulation, so configuration and engine loads are
 //     uniform (scalar) and a finished simulation's blocks exit at once.  Blocks are ordered so that
 //     the 8 XCDs (round-robin dispatch) each receive a contiguous range of chunks (L2 locality of the
-//     neighbour gathers).  Per-chunk partial counts replace global atomics; k_end reduces them.
+//     neighbour gathers).  Per-chunk partial counts replace global atomics; step_end reduces them.
 //
-// Step kernels: k_begin (per simulation) -> [k_drift] -> k_mask (cells: active flag, predict) ->
-// [k_mesh1d_*] -> k_flux (faces: gate + flux) -> k_apply (cells: accumulate in CSR order, apply, c2p)
-// -> k_grad (active cells: gradients, limiter, timestep) -> k_wakeup, k_limit (cells) -> k_end (per
+// Step kernels: k_mask (cells: the step from the engine, drift, active flag, predict) -> [rebuild] ->
+// k_flux (faces: gate + flux) -> k_apply (cells: accumulate in CSR order, apply, c2p) -> k_grad (active
+// cells: gradients, limiter, timestep) -> k_limit (cells: wakeup, timestep_limit, kick1; one block per
 // simulation: partial sums, next sync point).
 #pragma once
 #include "hfv_physics.hpp"
@@ -47,7 +47,8 @@ struct Cells {
   double* minv;  // [9][N] inverse of the gradient matrix (static geometry only)
   double* fr;    // [N][HFV_FR_W] flux inputs of static-geometry cells (layout: HFV_FR_*)
   double* dtq;   // [N] requested timesteps of the trait-level compute_timesteps (before timesteps_apply)
-  int8_t *bin, *wake;
+  int8_t* bin;
+  int8_t* nbin;  // the new bin of an active cell between k_grad and k_limit, HFV_NO_BIN for the others
   uint8_t* act;
 };
 
@@ -116,36 +117,46 @@ struct BlockJob {
 };
 
 #define HFV_MAX_SUBDRIFTS 8
+#define HFV_NO_BIN 127  // nbin of a cell that is not active: beyond every wakeup
 #define HFV_NCH_MAX 8
-// Engine of one simulation (src/engine.rs:33-101, 152-268).
+// Engine of one simulation (src/engine.rs:33-101, 152-268).  Between two launches it is the reference's
+// Engine + TimestepInfo.  During a launch it only changes at the end (step_end), apart from nf_mesh: every
+// kernel of the step reads the step's own SimStep.
 struct SimEngine {
   uint64_t ti_old, ti_current, ti_next;
   uint64_t ti_snap, between, dump_lo, dump_hi;  // pending dump sync points: dump_lo, +between, .. < dump_hi
   double time_base, time_base_inv, t_current, t_end;
-  double dt_pred;
-  double sub_dt[HFV_MAX_SUBDRIFTS];
-  int n_sub;
-  int stepping;  // this step runs for this simulation
+  double dt_pred;  // hfv_predict's interval
   int done;
-  int force;     // next k_begin runs a step at ti_current without the engine's time loop (hfv_step)
-  int8_t mab;
-  int8_t pad8[3];
-  int min_bin;
-  unsigned long long ti_min, n_active, n_face_active;
+  int force;     // the next step runs at ti_current without the engine's time loop (hfv_step)
   long long step_count, cell_updates, face_fluxes;
   long long last_active, last_face_active;
   int err;
   // FP32-flux contexts defer the predict: a cell's extrapolations are extrap + (ti_pred - tiex) *
   // time_base * (-rate), with the rate constant between the tag and now.  ti_pred advances by every
-  // engine step's predict interval (k_begin), not by the trait-level phases (no_pred), whose predict
-  // settles the sums itself.  chk: host-written primitives wait for predict's check_physical.
+  // engine step's predict interval, not by the trait-level phases (no_pred), whose predict settles the
+  // sums itself.  chk: host-written primitives wait for predict's check_physical.
   int chk;
   int no_pred;
-  int pred_step;
+  int nf_mesh;  // 2D/3D moving meshes: faces of the current mesh (the device rebuild's count)
   uint64_t ti_pred;
-  int n_down;  // 1D periodic moving meshes: faces of this step's rebuild where the generator order steps down
-  int nf_mesh;  // 2D moving meshes: faces of the current mesh (the device rebuild's count)
-  int nf_tmp;   // 2D moving meshes: the rebuild's provisional face cursor
+};
+
+// One step of a simulation, worked out from its engine by every block of k_mask (step_begin) and kept here
+// by the block of the simulation's first chunk for the step's other kernels.
+struct SimStep {
+  uint64_t ti_old, ti_current, ti_pred;
+  double time_base, time_base_inv, t_current, dt_pred;
+  int stepping;  // this step runs for this simulation
+  int done;      // the simulation has ended (not stepping)
+  int forced;    // a step at the caller's ti_current (SimEngine::force)
+  int pred_step, chk;
+  int mab;       // get_max_active_bin(ti_current)
+  int pend;      // begun and not ended yet
+  int err;       // the first hard error that a kernel of this step raised (merged into the engine's at the end)
+  int min_bin;   // sync_all: the smallest new bin
+  int n_down;    // 1D periodic moving meshes: faces of this step's rebuild where the generator order steps down
+  int nf_tmp;    // 2D/3D moving meshes: the rebuild's provisional face cursor
   int pad_;
 };
 
@@ -169,6 +180,7 @@ struct Batch {
   Faces F;
   const SimDesc* sims;
   SimEngine* eng;
+  SimStep* st;
   int nsims;
   const BlockJob* cjobs;  // cell kernels: grid = number of entries
   const BlockJob* fjobs;  // face kernels
@@ -570,11 +582,11 @@ constexpr bool flux_stages() {
 #endif
 
 // Hard errors are recorded for the batch and for the simulation that raised them; a batch keeps
-// stepping its other simulations (the failed one stops at its next k_begin).
-__device__ __forceinline__ void flush_events(const Events& ev, DevCounters* cnt, SimEngine* eng = nullptr, int s = -1) {
+// stepping its other simulations (the failed one stops at the end of its step).
+__device__ __forceinline__ void flush_events(const Events& ev, DevCounters* cnt, int* sim_err = nullptr) {
   if (ev.err) {
     atomicCAS(&cnt->err, 0, ev.err);
-    if (eng && s >= 0) atomicCAS(&eng[s].err, 0, ev.err);
+    if (sim_err) atomicCAS(sim_err, 0, ev.err);
   }
   if (ev.check_physical) atomicAdd(&cnt->check_physical, (unsigned long long)ev.check_physical);
   if (ev.brent) atomicAdd(&cnt->brent, (unsigned long long)ev.brent);
@@ -624,79 +636,86 @@ __device__ __forceinline__ int block_min_i32(int v) {
 }
 
 // ------------------------------------------------------------------ engine (per simulation)
-// Engine::run loop head (engine.rs:152-185): the pending dump sync points are drifted through, then
-// the step at ti_next.
-__global__ void k_begin(Batch B) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s == 0) B.cnt->nfall = 0;
-  if (s >= B.nsims) return;
-  SimEngine& E = B.eng[s];
-  E.stepping = 0;
-  E.n_sub = 0;
-  E.n_down = 0;
-  E.nf_tmp = 0;
-  E.n_active = 0;
-  E.n_face_active = 0;
-  E.ti_min = ~0ull;
-  E.min_bin = 127;
-  if (E.err) {  // a hard error stops this simulation only; the batch's other simulations go on
-    E.force = 0;
-    E.done = 1;
-    return;
-  }
-  if (E.force) {  // hfv_step: a step at ti_current with the caller's ti_old
-    E.force = 0;
-    E.stepping = 1;
-  } else {
-    if (E.done) return;
-    if (!(E.t_current < E.t_end)) {
-      E.done = 1;
-      return;
-    }
-    uint64_t cur = E.ti_current;
-    int ns = 0;
-    for (uint64_t d = E.dump_lo; d < E.dump_hi; d += E.between) {
-      if (d > cur) {
-        if (ns < HFV_MAX_SUBDRIFTS) E.sub_dt[ns] = (double)(d - cur) * E.time_base;
-        ns++;
-        cur = d;
-      }
-      if (E.between == 0) break;
-    }
-    E.dump_lo = E.dump_hi;
-    if (E.ti_next > cur) {
-      if (ns < HFV_MAX_SUBDRIFTS) E.sub_dt[ns] = (double)(E.ti_next - cur) * E.time_base;
+// Engine::run loop head (engine.rs:152-185): the drifts through the pending dump sync points to the step
+// at ti_next, at most HFV_MAX_SUBDRIFTS of them: f(dt) for each.  False where there are more.
+template <class Fn>
+__device__ __forceinline__ bool sub_drifts(const SimEngine& E, Fn&& f) {
+  uint64_t cur = E.ti_current;
+  int ns = 0;
+  for (uint64_t d = E.dump_lo;; d += E.between) {
+    const bool last = !(d < E.dump_hi);
+    const uint64_t t = last ? E.ti_next : d;
+    if (t > cur) {
+      if (ns < HFV_MAX_SUBDRIFTS) f((double)(t - cur) * E.time_base);
       ns++;
+      cur = t;
     }
-    if (ns > HFV_MAX_SUBDRIFTS) {
-      E.err = E_UNSUPPORTED;
-      atomicCAS(&B.cnt->err, 0, E_UNSUPPORTED);
-      ns = HFV_MAX_SUBDRIFTS;
-    }
-    E.n_sub = ns;
-    E.ti_current = E.ti_next;
-    E.t_current = (double)E.ti_current * E.time_base;
-    E.stepping = 1;
+    if (last) break;
+    if (E.between == 0) d = E.dump_hi;  // (a single dump)
   }
-  E.dt_pred = (double)(E.ti_current - E.ti_old) * E.time_base;
-  E.pred_step = !E.no_pred;
-  if (E.pred_step) E.ti_pred += E.ti_current - E.ti_old;
-  E.no_pred = 0;
-  E.mab = get_max_active_bin(E.ti_current);
+  return ns <= HFV_MAX_SUBDRIFTS;
 }
 
-// Engine::step / queue_step / update_ti_next (engine.rs:194-268).  One block (HFV_END_BLOCK threads) per
-// simulation sums the chunk partials of this step (eight loads in flight per thread), then one thread
-// moves the engine to its next sync point.
-#define HFV_END_BLOCK 1024
-__global__ void __launch_bounds__(HFV_END_BLOCK) k_end(Batch B) {
-  __shared__ uint32_t sa[HFV_END_BLOCK / 64], sf[HFV_END_BLOCK / 64];
-  __shared__ uint64_t st[HFV_END_BLOCK / 64];
-  const int s = blockIdx.x;
+// The step that the engine takes next (Engine::run's loop head), without changing the engine.  A pure
+// function of it, so each block of k_mask works it out for itself: a launch of its own for this (and one
+// for the drift) took 4-5 us a step, all of it launch and cold loads (k_limit has the figures).
+__device__ __forceinline__ SimStep step_begin(const SimEngine& E) {
+  SimStep S;
+  S.stepping = 0;
+  S.done = 0;
+  S.forced = 0;
+  S.ti_old = E.ti_old;
+  S.ti_current = E.ti_current;
+  S.ti_pred = E.ti_pred;
+  S.time_base = E.time_base;
+  S.time_base_inv = E.time_base_inv;
+  S.t_current = E.t_current;
+  S.chk = E.chk;
+  S.pend = 1;
+  S.err = 0;
+  S.min_bin = 127;
+  S.n_down = 0;
+  S.nf_tmp = 0;
+  S.pad_ = 0;
+  if (E.err) {  // a hard error stops this simulation only; the batch's other simulations go on
+    S.done = 1;
+  } else if (E.force) {  // hfv_step: a step at ti_current with the caller's ti_old
+    S.forced = 1;
+    S.stepping = 1;
+  } else if (E.done || !(E.t_current < E.t_end)) {
+    S.done = 1;
+  } else {
+    S.ti_current = E.ti_next;
+    S.t_current = (double)E.ti_next * E.time_base;
+    S.stepping = 1;
+  }
+  S.dt_pred = (double)(S.ti_current - S.ti_old) * S.time_base;
+  S.pred_step = !E.no_pred;
+  if (S.stepping && S.pred_step) S.ti_pred += S.ti_current - S.ti_old;
+  S.mab = get_max_active_bin(S.ti_current);
+  return S;
+}
+
+// Engine::step / queue_step / update_ti_next (engine.rs:194-268) of simulation s by one block: sums the chunk
+// partials of this step (eight loads in flight per thread), then one thread moves the engine to its next
+// sync point.  phase: a trait-level call, which ends the step whether or not it has been ended.
+__device__ __forceinline__ void step_end(const Batch& B, int s, int phase) {
+  __shared__ uint32_t sa[HFV_BLOCK / 64], sf[HFV_BLOCK / 64];
+  __shared__ uint64_t st[HFV_BLOCK / 64];
   SimEngine& E = B.eng[s];
-  if (!E.stepping) return;
+  SimStep& S = B.st[s];
+  if (!(S.pend || (phase && S.stepping))) return;  // block-uniform: only this block's last thread changes it
+  if (!S.stepping) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      E.done = S.done ? 1 : E.done;
+      E.force = 0;
+      S.pend = 0;
+    }
+    return;
+  }
   const SimDesc& D = B.sims[s];
-  const int T = blockDim.x;
+  constexpr int T = HFV_BLOCK;
   uint32_t na = 0, nfc = 0;
   uint64_t tmin = ~0ull;
   for (int k0 = D.cchunk0 + (int)threadIdx.x; k0 < D.cchunk1; k0 += 8 * T) {
@@ -714,15 +733,15 @@ __global__ void __launch_bounds__(HFV_END_BLOCK) k_end(Batch B) {
       tmin = t[u] < tmin ? t[u] : tmin;
     }
   }
-  for (int k0 = D.fchunk0 + (int)threadIdx.x; k0 < D.fchunk1; k0 += 8 * T) {
-    uint32_t a[8];
+  for (int k0 = D.fchunk0 + (int)threadIdx.x; k0 < D.fchunk1; k0 += 16 * T) {
+    uint32_t a[16];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < 16; ++u) {
       const int k = k0 + u * T;
       a[u] = k < D.fchunk1 ? B.P.face[k] : 0u;
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) nfc += a[u];
+    for (int u = 0; u < 16; ++u) nfc += a[u];
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -738,7 +757,6 @@ __global__ void __launch_bounds__(HFV_END_BLOCK) k_end(Batch B) {
   }
   __syncthreads();
   if (threadIdx.x != 0) return;
-  if (E.pred_step) E.chk = 0;  // this step's k_mask has checked the host-written primitives
   na = 0;
   nfc = 0;
   tmin = ~0ull;
@@ -747,20 +765,29 @@ __global__ void __launch_bounds__(HFV_END_BLOCK) k_end(Batch B) {
     nfc += sf[w];
     tmin = st[w] < tmin ? st[w] : tmin;
   }
-  E.n_active = na;
-  E.n_face_active = nfc;
-  E.ti_min = tmin;
+  // the step's clocks become the engine's
+  E.force = 0;
+  E.no_pred = 0;
+  E.ti_current = S.ti_current;
+  E.t_current = S.t_current;
+  E.ti_pred = S.ti_pred;
+  if (!S.forced) E.dump_lo = E.dump_hi;
+  if (S.pred_step) E.chk = 0;  // this step's k_mask has checked the host-written primitives
+  const int err = S.err;
+  S.pend = 0;
+  S.err = 0;
+  if (err && !E.err) E.err = err;
   if (E.err) {  // the reference panics inside this step: it does not complete
     E.done = 1;
     return;
   }
-  if (E.n_active == 0 || E.ti_min == ~0ull) {  // the reference panics: "At least one particle must be active"
+  if (na == 0 || tmin == ~0ull) {  // the reference panics: "At least one particle must be active"
     E.err = E_UNSUPPORTED;
     atomicCAS(&B.cnt->err, 0, E_UNSUPPORTED);
     E.done = 1;
     return;
   }
-  uint64_t ti_next = E.ti_current + E.ti_min;
+  const uint64_t ti_next = E.ti_current + tmin;
   E.dump_lo = E.ti_snap;
   if (E.between) {
     while (E.ti_snap < ti_next) E.ti_snap += E.between;
@@ -769,10 +796,10 @@ __global__ void __launch_bounds__(HFV_END_BLOCK) k_end(Batch B) {
   E.ti_old = E.ti_next;
   E.ti_next = ti_next;
   E.step_count++;
-  E.cell_updates += (long long)E.n_active;
-  E.face_fluxes += (long long)E.n_face_active;
-  E.last_active = (long long)E.n_active;
-  E.last_face_active = (long long)E.n_face_active;
+  E.cell_updates += (long long)na;
+  E.face_fluxes += (long long)nfc;
+  E.last_active = (long long)na;
+  E.last_face_active = (long long)nfc;
 }
 
 // ------------------------------------------------------------------ drift (space.rs:833-854)
@@ -781,7 +808,7 @@ __global__ void __launch_bounds__(HFV_END_BLOCK) k_end(Batch B) {
 // gradients (its v_rel is not reflected), so that this step's predict (optimal_order.rs:20, after the
 // drift) extrapolates the reflected state; FP32-flux contexts first sum their unsummed predict time up
 // to the start of this step with the old rate.
-__device__ void drift_cell(const Cells& C, const Cfg& cfg, const SimEngine& E, int64_t i, double dt, Events& ev) {
+__device__ void drift_cell(const Cells& C, const Cfg& cfg, const SimStep& S, int64_t i, double dt, Events& ev) {
   const int64_t n = C.n;
   const int dim = cfg.dim;
   double loc[3], cen[3], gc[3];
@@ -804,7 +831,9 @@ __device__ void drift_cell(const Cells& C, const Cfg& cfg, const SimEngine& E, i
       double old[3] = {loc[0], loc[1], loc[2]};
       for (int a = 0; a < dim; ++a) {
         int guard = 0;
+#pragma unroll 1
         while (loc[a] < 0. && ++guard < 64) loc[a] += cfg.box[a];
+#pragma unroll 1
         while (loc[a] >= cfg.box[a] && ++guard < 128) loc[a] -= cfg.box[a];
       }
       for (int a = 0; a < 3; ++a) {
@@ -831,8 +860,8 @@ __device__ void drift_cell(const Cells& C, const Cfg& cfg, const SimEngine& E, i
         // density gradient for the pressure gradient
         const bool f32 = cfg.precision == HFV_FP32_FLUX;
         if (f32) {
-          const uint64_t t0 = E.pred_step ? E.ti_pred - (E.ti_current - E.ti_old) : E.ti_pred;
-          const double el = (double)(t0 - C.tiex[i]) * E.time_base;
+          const uint64_t t0 = S.pred_step ? S.ti_pred - (S.ti_current - S.ti_old) : S.ti_pred;
+          const double el = (double)(t0 - C.tiex[i]) * S.time_base;
           st_ex(C, i, true, ld_ex(C, i, true) + (p_old.c[0] > 0. ? (-el) * ld_tex(C, i, true) : vacuum<double>()));
           C.tiex[i] = t0;
         }
@@ -861,33 +890,48 @@ __device__ void drift_cell(const Cells& C, const Cfg& cfg, const SimEngine& E, i
   }
 }
 
-// Engine::run's drift through the step's sync points (moving meshes only).
-__global__ void __launch_bounds__(HFV_BLOCK) k_drift(Batch B) {
-  const BlockJob J = B.cjobs[blockIdx.x];
-  if (J.sim < 0) return;
-  const SimEngine& E = B.eng[J.sim];
-  const Cfg& cfg = B.sims[J.sim].cfg;
-  if (!E.stepping || E.n_sub == 0 || cfg.motion == MOT_FIXED) return;
-  const int64_t i = (int64_t)J.lo + threadIdx.x;
-  if (i >= J.hi) return;
-  Events ev;
-  for (int k = 0; k < E.n_sub; ++k) drift_cell(B.C, cfg, E, i, E.sub_dt[k], ev);
-  flush_events(ev, B.cnt, B.eng, J.sim);
-}
-
 // ------------------------------------------------------------------ k_mask
-// Active mask (optimal_order.rs:17) and predict (euler_eqns_fvs.rs:20-24, part.rs:121-149) of every
-// cell.  mode 0: step; 1: predict only (dt from the engine's dt_pred); 2: mask only.
-// FP32-flux contexts defer the step's predict (k_begin advanced ti_pred; the flux kernel's readers add
+// The step of every simulation from its engine (step_begin), the drift of moving generators through the
+// step's sync points (engine.rs:152-185), the active mask (optimal_order.rs:17) and the predict
+// (euler_eqns_fvs.rs:20-24, part.rs:121-149) of every cell: all of them cell by cell, so one launch.
+// mode 0: step; 1: predict only (dt from the engine's dt_pred); 2: mask only.
+// FP32-flux contexts defer the step's predict (step_begin advances ti_pred; the flux kernel's readers add
 // rate x elapsed time, face_side): check_physical runs only after host writes of the primitives (a no-op otherwise,
 // since c2p and the apply_flux reset leave physical states), settling the sums first.  Mode 1 settles
 // the sums and adds dt_pred at once.
+// MOVING: the context holds moving meshes (the fixed ones' kernel carries no drift registers).
+template <bool MOVING>
 __global__ void __launch_bounds__(HFV_BLOCK) k_mask(Batch B, int mode) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) B.cnt->nfall = 0;
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimEngine& E = B.eng[s];
-  if (mode != 1 && !E.stepping) return;
+  const SimStep S = step_begin(E);
+  if (mode != 1) {
+    // (err is the running step's own: a block of this launch may have raised it already)
+    if (J.chunk == B.sims[s].cchunk0 && threadIdx.x == 0) {
+      SimStep& G = B.st[s];
+      G.ti_old = S.ti_old;
+      G.ti_current = S.ti_current;
+      G.ti_pred = S.ti_pred;
+      G.time_base = S.time_base;
+      G.time_base_inv = S.time_base_inv;
+      G.t_current = S.t_current;
+      G.dt_pred = S.dt_pred;
+      G.stepping = S.stepping;
+      G.done = S.done;
+      G.forced = S.forced;
+      G.pred_step = S.pred_step;
+      G.chk = S.chk;
+      G.mab = S.mab;
+      G.pend = S.pend;
+      G.min_bin = S.min_bin;
+      G.n_down = S.n_down;
+      G.nf_tmp = S.nf_tmp;
+    }
+    if (!S.stepping) return;
+  }
   const Cfg& cfg = B.sims[s].cfg;
   const Cells& C = B.C;
   const int64_t n = C.n;
@@ -895,23 +939,38 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mask(Batch B, int mode) {
   const bool valid = i < J.hi;
   bool act = false;
   Events ev;
+  if (mode == 0 && !S.forced) {
+    const bool moves = MOVING && cfg.motion != MOT_FIXED;
+    const bool fits = sub_drifts(E, [&](double dt) {
+      if constexpr (MOVING) {
+        int32_t c = (int32_t)i;
+        asm volatile("" : "+v"(c));  // addresses formed per drift: hoisted out of the loop they fill 256 VGPRs
+        if (moves && valid) drift_cell(C, cfg, S, c, dt, ev);
+      }
+    });
+    if (!fits) ev.fail(E_UNSUPPORTED);
+  }
   if (valid) {
     if (mode != 1) {
-      act = C.bin[i] <= E.mab;
+      act = C.bin[i] <= S.mab;
       C.act[i] = act;
+      C.nbin[i] = HFV_NO_BIN;
     }
     const bool f32 = cfg.precision == HFV_FP32_FLUX;
-    if (mode != 2 && (!f32 || mode == 1 || E.chk)) {
+    if (mode != 2 && (!f32 || mode == 1 || S.chk)) {
       St<double> prim = ld5(C.prim, n, i);
       // the rate of this prim/grad/v_rel, kept by k_grad (k_pack_fr after host changes);
       // extrapolations += time_extrapolations(dt) (its vacuum branch adds +0)
       const St<double> rate = prim.c[0] > 0. ? ld_tex(C, i, f32) : vacuum<double>();
+      // a separate predict takes its interval and the clock from the engine as the host left it
+      const uint64_t ti_pred = mode == 1 ? E.ti_pred : S.ti_pred;
+      const double dt_pred = mode == 1 ? E.dt_pred : S.dt_pred;
       if (f32) {
-        const double dt = (double)(E.ti_pred - C.tiex[i]) * E.time_base + (mode == 1 ? E.dt_pred : 0.);
+        const double dt = (double)(ti_pred - C.tiex[i]) * E.time_base + (mode == 1 ? dt_pred : 0.);
         st_ex(C, i, true, ld_ex(C, i, true) + (prim.c[0] > 0. ? (-dt) * rate : vacuum<double>()));
-        C.tiex[i] = E.ti_pred;
+        C.tiex[i] = ti_pred;
       } else {
-        St<double> te = prim.c[0] > 0. ? (-E.dt_pred) * rate : vacuum<double>();
+        St<double> te = prim.c[0] > 0. ? (-dt_pred) * rate : vacuum<double>();
         st_ex(C, i, false, ld_ex(C, i, false) + te);
       }
       check_physical(prim, ev);
@@ -942,7 +1001,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mask(Batch B, int mode) {
       B.P.act[J.chunk] = cnt;
     }
   }
-  if (valid) flush_events(ev, B.cnt, B.eng, s);
+  if (valid) flush_events(ev, B.cnt, &B.st[s].err);
 }
 
 // ------------------------------------------------------------------ 1D moving mesh on the device
@@ -957,7 +1016,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mesh1d_faces(Batch B) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  if (!D.moving1d || !B.eng[s].stepping) return;
+  if (!D.moving1d || !B.st[s].stepping) return;
   const int64_t f = (int64_t)J.lo + threadIdx.x;
   if (f >= J.hi) return;
   int64_t k = f - D.face_base, n = D.n, cb = D.cell_base;
@@ -967,7 +1026,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mesh1d_faces(Batch B) {
       double a = B.C.loc[cb + k - 1], b = B.C.loc[cb + k];
       if (!(a < b)) {
         atomicCAS(&B.cnt->err, 0, E_UNSUPPORTED);
-        atomicCAS(&B.eng[s].err, 0, E_UNSUPPORTED);
+        atomicCAS(&B.st[s].err, 0, E_UNSUPPORTED);
       }
       x = 0.5 * (a + b);
     } else {
@@ -978,7 +1037,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mesh1d_faces(Batch B) {
     const bool down = !(a < b);
     x = down ? 0.5 * (a + (b + D.cfg.box[0])) : 0.5 * (a + b);
     B.F.shc[f] = down ? 1 : 0;  // +box along x
-    if (down) atomicAdd(&B.eng[s].n_down, 1);
+    if (down) atomicAdd(&B.st[s].n_down, 1);
   }
   B.F.fcen[f] = x;
 }
@@ -986,7 +1045,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mesh1d_cells(Batch B) {
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
   const SimDesc& D = B.sims[J.sim];
-  if (!D.moving1d || !B.eng[J.sim].stepping) return;
+  if (!D.moving1d || !B.st[J.sim].stepping) return;
   const int64_t i = (int64_t)J.lo + threadIdx.x;
   if (i >= J.hi || !B.C.act[i]) return;
   const int64_t N = B.C.n;
@@ -996,9 +1055,9 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mesh1d_cells(Batch B) {
     xl = B.F.fcen[fb + k];
     xr = B.F.fcen[fb + k + 1];
   } else {
-    if (B.eng[J.sim].n_down != 1) {  // not a rotation of the line's order: the topology changed
+    if (B.st[J.sim].n_down != 1) {  // not a rotation of the line's order: the topology changed
       atomicCAS(&B.cnt->err, 0, E_UNSUPPORTED);
-      atomicCAS(&B.eng[J.sim].err, 0, E_UNSUPPORTED);
+      atomicCAS(&B.st[J.sim].err, 0, E_UNSUPPORTED);
     }
     // the left face's centroid is in cell k-1's frame: a box to the right when it carries the shift
     xl = B.F.fcen[fb + k] - (B.F.shc[fb + k] ? D.cfg.box[0] : 0.);
@@ -1040,13 +1099,13 @@ template <class T>
 struct SoaCell {
   const Cells* C;
   const Gas<double>* g;
-  const SimEngine* E;
+  const SimStep* S;
   uint32_t i;
-  __device__ __forceinline__ SoaCell(const Cells& c, const Gas<double>& gd, const SimEngine& e, int32_t idx)
-      : C(&c), g(&gd), E(&e), i((uint32_t)idx) {}
+  __device__ __forceinline__ SoaCell(const Cells& c, const Gas<double>& gd, const SimStep& st, int32_t idx)
+      : C(&c), g(&gd), S(&st), i((uint32_t)idx) {}
   __device__ __forceinline__ double dt() const { return ldo(C->dt, i); }
   // predict time not yet summed into the stored extrapolations (FP32-flux contexts)
-  __device__ __forceinline__ double el() const { return (double)(E->ti_pred - C->tiex[i]) * E->time_base; }
+  __device__ __forceinline__ double el() const { return (double)(S->ti_pred - C->tiex[i]) * S->time_base; }
   __device__ __forceinline__ St<double> prim() const {
     const St<double> p = ld5(C->prim, C->n, i);
     return mkst(rnd<T>(p.c[0]), mk3(rnd<T>(p.c[1]), rnd<T>(p.c[2]), rnd<T>(p.c[3])), rnd<T>(p.c[4]));
@@ -1316,7 +1375,7 @@ template <class T, int SOLVER, bool STATIC>
 __device__ __forceinline__ void flux_chunk(const Batch& B, const BlockJob J) {
   if (J.sim < 0) return;
   const int s = J.sim;
-  if (!B.eng[s].stepping || B.sims[s].static_geom != (STATIC ? 1 : 0)) return;
+  if (!B.st[s].stepping || B.sims[s].static_geom != (STATIC ? 1 : 0)) return;
   const Cfg& cfg = B.sims[s].cfg;
   const int64_t f = (int64_t)J.lo + threadIdx.x;
   constexpr bool DEFER = SOLVER == SOLVER_AIRS;
@@ -1397,8 +1456,8 @@ __device__ __forceinline__ void flux_chunk(const Batch& B, const BlockJob J) {
           if (c < ns) ldsf[c * HFV_FR32_LDS + HFV_FR32_EX + q] = (float)xv[j];
         }
         if ((int)threadIdx.x < ns) {
-          const SimEngine& E = B.eng[s];
-          ldsf[threadIdx.x * HFV_FR32_LDS + HFV_FR32_EL] = (float)((double)(E.ti_pred - tv) * E.time_base);
+          const SimStep& S = B.st[s];
+          ldsf[threadIdx.x * HFV_FR32_LDS + HFV_FR32_EL] = (float)((double)(S.ti_pred - tv) * S.time_base);
         }
       } else {
 #pragma unroll
@@ -1430,12 +1489,12 @@ __device__ __forceinline__ void flux_chunk(const Batch& B, const BlockJob J) {
       }
       __syncthreads();  // the staged records are dead from here on
     } else if (cur) {
-      computed = face_flux<T, SOLVER, DEFER, true, SoaCell<T>>(B, cfg, f, SoaCell<T>(B.C, cfg.gd, B.eng[s], l),
-                                                               SoaCell<T>(B.C, cfg.gd, B.eng[s], r), r, la, ra, outv, ev);
+      computed = face_flux<T, SOLVER, DEFER, true, SoaCell<T>>(B, cfg, f, SoaCell<T>(B.C, cfg.gd, B.st[s], l),
+                                                               SoaCell<T>(B.C, cfg.gd, B.st[s], r), r, la, ra, outv, ev);
     }
   } else if (cur) {
-    computed = face_flux<T, SOLVER, DEFER, false, SoaCell<T>>(B, cfg, f, SoaCell<T>(B.C, cfg.gd, B.eng[s], l),
-                                                              SoaCell<T>(B.C, cfg.gd, B.eng[s], r), r, la, ra, outv, ev);
+    computed = face_flux<T, SOLVER, DEFER, false, SoaCell<T>>(B, cfg, f, SoaCell<T>(B.C, cfg.gd, B.st[s], l),
+                                                              SoaCell<T>(B.C, cfg.gd, B.st[s], r), r, la, ra, outv, ev);
   }
   // records of faces with an active cell (deferred ones zero here, overwritten by k_flux_fallback)
   curs[threadIdx.x] = cur ? 1 : 0;
@@ -1477,7 +1536,7 @@ __device__ __forceinline__ void flux_chunk(const Batch& B, const BlockJob J) {
   uint32_t cnt = block_sum_u32(computed ? 1u : 0u);
   if (threadIdx.x == 0) B.P.face[J.chunk] = cnt;
   ev.deferred = 0;
-  flush_events(ev, B.cnt, B.eng, s);
+  flush_events(ev, B.cnt, &B.st[s].err);
 }
 
 // One block per fpt face chunks (fpt faces per thread: 1, 2 or 4, the autotuner's launch-shape choice):
@@ -1507,10 +1566,10 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_flux_fallback(Batch B) {
     Events ev;
     double outv[7];
     const Cfg& cfg = B.sims[s].cfg;
-    face_flux<T, SOLVER_AIRS, false, false, SoaCell<T>>(B, cfg, f, SoaCell<T>(B.C, cfg.gd, B.eng[s], l),
-                                                        SoaCell<T>(B.C, cfg.gd, B.eng[s], r), r, la, ra, outv, ev);
+    face_flux<T, SOLVER_AIRS, false, false, SoaCell<T>>(B, cfg, f, SoaCell<T>(B.C, cfg.gd, B.st[s], l),
+                                                        SoaCell<T>(B.C, cfg.gd, B.st[s], r), r, la, ra, outv, ev);
     store_rec(B.F.rec, f, outv, sizeof(T) == 4);
-    flush_events(ev, B.cnt, B.eng, s);
+    flush_events(ev, B.cnt, &B.st[s].err);
   }
 }
 
@@ -1552,7 +1611,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_apply(Batch B, int mode) {
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
   const int s = J.sim;
-  if (!B.eng[s].stepping) return;
+  if (!B.st[s].stepping) return;
   // fused step: a chunk with no active cell whose cells have no active neighbour (no chunk on its list of
   // neighbour chunks holds an active cell) has nothing to accumulate, apply or pack on a fixed mesh, and
   // nothing for the limiter sweeps (which read the decision from cflag)
@@ -1677,7 +1736,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_apply(Batch B, int mode) {
   // the pc pack changes where prim changed (active cells), or everywhere on moving meshes / on request
   if ((mode & 4) && (have_prim || (mode & 8) || cfg.motion != MOT_FIXED))
     store_pc(C.pc, i, have_prim ? prim : ld5(C.prim, n, i), ld3(C.cen, n, i));
-  flush_events(ev, B.cnt, B.eng, s);
+  flush_events(ev, B.cnt, &B.st[s].err);
 }
 
 // The pc pack of cells [lo, hi) from the SoA fields (after the host changed the state or mesh).
@@ -1783,7 +1842,7 @@ __device__ __forceinline__ void boundary_neighbour(const Faces& F, const Cfg& cf
 // gradient matrix, are the values k_geom_cells computed once with the same expressions and order.  (On
 // 1D/2D meshes recomputing them reads fewer bytes than the precomputed lines, so those stay dynamic.)
 template <bool STATIC>
-__device__ __forceinline__ void grad_cell(const Batch& B, const Cfg& cfg, const SimEngine& E, int64_t i, int do_grad,
+__device__ __forceinline__ void grad_cell(const Batch& B, const Cfg& cfg, const SimStep& S, int64_t i, int do_grad,
                                           int do_ts, bool pack_fr, double* frv, bool v_zero, const double4* gst,
                                           uint64_t* dti_out, Events& ev) {
   const Cells& C = B.C;
@@ -2088,10 +2147,10 @@ __device__ __forceinline__ void grad_cell(const Batch& B, const Cfg& cfg, const 
   }
   // ---- timesteps_apply
   int8_t bin = C.bin[i];
-  uint64_t dti = make_integer_timestep(dt_req, bin, HFV_NUM_TIME_BINS, E.ti_current, E.time_base_inv);
-  const double dt_new = (double)dti * E.time_base;
+  uint64_t dti = make_integer_timestep(dt_req, bin, HFV_NUM_TIME_BINS, S.ti_current, S.time_base_inv);
+  const double dt_new = (double)dti * S.time_base;
   C.dt[i] = dt_new;
-  C.bin[i] = get_time_bin(dti);
+  C.nbin[i] = get_time_bin(dti);
   *dti_out = dti;
   // the time-extrapolation rate and the flux record for the next step (prim, gradients, v_rel and dt
   // are final here)
@@ -2106,8 +2165,8 @@ __global__ void __launch_bounds__(HFV_BLOCK, HFV_GRAD_WAVES) k_grad(Batch B, int
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
   const int s = J.sim;
-  const SimEngine& E = B.eng[s];
-  if (!E.stepping || B.sims[s].static_grad != (STATIC ? 1 : 0)) return;
+  const SimStep& S = B.st[s];
+  if (!S.stepping || B.sims[s].static_grad != (STATIC ? 1 : 0)) return;
   if (do_grad == 1 && do_ts == 1 && !B.P.act[J.chunk]) {  // fused step, no active cell in the chunk
     if (threadIdx.x == 0) B.P.ti[J.chunk] = ~0ull;
     return;
@@ -2158,7 +2217,7 @@ __global__ void __launch_bounds__(HFV_BLOCK, HFV_GRAD_WAVES) k_grad(Batch B, int
   }
   double frv[HFV_FR_W];
   if (a)
-    grad_cell<STATIC>(B, cfg, E, i, do_grad, do_ts, pack, frv, B.sims[s].static_geom != 0, staged ? lds4 : nullptr,
+    grad_cell<STATIC>(B, cfg, S, i, do_grad, do_ts, pack, frv, B.sims[s].static_geom != 0, staged ? lds4 : nullptr,
                       &my, ev);
   if (pack) {
     if (staged) __syncthreads();  // the staged lines are dead from here on
@@ -2171,7 +2230,7 @@ __global__ void __launch_bounds__(HFV_BLOCK, HFV_GRAD_WAVES) k_grad(Batch B, int
     uint64_t t = block_min_u64(my);
     if (threadIdx.x == 0) B.P.ti[J.chunk] = t;
   }
-  flush_events(ev, B.cnt, B.eng, s);
+  flush_events(ev, B.cnt, &B.st[s].err);
 }
 
 // timesteps_apply (hydrodynamics.rs:145-158) of the requested timesteps in dtq (the caller's, e.g. the
@@ -2179,14 +2238,14 @@ __global__ void __launch_bounds__(HFV_BLOCK, HFV_GRAD_WAVES) k_grad(Batch B, int
 __global__ void __launch_bounds__(HFV_BLOCK) k_ts_apply(Batch B) {
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
-  const SimEngine& E = B.eng[J.sim];
-  if (!E.stepping) return;
+  const SimStep& S = B.st[J.sim];
+  if (!S.stepping) return;
   const int64_t i = (int64_t)J.lo + threadIdx.x;
   uint64_t my = ~0ull;
   if (i < J.hi && B.C.act[i]) {
-    const uint64_t dti = make_integer_timestep(B.C.dtq[i], B.C.bin[i], HFV_NUM_TIME_BINS, E.ti_current, E.time_base_inv);
-    B.C.dt[i] = (double)dti * E.time_base;
-    B.C.bin[i] = get_time_bin(dti);
+    const uint64_t dti = make_integer_timestep(B.C.dtq[i], B.C.bin[i], HFV_NUM_TIME_BINS, S.ti_current, S.time_base_inv);
+    B.C.dt[i] = (double)dti * S.time_base;
+    B.C.nbin[i] = get_time_bin(dti);
     my = dti;
   }
   const uint64_t t = block_min_u64(my);
@@ -2329,102 +2388,102 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_geom_faces(Batch B, int s, int64_
 }
 
 // ------------------------------------------------------------------ limiter
-// timestep_limiter first sweep (hydrodynamics.rs:165-179): wakeup from active neighbours' new bins;
-// timestep_sync (hydrodynamics.rs:186-191) reduces the minimum bin per simulation instead.
-// A chunk without active cells or active neighbours (k_apply's decision in cflag): its wakeups are the
-// cells' own bins and k_limit changes nothing there, so the fused step (fused = 1) skips it in both.
-__device__ __forceinline__ bool limiter_idle(const Batch& B, const BlockJob& J) {
-  return !B.sims[J.sim].cfg.sync_all && !B.P.cflag[J.chunk];
-}
-
-__global__ void __launch_bounds__(HFV_BLOCK) k_wakeup(Batch B, int fused) {
+// timestep_sync (hydrodynamics.rs:186-191): the minimum bin of every cell of a sync_all simulation (launched
+// only where one is loaded).
+__global__ void __launch_bounds__(HFV_BLOCK) k_sync_min(Batch B) {
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
   const int s = J.sim;
-  if (!B.eng[s].stepping) return;
-  if (fused && limiter_idle(B, J)) return;
-  const Cells& C = B.C;
-  const Faces& F = B.F;
+  if (!B.st[s].stepping || !B.sims[s].cfg.sync_all) return;
   const int64_t i = (int64_t)J.lo + threadIdx.x;
-  const bool valid = i < J.hi;
-  if (B.sims[s].cfg.sync_all) {
-    int m = block_min_i32(valid ? (int)C.bin[i] : 0x7fffffff);
-    if (threadIdx.x == 0) atomicMin(&B.eng[s].min_bin, m);
+  int m = 0x7fffffff;
+  if (i < J.hi) m = B.C.act[i] ? (int)B.C.nbin[i] : (int)B.C.bin[i];
+  m = block_min_i32(m);
+  if (threadIdx.x == 0) atomicMin(&B.st[s].min_bin, m);
+}
+
+// The limiter (hydrodynamics.rs:165-179: a cell is woken by its active neighbours' new bins), with
+// Particle::timestep_limit (part.rs:263-297), reset_extrapolations (hydrodynamics.rs:193-195) and kick1
+// (hydro_kick1 part.rs:87-104, grav_kick with a_grav = 0), and in blocks of their own the end of each
+// simulation's step (step_end).  The new bins of the active cells are in nbin and the final ones go to bin,
+// so that no block reads what another one writes and one launch does the work of three (wakeup, limit, end:
+// 13-15 us a step on meshes where each is only launch and cold loads); a neighbour costs one byte.
+// A chunk without active cells or active neighbours (k_apply's decision in cflag) has nothing to change, so
+// the fused step skips it.  phase: a trait-level call; it also applies kick1's "momentum += 0 * mass" (a
+// no-op after kick2 of the same step, which the fused step has already done).
+// Grid: one block per slot, then the cell block table.
+__global__ void __launch_bounds__(HFV_BLOCK) k_limit(Batch B, int phase) {
+  if ((int)blockIdx.x < B.nsims) {
+    step_end(B, (int)blockIdx.x, phase);
     return;
   }
-  if (!valid) return;
-  int8_t w = C.bin[i];
-  const int32_t k0 = F.off[i], k1 = F.off[i + 1];
-  // entries in chunks of 8: a chunk's neighbours, then their active flags and bins, all in flight together
-  // (the bin is read whether or not the neighbour is active: same result, no dependent load; a minimum,
-  // so the order does not matter)
-  for (int32_t kb = k0; kb < k1; kb += 8) {
-    int32_t o[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) o[u] = kb + u < k1 ? F.nbr[kb + u] : -1;
-    uint32_t ab[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) ab[u] = o[u] >= 0 ? ((uint32_t)C.act[o[u]] << 8) | (uint8_t)C.bin[o[u]] : 0u;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      if (!(ab[u] >> 8)) continue;
-      const int8_t cand = (int8_t)((int8_t)(ab[u] & 0xFF) + 2);
-      if (cand < w) w = cand;
-    }
-  }
-  C.wake[i] = w;
-}
-
-// Particle::timestep_limit (part.rs:263-297) + reset_extrapolations (hydrodynamics.rs:193-195) +
-// kick1 (hydro_kick1 part.rs:87-104, grav_kick with a_grav = 0).
-// canon: apply kick1's "momentum += 0 * mass" (a no-op after kick2 of the same step, which the fused
-// step has already done; the trait-level phases keep it).
-__global__ void __launch_bounds__(HFV_BLOCK) k_limit(Batch B, int canon) {
-  const BlockJob J = B.cjobs[blockIdx.x];
+  const BlockJob J = B.cjobs[blockIdx.x - B.nsims];
   if (J.sim < 0) return;
   const int s = J.sim;
-  const SimEngine& E = B.eng[s];
-  if (!E.stepping) return;
-  if (!canon && limiter_idle(B, J)) return;
+  const SimStep& S = B.st[s];
+  if (!S.stepping) return;
+  const Cfg& cfg = B.sims[s].cfg;
+  if (!phase && !cfg.sync_all && !B.P.cflag[J.chunk]) return;
   const int64_t i = (int64_t)J.lo + threadIdx.x;
   if (i >= J.hi) return;
   const Cells& C = B.C;
-  const Cfg& cfg = B.sims[s].cfg;
+  const Faces& F = B.F;
   const int64_t n = C.n;
-  int8_t wakeup = cfg.sync_all ? (int8_t)E.min_bin : C.wake[i];
-  int8_t bin = C.bin[i];
-  if (wakeup < bin) {
-    double dt = C.dt[i];
-    uint64_t ti_current = E.ti_current;
-    double time_base = E.time_base;
+  const bool a = C.act[i];
+  const int8_t bin0 = C.bin[i];
+  int8_t bin = a ? C.nbin[i] : bin0;
+  int wakeup = bin;
+  if (cfg.sync_all) {
+    wakeup = S.min_bin;
+  } else {
+    // entries in chunks of 8: a chunk's neighbours, then their new bins, all in flight together (a minimum,
+    // so the order does not matter)
+    const int32_t k0 = F.off[i], k1 = F.off[i + 1];
+    for (int32_t kb = k0; kb < k1; kb += 8) {
+      int32_t o[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) o[u] = kb + u < k1 ? F.nbr[kb + u] : -1;
+      int nb[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) nb[u] = o[u] >= 0 ? (int)C.nbin[o[u]] : HFV_NO_BIN;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) wakeup = nb[u] + 2 < wakeup ? nb[u] + 2 : wakeup;
+    }
+  }
+  double dt = 0.;
+  const bool woken = wakeup < bin;
+  if (woken) {
+    dt = C.dt[i];
+    const uint64_t ti_current = S.ti_current;
+    const double time_base = S.time_base;
     if (bin <= get_max_active_bin(ti_current)) {
-      bin = wakeup;
+      bin = (int8_t)wakeup;
       dt = (double)get_integer_timestep(bin) * time_base;
     } else {
       uint64_t ti_end_old = get_integer_time_end(ti_current, bin);
       dt -= (double)(ti_end_old - ti_current) * time_base;
-      bin = wakeup;
+      bin = (int8_t)wakeup;
       uint64_t dti_new = get_integer_timestep(bin);
       uint64_t ti_end = get_integer_time_end(ti_current, bin);
       dt += (ti_end == ti_current) ? (double)dti_new * time_base : (double)(ti_end - ti_current) * time_base;
     }
-    C.bin[i] = bin;
     C.dt[i] = dt;
     if (B.sims[s].staged) C.fr[HFV_FR_W * (uint64_t)i + HFV_FR_DT] = dt;
   }
-  if (C.act[i]) {
+  if (bin != bin0) C.bin[i] = bin;
+  if (a) {
     st_ex(C, i, cfg.precision == HFV_FP32_FLUX, vacuum<double>());
-    if (cfg.precision == HFV_FP32_FLUX) C.tiex[i] = E.ti_pred;  // the sum restarts at zero now
+    if (cfg.precision == HFV_FP32_FLUX) C.tiex[i] = S.ti_pred;  // the sum restarts at zero now
     if (cfg.motion != MOT_FIXED) {
       double rho = C.prim[i];
       if (rho > 0.) {
-        double kick_fac = 0.5 * C.dt[i] / rho;
+        double kick_fac = 0.5 * (woken ? dt : C.dt[i]) / rho;
         const Gr<double> g = ld_grad(C, i, cfg.precision == HFV_FP32_FLUX);
         const double dp[3] = {g.g[4].x, g.g[4].y, g.g[4].z};
-        for (int a = 0; a < cfg.dim; ++a) C.v[a * n + i] -= kick_fac * dp[a];
+        for (int q = 0; q < cfg.dim; ++q) C.v[q * n + i] -= kick_fac * dp[q];
       }
     }
-    if (canon) {
+    if (phase) {
       C.cons[1 * n + i] += 0.0;
       C.cons[2 * n + i] += 0.0;
       C.cons[3 * n + i] += 0.0;
@@ -2460,7 +2519,7 @@ __global__ void k_init_ic(Batch B, int s, int64_t lo, int64_t hi, const double* 
   }
   st5(C.cons, n, i, c);
   st5(C.prim, n, i, prim);
-  flush_events(ev, B.cnt, B.eng, s);
+  flush_events(ev, B.cnt, &B.eng[s].err);
 }
 
 // Space::status sums (space.rs:1248-1280) over cells [lo, hi): one block, fixed-order tree reduction.

@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_clear(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  if (!D.vmesh || !B.eng[s].stepping) return;
+  if (!D.vmesh || !B.st[s].stepping) return;
   const int64_t gi = (int64_t)J.lo + threadIdx.x;
   if (gi >= J.hi) return;
   const int64_t k = D.cell_base + s + (gi - D.cell_base);
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_bin(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  if (!D.vmesh || !B.eng[s].stepping) return;
+  if (!D.vmesh || !B.st[s].stepping) return;
   const int64_t gi = (int64_t)J.lo + threadIdx.x;
   if (gi >= J.hi) return;
   const int64_t N = B.C.n;
@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_scan_up(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  if (!D.vmesh || !B.eng[s].stepping) return;
+  if (!D.vmesh || !B.st[s].stepping) return;
   int64_t len;
   const int32_t* a = v2_scan_region<A>(V, D, s, len);
   const int64_t k = (int64_t)J.lo - D.cell_base + threadIdx.x;
@@ -159,8 +159,8 @@ template <int A>
 __global__ void __launch_bounds__(HFV_SCAN_BLOCK) k_v2_scan_mid(Batch B, V2Bufs V) {
   const int s = blockIdx.x;
   const SimDesc& D = B.sims[s];
-  SimEngine& E = B.eng[s];
-  if (!D.vmesh || !E.stepping) return;
+  SimStep& S = B.st[s];
+  if (!D.vmesh || !S.stepping) return;
   int64_t len;
   int32_t* a = v2_scan_region<A>(V, D, s, len);
   __shared__ int32_t wsum[HFV_SCAN_BLOCK / 64];
@@ -190,15 +190,15 @@ __global__ void __launch_bounds__(HFV_SCAN_BLOCK) k_v2_scan_mid(Batch B, V2Bufs 
   if (threadIdx.x == 0) {
     a[len] = carry;
     tot_s = carry;
-    if (A == 1) E.nf_mesh = E.err ? 0 : carry;  // a failed cell emitted nothing: the simulation stops
+    if (A == 1) B.eng[s].nf_mesh = S.err ? 0 : carry;  // a failed cell emitted nothing: the simulation stops
     if (A == 2 && carry > D.conn_cap) {
       atomicCAS(&B.cnt->err, 0, E_MESH);
-      atomicCAS(&E.err, 0, E_MESH);
+      atomicCAS(&S.err, 0, E_MESH);
     }
   }
   __syncthreads();
   if (A == 2) {  // offsets past the last cell: the slot's end of the CSR
-    const int32_t end = (int32_t)D.conn_base + (E.err ? 0 : tot_s);
+    const int32_t end = (int32_t)D.conn_base + (S.err ? 0 : tot_s);
     for (int64_t k = D.n + threadIdx.x; k < D.noff; k += blockDim.x) B.F.off[D.cell_base + k] = end;
   }
 }
@@ -209,8 +209,8 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_scan_down(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  const SimEngine& E = B.eng[s];
-  if (!D.vmesh || !E.stepping) return;
+  const SimStep& S = B.st[s];
+  if (!D.vmesh || !S.stepping) return;
   int64_t len;
   int32_t* a = v2_scan_region<A>(V, D, s, len);
   const int64_t k = (int64_t)J.lo - D.cell_base + threadIdx.x;
@@ -220,7 +220,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_scan_down(Batch B, V2Bufs V) {
   a[k] = x;
   if (A == 0) V.gfill[D.cell_base + s + k] = x;
   if (A == 2) {
-    const int32_t o = (int32_t)D.conn_base + (E.err ? 0 : x);
+    const int32_t o = (int32_t)D.conn_base + (S.err ? 0 : x);
     B.F.off[D.cell_base + k] = o;
     V.cfill[D.cell_base + k] = o;
   }
@@ -231,7 +231,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_place(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  if (!D.vmesh || !B.eng[s].stepping) return;
+  if (!D.vmesh || !B.st[s].stepping) return;
   const int64_t gi = (int64_t)J.lo + threadIdx.x;
   if (gi >= J.hi) return;
   const int32_t p = atomicAdd(&V.gfill[D.cell_base + s + V.gkey[gi]], 1);
@@ -279,7 +279,7 @@ __device__ __forceinline__ bool v2_emits(const Batch& B, int64_t cb, int32_t nb,
 // Cell2::finish), the emitted faces appended to vf in edge order, and the cell's geometry
 // (Particle::update_geometry, part.rs:151-158).
 template <int TL>
-__device__ void v2_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimEngine& E, int s, int64_t gi,
+__device__ void v2_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int s, int64_t gi,
                           int32_t i, double xi, double yi, double zi, const V2TeamPoly<TL>& P, int m) {
   const int64_t N = B.C.n, cb = D.cell_base;
   double area = 0., cx = 0., cy = 0., r2 = 0.;
@@ -296,11 +296,11 @@ __device__ void v2_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, Sim
     const double q = bxx * bxx + byy * byy;
     r2 = r2 < q ? q : r2;
   }
-  const int32_t start = atomicAdd(&E.nf_tmp, cnt);
+  const int32_t start = atomicAdd(&S.nf_tmp, cnt);
   if ((int64_t)start + cnt > D.face_cap) {
     V.femit[cb + s + i] = 0;
     atomicCAS(&B.cnt->err, 0, E_MESH);
-    atomicCAS(&E.err, 0, E_MESH);
+    atomicCAS(&S.err, 0, E_MESH);
     return;
   }
   V.vst[gi] = start;
@@ -626,8 +626,8 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_cells(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  SimEngine& E = B.eng[s];
-  if (D.vmesh != 2 || !E.stepping) return;
+  SimStep& S = B.st[s];
+  if (D.vmesh != 2 || !S.stepping) return;
   const int team = threadIdx.x / HFV_V2_TEAM, lane = threadIdx.x % HFV_V2_TEAM;
   const int tiw = (threadIdx.x & 63) / HFV_V2_TEAM;
   const int64_t gi = (int64_t)J.lo + (blockIdx.x % HFV_V2_SUB) * (HFV_BLOCK / HFV_V2_TEAM) + team;
@@ -649,9 +649,9 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_cells(Batch B, V2Bufs V) {
   } else if (r != 0) {
     V.femit[cb + s + i] = 0;
     atomicCAS(&B.cnt->err, 0, E_MESH);
-    atomicCAS(&E.err, 0, E_MESH);
+    atomicCAS(&S.err, 0, E_MESH);
   } else {
-    v2_finish(B, V, D, E, s, gi, i, xi, yi, zi, P, m);
+    v2_finish(B, V, D, S, s, gi, i, xi, yi, zi, P, m);
   }
 }
 
@@ -661,13 +661,13 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  const SimEngine& E = B.eng[s];
-  if (!D.vmesh || !E.stepping) return;
+  const SimStep& S = B.st[s];
+  if (!D.vmesh || !S.stepping) return;
   const int64_t f = (int64_t)J.lo + threadIdx.x;
   if (f >= J.hi) return;
   Faces& F = B.F;
   const int64_t fl = f - D.face_base, cb = D.cell_base, NF = F.nf, N = B.C.n;
-  if (fl >= E.nf_mesh) {
+  if (fl >= B.eng[s].nf_mesh) {
     F.left[f] = -1;
     F.right[f] = -1;
     return;
@@ -700,10 +700,10 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_csr_fill(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  const SimEngine& E = B.eng[s];
-  if (!D.vmesh || !E.stepping || E.err) return;
+  const SimStep& S = B.st[s];
+  if (!D.vmesh || !S.stepping || S.err) return;
   const int64_t f = (int64_t)J.lo + threadIdx.x;
-  if (f >= J.hi || f - D.face_base >= E.nf_mesh) return;
+  if (f >= J.hi || f - D.face_base >= B.eng[s].nf_mesh) return;
   const int32_t l = B.F.left[f], r = B.F.right[f];
   int32_t p = atomicAdd(&V.cfill[l], 1);
   B.F.conn[p] = (int32_t)(f << 1);
@@ -723,8 +723,8 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_csr_sort(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  SimEngine& E = B.eng[s];
-  if (!D.vmesh || !E.stepping || E.err) return;
+  SimStep& S = B.st[s];
+  if (!D.vmesh || !S.stepping || S.err) return;
   const int64_t gi = (int64_t)J.lo + threadIdx.x;
   if (gi >= J.hi) return;  // (no block barrier follows)
   const int32_t e0 = B.F.off[gi], e1 = B.F.off[gi + 1];

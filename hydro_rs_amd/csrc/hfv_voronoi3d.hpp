@@ -667,7 +667,7 @@ __device__ int v3_build(const Batch& B, const SimDesc& D, const V2Bufs& V, int s
 // Cell3::finish on the clipped cell.  Returns 0, 1 (a periodic cell touching the initial region: retry
 // with a larger K) or 3 (a face of more than HFV_V3_FAN vertices); on 0 the faces and the geometry are
 // written.
-__device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimEngine& E, int s, int64_t gi, int32_t i,
+__device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int s, int64_t gi, int32_t i,
                          double xi, double yi, double zi, V3Cell& C, int np, int nt, double r2) {
   const int lane = __lane_id();
   const int p = lane;
@@ -783,13 +783,13 @@ __device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimE
   const uint64_t me = __ballot(emit);
   const int cnt = __popcll(me);
   int start = 0;
-  if (lane == 0) start = atomicAdd(&E.nf_tmp, cnt);
+  if (lane == 0) start = atomicAdd(&S.nf_tmp, cnt);
   start = __shfl(start, 0, 64);
   if ((int64_t)start + cnt > D.face_cap) {
     if (lane == 0) {
       V.femit[cb + s + i] = 0;
       atomicCAS(&B.cnt->err, 0, E_MESH);
-      atomicCAS(&E.err, 0, E_MESH);
+      atomicCAS(&S.err, 0, E_MESH);
     }
     return 0;
   }
@@ -837,8 +837,8 @@ __global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V) {
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  SimEngine& E = B.eng[s];
-  if (D.vmesh != 3 || !E.stepping) return;
+  SimStep& S = B.st[s];
+  if (D.vmesh != 3 || !S.stepping) return;
   const int64_t gi = (int64_t)J.lo + blockIdx.x % HFV_BLOCK;
   if (gi >= J.hi) return;
   if (!B.C.act[gi]) return;  // unbuilt in a partial build (femit stays 0)
@@ -850,12 +850,12 @@ __global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V) {
   double r2 = 0.;
   for (int K = 2; K <= kmax && r == 1; ++K) {
     r = v3_build(B, D, V, s, i, xi, yi, zi, K, C, np, nt, r2);
-    if (r == 0) r = v3_finish(B, V, D, E, s, gi, i, xi, yi, zi, C, np, nt, r2);
+    if (r == 0) r = v3_finish(B, V, D, S, s, gi, i, xi, yi, zi, C, np, nt, r2);
   }
   if (r != 0 && __lane_id() == 0) {
     V.femit[cb + s + i] = 0;
     atomicCAS(&B.cnt->err, 0, E_MESH);
-    atomicCAS(&E.err, 0, E_MESH);
+    atomicCAS(&S.err, 0, E_MESH);
   }
 }
 

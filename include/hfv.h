@@ -347,9 +347,9 @@ int hfv_get_launch_shape(hfv_ctx* ctx, int* flux_faces_per_thread, double* ns_pe
 
 /* ---------------------------------------------------------------- measurement */
 /* Device time of the step's kernels, from HIP events recorded on the context's stream around each
- * launch (no counterpart in the reference, which has no device).  Slots: 0 mask+predict, 1 mesh
- * rebuild (moving meshes), 2 face flux, 3 accumulate+c2p, 4 gradients+timestep, 5 limiter
- * wakeup, 6 limiter+kick1, 7 drift. */
+ * launch (no counterpart in the reference, which has no device).  Slots: 0 drift+mask+predict, 1 mesh
+ * rebuild (moving meshes), 2 face flux, 3 accumulate+c2p, 4 gradients+timestep, 5 the minimum bin of
+ * sync_all simulations, 6 limiter (wakeup, limit, kick1) and the end of the step, 7 unused (part of 0). */
 #define HFV_NUM_KERNEL_SLOTS 8
 typedef struct {
   int64_t launches[HFV_NUM_KERNEL_SLOTS];
