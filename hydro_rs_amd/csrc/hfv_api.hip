@@ -175,6 +175,7 @@ struct hfv_ctx {
   std::vector<int> loaded;
   std::vector<SimDesc> desc;           // host copy
   std::vector<int64_t> ccap, fcap, kcap, cbase, fbase, kbase;
+  std::vector<int64_t> sebase, secap;  // sliced gradient geometry (Faces::soff): base and capacity per slot
   std::vector<int64_t> nused, fused, kused;
   int64_t n = 0, nf = 0, nconn = 0;    // capacities (totals)
   Cells C{};
@@ -186,6 +187,8 @@ struct hfv_ctx {
   // launched grid sizes: positions holding the chunks of live slots (loaded, and in a batch not finished),
   // rounded up to 8; the block tables are rebuilt without finished slots as they finish
   int64_t ncg = 8, nfg = 8, live_chunks = 0;
+  int cgsh = 0, fgsh = 0;     // log2 of the group sizes that the tables were dealt in
+  int64_t face_items = 0;     // faces that the only simulation's face kernels cover
   std::vector<BlockJob> hcjobs, hfjobs;
   BlockJob *dcjobs = nullptr, *dfjobs = nullptr;
   Partials P{};
@@ -197,6 +200,7 @@ struct hfv_ctx {
   std::vector<int> v_zero;   // per slot: every particle velocity is +0 (fixed meshes keep it so)
   std::vector<int> has_stage;  // per slot: some face chunk has a staging list
   std::vector<int> has_gstage;  // per slot: some cell chunk has a neighbour staging list
+  std::vector<int> has_slices;  // per slot: the mesh's CSR rows fit its sliced gradient geometry
   // per slot, set by hfv_autotune / hfv_set_tuning: LDS-staged flux tiling allowed (1) or not (0);
   // precomputed gradient geometry and LDS-staged gradient neighbours on (1), off (0) or by dimension
   // (-1: on for 3D)
@@ -243,8 +247,9 @@ struct hfv_ctx {
     B.eng = deng;
     B.st = dst;
     B.nsims = nslots;
-    B.cjobs = dcjobs;
-    B.fjobs = dfjobs;
+    // one simulation of its own: jobs by arithmetic
+    B.cjobs = JobGrid{dcjobs, batch || !loaded[0] ? 0 : (int32_t)nused[0], cgsh};
+    B.fjobs = JobGrid{dfjobs, batch || !loaded[0] ? 0 : (int32_t)face_items, fgsh};
     B.P = P;
     B.cnt = dcnt;
     B.fall = fall;
@@ -284,23 +289,30 @@ void drop_graph(hfv_ctx* c) {
   c->graph_ok = false;
 }
 
-// Buffers of the 2D device rebuild for the whole capacity (hfv_voronoi2d.hpp), on first need.
+// Buffers of the 2D and 3D device rebuilds for the whole capacity (hfv_voronoi2d.hpp), on first need.
 int ensure_v2(hfv_ctx* c) {
   if (c->v2_alloc) return HFV_OK;
   const int64_t ns = c->n + c->nslots + 1;
   V2Bufs v;
   v.gcnt = dalloc<int32_t>(c, ns);
   v.gfill = dalloc<int32_t>(c, ns);
-  v.femit = dalloc<int32_t>(c, ns);
-  v.ccnt = dalloc<int32_t>(c, ns);
+  v.femit = dalloc<int32_t>(c, c->n);
+  v.ccnt = dalloc<int32_t>(c, c->n);
   v.gord = dalloc<int32_t>(c, c->n);
   v.gkey = dalloc<int32_t>(c, c->n);
   v.vst = dalloc<int32_t>(c, c->n);
-  v.cfill = dalloc<int32_t>(c, c->n);
   v.vf = dalloc<V2Face>(c, c->nf);
-  v.part = dalloc<int32_t>(c, c->ncchunk);
-  if (!v.gcnt || !v.gfill || !v.femit || !v.ccnt || !v.gord || !v.gkey || !v.vst || !v.cfill || !v.vf || !v.part)
-    return set_err(HFV_ERR_HIP, "out of device memory (2D rebuild buffers)");
+  v.bkt = dalloc<uint64_t>(c, HFV_BUCKET * c->n);
+  v.over = dalloc<V2Over>(c, c->nconn);
+  v.part0 = dalloc<int32_t>(c, c->ncchunk);
+  v.part1 = dalloc<int32_t>(c, c->ncchunk);
+  v.part2 = dalloc<int32_t>(c, c->ncchunk);
+  if (!v.gcnt || !v.gfill || !v.femit || !v.ccnt || !v.gord || !v.gkey || !v.vst || !v.vf || !v.bkt || !v.over ||
+      !v.part0 || !v.part1 || !v.part2)
+    return set_err(HFV_ERR_HIP, "out of device memory (rebuild buffers)");
+  HIP_OK(hipMemsetAsync(v.gcnt, 0, sizeof(int32_t) * ns, c->stream));
+  HIP_OK(hipMemsetAsync(v.vst, 0, sizeof(int32_t) * c->n, c->stream));
+  HIP_OK(hipStreamSynchronize(c->stream));
   c->v2 = v;
   c->v2_alloc = true;
   drop_graph(c);  // a captured step holds the old buffer set
@@ -372,6 +384,12 @@ int write_jobs(hfv_ctx* c) {
   const int64_t gc = group_size(c, lc), gf = group_size(c, lf);
   const int64_t ncg = grid_size(lc, gc), nfg = grid_size(lf, gf);
   if (ncg != c->ncg || nfg != c->nfg) drop_graph(c);  // the step graph holds the grid sizes
+  const int cgsh = __builtin_ctzll((uint64_t)gc), fgsh = __builtin_ctzll((uint64_t)gf);
+  const int64_t items = c->batch || !c->loaded[0] ? 0 : face_range(c, 0);
+  if (cgsh != c->cgsh || fgsh != c->fgsh || items != c->face_items) drop_graph(c);
+  c->cgsh = cgsh;
+  c->fgsh = fgsh;
+  c->face_items = items;
   c->ncg = ncg;
   c->nfg = nfg;
   c->live_chunks = lc;
@@ -464,7 +482,6 @@ int alloc_batch(hfv_ctx* c) {
   F.off = dalloc<int32_t>(c, n + 1);
   F.conn = dalloc<int32_t>(c, nk);
   F.nbr = dalloc<int32_t>(c, nk);
-  F.cur = dalloc<uint8_t>(c, nf);
   // chunks: a slot's cell capacity and face capacity in blocks of BLOCK items
   c->cchunk0.assign(S, 0);
   c->fchunk0.assign(S, 0);
@@ -497,12 +514,28 @@ int alloc_batch(hfv_ctx* c) {
   F.gcell = dalloc<int32_t>(c, ncc * HFV_GSTAGE_MAX);
   F.gcnt = dalloc<uint16_t>(c, ncc);
   F.nloc = dalloc<uint16_t>(c, nk);
-  C.minv = dalloc<double>(c, 9 * n);
-  F.eg = dalloc<double>(c, 8 * nk);
+  C.minv = dalloc<double>(c, 6 * n);
+  // sliced gradient geometry: a slot's slices hold the longest of their 64 cells' CSR rows each; a mesh
+  // whose slices need more than this evaluates its gradient geometry per step
+  c->sebase.assign(S, 0);
+  c->secap.assign(S, 0);
+  int64_t nse = 0;
+  for (int s = 0; s < S; ++s) {
+    c->sebase[s] = nse;
+    c->secap[s] = (c->kcap[s] + c->kcap[s] / 2 + 64 * 8) / 64 * 64;
+    nse += c->secap[s];
+  }
+  F.nse = nse;
+  F.soff = dalloc<int64_t>(c, 4 * ncc);
+  F.seref = dalloc<int32_t>(c, nse);
+  F.secode = dalloc<uint8_t>(c, nse);
+  F.sew = dalloc<double>(c, nse);
+  F.sedx = dalloc<double>(c, 3 * nse);
   F.fs = dalloc<double>(c, 4 * nf);
   c->v_zero.assign(S, 1);
   c->has_stage.assign(S, 0);
   c->has_gstage.assign(S, 0);
+  c->has_slices.assign(S, 0);
   c->tune_stage.assign(S, -1);
   c->tune_sgrad.assign(S, -1);
   c->tune_gstage.assign(S, -1);
@@ -526,7 +559,6 @@ int alloc_batch(hfv_ctx* c) {
   HIP_OK(hipMemsetAsync(C.bin, 0, (size_t)n, st));
   HIP_OK(hipMemsetAsync(C.nbin, HFV_NO_BIN, (size_t)n, st));
   HIP_OK(hipMemsetAsync(C.act, 0, (size_t)n, st));
-  HIP_OK(hipMemsetAsync(F.cur, 0, (size_t)nf, st));
   HIP_OK(hipMemsetAsync(c->P.act, 0, sizeof(uint32_t) * (size_t)ncc, st));
   HIP_OK(hipMemsetAsync(c->P.face, 0, sizeof(uint32_t) * (size_t)nfc, st));
   HIP_OK(hipMemsetAsync(c->P.ti, 0xFF, sizeof(uint64_t) * (size_t)ncc, st));
@@ -781,6 +813,20 @@ int upload_mesh(hfv_ctx* c, int s, const hfv_mesh_arrays* m, const uint8_t* upda
       HIP_OK(hipMemcpyAsync(F.gcnt + k0, gcnt.data(), sizeof(uint16_t) * ncch, hipMemcpyHostToDevice, st));
     }
     if (tot) HIP_OK(hipMemcpyAsync(F.nloc + kb, nloc.data(), sizeof(uint16_t) * tot, hipMemcpyHostToDevice, st));
+    // the bases of the sliced gradient geometry: each slice of 64 cells holds its longest CSR row per cell
+    {
+      std::vector<int64_t> soff(4 * ncch, c->sebase[s]);
+      int64_t used = 0;
+      for (int64_t w = 0; w < 4 * ncch; ++w) {
+        soff[w] = c->sebase[s] + used;
+        int64_t longest = 0;
+        for (int64_t i = 64 * w; i < std::min<int64_t>(64 * (w + 1), n); ++i) longest = std::max<int64_t>(longest, m->count[i]);
+        used += 64 * longest;
+      }
+      c->has_slices[s] = used <= c->secap[s] ? 1 : 0;
+      HIP_OK(hipMemcpyAsync(F.soff + 4 * c->cchunk0[s], soff.data(), sizeof(int64_t) * 4 * ncch, hipMemcpyHostToDevice, st));
+      HIP_OK(hipStreamSynchronize(st));
+    }
     // the other cell chunks each cell chunk's neighbours lie in (k_apply's idle test); meshes that change
     // on the device (2D moving) keep 0xFF: their chunks always run
     {
@@ -808,6 +854,7 @@ int upload_mesh(hfv_ctx* c, int s, const hfv_mesh_arrays* m, const uint8_t* upda
       HIP_OK(hipMemcpyAsync(F.nch + k0 * HFV_NCH_MAX, nch.data(), sizeof(int32_t) * cap_ch * HFV_NCH_MAX,
                             hipMemcpyHostToDevice, st));
       HIP_OK(hipMemcpyAsync(F.nchn + k0, nchn.data(), (size_t)cap_ch, hipMemcpyHostToDevice, st));
+      HIP_OK(hipStreamSynchronize(st));  // (the lists end with this block)
     }
     c->has_gstage[s] = std::any_of(gcnt.begin(), gcnt.end(), [](uint16_t k) { return k > 0; }) ? 1 : 0;
     HIP_OK(hipStreamSynchronize(st));
@@ -859,6 +906,8 @@ int upload_mesh(hfv_ctx* c, int s, const hfv_mesh_arrays* m, const uint8_t* upda
   if (D.vmesh) {
     TRY(v_grid(p, n, D));
     TRY(ensure_v2(c));
+    // (a step that stopped halfway, or another simulation, leaves no counts behind)
+    HIP_OK(hipMemsetAsync(c->v2.gcnt + cb + s, 0, sizeof(int32_t) * (n + 1), st));
     c->heng[s].nf_mesh = (int)nf;
     HIP_OK(hipMemcpyAsync(&c->deng[s].nf_mesh, &c->heng[s].nf_mesh, sizeof(int), hipMemcpyHostToDevice, st));
     HIP_OK(hipStreamSynchronize(st));
@@ -913,7 +962,8 @@ int refresh_geometry(hfv_ctx* c, int s) {
   const hfv_params& p = c->params[s];
   const bool st = c->use_static && p.motion == HFV_FIXED && c->v_zero[s] && c->nused[s] > 0;
   c->desc[s].static_geom = st ? 1 : 0;
-  c->desc[s].static_grad = st && (c->tune_sgrad[s] < 0 ? p.dim == 3 : c->tune_sgrad[s] != 0) ? 1 : 0;
+  c->desc[s].static_grad =
+      st && c->has_slices[s] && (c->tune_sgrad[s] < 0 ? p.dim == 3 : c->tune_sgrad[s] != 0) ? 1 : 0;
   // LDS tiling of the flux kernel: by default in 2D/3D; a 1D chunk's faces and cells are already
   // contiguous, so staging there only adds work (512-member ensemble: 2.56e9 -> 2.63e9 without it)
   c->desc[s].staged = st && c->has_stage[s] && (c->tune_stage[s] < 0 ? p.dim != 1 : c->tune_stage[s] != 0) ? 1 : 0;
@@ -1061,8 +1111,8 @@ void launch_grad(hfv_ctx* c, const Batch& B, int do_grad, int do_ts) {
 
 void launch_mask(hfv_ctx* c, const Batch& B, int mode) {
   const dim3 g((unsigned)c->ncg), b(BLOCK);
-  if (c->any_moving) hipLaunchKernelGGL(k_mask<true>, g, b, 0, c->stream, B, mode);
-  else hipLaunchKernelGGL(k_mask<false>, g, b, 0, c->stream, B, mode);
+  if (c->any_moving) hipLaunchKernelGGL(k_mask<true>, g, b, 0, c->stream, B, c->v2, mode);
+  else hipLaunchKernelGGL(k_mask<false>, g, b, 0, c->stream, B, c->v2, mode);
 }
 
 void launch_sync_min(hfv_ctx* c, const Batch& B) {
@@ -1084,30 +1134,14 @@ void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
   }
   if (c->any_vmesh) {
     const V2Bufs& V = c->v2;
-    const dim3 gs((unsigned)c->nslots), gsb(HFV_SCAN_BLOCK);
-    hipLaunchKernelGGL(k_v2_clear, gc, gb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_bin, gc, gb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_scan_up<0>, gc, gb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_scan_mid<0>, gs, gsb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_scan_down<0>, gc, gb, 0, st, B, V);
+    hipLaunchKernelGGL(k_v2_sum<0>, gc, gb, 0, st, B, V);
+    hipLaunchKernelGGL(k_v2_bins, gc, gb, 0, st, B, V);
     hipLaunchKernelGGL(k_v2_place, gc, gb, 0, st, B, V);
-    if (c->any_vmesh2) {
-      hipLaunchKernelGGL(k_v2_cells<false>, dim3((unsigned)(c->ncg * HFV_V2_SUB)), gb, 0, st, B, V);
-      hipLaunchKernelGGL(k_v2_cells<true>, dim3((unsigned)(c->ncg * HFV_V2_SUB)), gb, 0, st, B, V);
-    }
-    if (c->any_vmesh3) {
-      const dim3 g3((unsigned)(c->ncg * BLOCK)), w3(64);
-      hipLaunchKernelGGL(k_v3_cells, g3, w3, 0, st, B, V);
-    }
-    hipLaunchKernelGGL(k_v2_scan_up<1>, gc, gb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_scan_mid<1>, gs, gsb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_scan_down<1>, gc, gb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_faces, gf, gb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_scan_up<2>, gc, gb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_scan_mid<2>, gs, gsb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_scan_down<2>, gc, gb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_csr_fill, gf, gb, 0, st, B, V);
-    hipLaunchKernelGGL(k_v2_csr_sort, gc, gb, 0, st, B, V);
+    if (c->any_vmesh2) hipLaunchKernelGGL(k_v2_cells, dim3((unsigned)(c->ncg * HFV_V2_SUB)), gb, 0, st, B, V);
+    if (c->any_vmesh3) hipLaunchKernelGGL(k_v3_cells, dim3((unsigned)(c->ncg * BLOCK)), dim3(64), 0, st, B, V);
+    hipLaunchKernelGGL(k_v2_faces, gc, gb, 0, st, B, V);
+    hipLaunchKernelGGL(k_v2_sum<1>, gc, gb, 0, st, B, V);
+    hipLaunchKernelGGL(k_v2_conn, gc, gb, 0, st, B, V);
   }
 }
 

@@ -15,8 +15,8 @@
 //     fr[N][32] (AoS flux record of static-geometry cells, HFV_FR_*: prim, time-extrapolation rate,
 //     sound speed, gradients, dt, gc; two 128-byte lines staged whole by the flux kernel)
 //   faces, SoA: area, nrm[3], fcen[3], left (int32), right (int32, -1 = wall), shc (uint8 periodic
-//     shift code, 2 bits per axis), cur (uint8: record of this step); rec[F][8] (AoS, one 64-byte line
-//     per face: dt*F[5], v_max, a_over_r, unused)
+//     shift code, 2 bits per axis); rec[F][8] (AoS, one 64-byte line per face: dt*F[5], v_max, a_over_r,
+//     unused; current where a cell of the face is active)
 //   csr: off[N+1] (int32), conn[2F] (int32: face << 1 | side, side 1 = the cell is the face's right),
 //     nbr[2F] (int32: the face's other cell, -1 for a wall)
 //   staging lists: per face chunk its distinct cells (scell, scnt), per face its cells' list slots
@@ -34,6 +34,8 @@
 #pragma once
 #include "hfv_physics.hpp"
 
+#define HFV_BLOCK 256
+
 namespace hfv {
 
 struct Cells {
@@ -44,7 +46,7 @@ struct Cells {
   uint64_t* tiex;  // [N] FP32-flux contexts: the predict clock (SimEngine::ti_pred) at which extrap is due
   // extrap, tex and grad hold floats (same layouts) in FP32-flux contexts: ld_ex/st_ex/ld_tex/st_tex/
   // ld_grad/st_grad
-  double* minv;  // [9][N] inverse of the gradient matrix (static geometry only)
+  double* minv;  // [6][N] inverse of the (symmetric) gradient matrix: xx xy xz yy yz zz (static gradient geometry only)
   double* fr;    // [N][HFV_FR_W] flux inputs of static-geometry cells (layout: HFV_FR_*)
   double* dtq;   // [N] requested timesteps of the trait-level compute_timesteps (before timesteps_apply)
   int8_t* bin;
@@ -57,8 +59,16 @@ struct Faces {
   double *area, *nrm, *fcen, *rec;
   int32_t *left, *right, *off, *conn;
   int32_t* nbr;  // per CSR entry: the face's other cell (-1: wall)
-  uint8_t *shc, *cur;
-  double* eg;    // [2F][8] per CSR entry: w, ds[3], dxf[3] (static gradient geometry only)
+  uint8_t* shc;
+  // Static gradient geometry, in slices: the entries of the 64 cells of a wave, entry k of lane l at
+  // soff[4 chunk + wave] + 64 k + l, so that a wave reads whole lines and no address waits for a load.  Per
+  // entry the neighbour (its cell, or its stage slot where the chunk stages; -1: wall), the shift code with
+  // the side in bit 6, the weight area / |ds|^2 and the face offset dxf[3] (component stride nse).
+  int64_t nse;
+  int64_t* soff;
+  int32_t* seref;
+  uint8_t* secode;
+  double *sew, *sedx;
   double* fs;    // [F][4] per face: dx_centroid[3], a_over_r (static geometry only)
   // LDS staging of the flux kernel: per face chunk, its distinct cells (scell[chunk][HFV_STAGE_MAX],
   // ascending) and their count (scnt, 0 = more than HFV_STAGE_MAX: no staging); per face, the local
@@ -116,6 +126,27 @@ struct BlockJob {
   int32_t sim, lo, hi, chunk;
 };
 
+// The block table of the cell or the face kernels (the grid is its number of entries).  A context of one
+// simulation works its jobs out from the block index instead of loading them (n items, chunks dealt to the
+// XCDs in groups of 1 << gsh as grid_position deals them): one cold load less at the head of every kernel.
+struct JobGrid {
+  const BlockJob* jobs;
+  int32_t n;  // 0: by table
+  int32_t gsh;
+  __device__ __forceinline__ BlockJob operator[](uint32_t b) const {
+    if (!n) return jobs[b];
+    const uint32_t q = b >> 3;
+    const uint32_t j = ((((q >> gsh) << 3) + (b & 7u)) << gsh) + (q & ((1u << gsh) - 1u));
+    const int64_t lo = (int64_t)j * HFV_BLOCK;
+    BlockJob J;
+    J.sim = lo < n ? 0 : -1;
+    J.lo = (int32_t)lo;
+    J.hi = (int32_t)(lo + HFV_BLOCK < n ? lo + HFV_BLOCK : n);
+    J.chunk = (int32_t)j;
+    return J;
+  }
+};
+
 #define HFV_MAX_SUBDRIFTS 8
 #define HFV_NO_BIN 127  // nbin of a cell that is not active: beyond every wakeup
 #define HFV_NCH_MAX 8
@@ -157,7 +188,7 @@ struct SimStep {
   int min_bin;   // sync_all: the smallest new bin
   int n_down;    // 1D periodic moving meshes: faces of this step's rebuild where the generator order steps down
   int nf_tmp;    // 2D/3D moving meshes: the rebuild's provisional face cursor
-  int pad_;
+  int n_over;    // 2D/3D moving meshes: CSR entries beyond their cells' buckets in this step's rebuild
 };
 
 // Batch-global counters (soft events; the first hard error of any simulation).
@@ -182,8 +213,8 @@ struct Batch {
   SimEngine* eng;
   SimStep* st;
   int nsims;
-  const BlockJob* cjobs;  // cell kernels: grid = number of entries
-  const BlockJob* fjobs;  // face kernels
+  JobGrid cjobs;  // cell kernels
+  JobGrid fjobs;  // face kernels
   Partials P;
   DevCounters* cnt;
   int2* fall;  // (face, simulation) queued for k_flux_fallback
@@ -223,7 +254,6 @@ static_assert(HFV_FR32_EL < HFV_FR32_LDS, "staged FP32 record words");
 
 #define HFV_NUM_TIME_BINS 56
 #define HFV_MAX_NR_TIMESTEPS (1ull << 57)
-#define HFV_BLOCK 256
 
 // ------------------------------------------------------------------ timeline (src/timeline.rs)
 __device__ __host__ __forceinline__ uint64_t get_integer_timestep(int bin) {
@@ -247,10 +277,10 @@ __device__ __host__ __forceinline__ uint64_t get_integer_time_end(uint64_t ti_cu
   return ti_current - m + dti;
 }
 __device__ __host__ __forceinline__ int8_t get_max_active_bin(uint64_t ti) {
+  // the first bin from 1 whose bit bin + 1 is set, 62 where there is none
   if (ti == 0) return HFV_NUM_TIME_BINS;
-  int bin = 1;
-  while (bin < 62 && ((1ull << (bin + 1)) & ti) == 0) bin += 1;
-  return (int8_t)bin;
+  const uint64_t t = ti & ~3ull;
+  return (int8_t)(t ? __builtin_ctzll(t) - 1 : 62);
 }
 __device__ __host__ __forceinline__ uint64_t sat_u64(double x) {
   if (!(x > 0.)) return 0;
@@ -571,7 +601,7 @@ constexpr bool flux_stages() {
 #ifndef HFV_GRAD_CHUNK
 #define HFV_GRAD_CHUNK 4
 #endif
-// CSR entries of a cell whose loads (CSR value, face flag, record) k_apply issues together: 4 against a
+// CSR entries of a cell whose loads (CSR value, record) k_apply issues together: 4 against a
 // three-stage pipeline, KH 128^3 accumulation -6% (FP64) / -27% (FP32 flux); 6 and 8 gained 0.3% more on
 // KH at occupancy 3 and cost the ensemble 2%
 #ifndef HFV_APPLY_CHUNK
@@ -676,7 +706,7 @@ __device__ __forceinline__ SimStep step_begin(const SimEngine& E) {
   S.min_bin = 127;
   S.n_down = 0;
   S.nf_tmp = 0;
-  S.pad_ = 0;
+  S.n_over = 0;
   if (E.err) {  // a hard error stops this simulation only; the batch's other simulations go on
     S.done = 1;
   } else if (E.force) {  // hfv_step: a step at ti_current with the caller's ti_old
@@ -890,6 +920,57 @@ __device__ void drift_cell(const Cells& C, const Cfg& cfg, const SimStep& S, int
   }
 }
 
+// ------------------------------------------------------------------ 2D/3D moving meshes: the rebuild's buffers
+// (hfv_voronoi2d.hpp) and its bin counts
+// A face in the provisional order: area (length in 2D), centroid and unit normal relative to the emitting
+// generator, the neighbour's local index (< 0: a wall) and periodic image code.
+struct V2Face {
+  double area, cx, cy, cz, nx, ny, nz;
+  int32_t nb, code;
+};
+
+// CSR entries a cell's bucket holds between k_v2_faces and k_v2_conn (further ones go to a list that the
+// cells concerned search): a random 3D mesh has 15.5 faces a cell, one cell in a hundred has more than 24
+#define HFV_BUCKET 24
+// An entry beyond its cell's bucket.
+struct V2Over {
+  int32_t cell, conn, nbr;
+};
+
+struct V2Bufs {
+  int32_t* gcnt;   // [N + S + 1], simulation s at cell_base + s: bin counts, then bin starts (nbins + 1); zero
+                   // between the steps
+  int32_t* gfill;  // same layout: placement cursors
+  int32_t* gord;   // [N] at cell_base: local cell indices grouped by bin
+  int32_t* gkey;   // [N] bin of each cell
+  int32_t* femit;  // [N] faces a cell emits
+  int32_t* vst;    // [N] start of a cell's faces in vf
+  int32_t* ccnt;   // [N] CSR entries per cell
+  V2Face* vf;      // [F] at face_base: faces in provisional order
+  uint64_t* bkt;   // [HFV_BUCKET][N] entries of a cell: (CSR value << 32) | neighbour
+  V2Over* over;    // [CSR capacity] at conn_base: entries beyond their cells' buckets
+  int32_t* part0;  // [cell chunks] sums of gcnt over the chunk's bins
+  int32_t* part1;  // [cell chunks] sums of femit over the chunk's cells
+  int32_t* part2;  // [cell chunks] sums of ccnt
+};
+
+__device__ __forceinline__ int v2_bin(double x, double w, int nb) {
+  int b = (int)floor(x / w);
+  if (b < 0) b = 0;
+  if (b >= nb) b = nb - 1;
+  return b;
+}
+
+// Counts the generator of cell gi (by k_mask, after its drift) into its bin.
+__device__ __forceinline__ void v_count_bin(const Batch& B, const V2Bufs& V, const SimDesc& D, int s, int64_t gi) {
+  const int64_t N = B.C.n;
+  const int key = (v2_bin(B.C.loc[gi], D.vw[0], D.vnb[0]) * D.vnb[1] + v2_bin(B.C.loc[N + gi], D.vw[1], D.vnb[1])) *
+                      D.vnb[2] +
+                  (D.vmesh == 3 ? v2_bin(B.C.loc[2 * N + gi], D.vw[2], D.vnb[2]) : 0);
+  V.gkey[gi] = key;
+  atomicAdd(&V.gcnt[D.cell_base + s + key], 1);
+}
+
 // ------------------------------------------------------------------ k_mask
 // The step of every simulation from its engine (step_begin), the drift of moving generators through the
 // step's sync points (engine.rs:152-185), the active mask (optimal_order.rs:17) and the predict
@@ -901,7 +982,7 @@ __device__ void drift_cell(const Cells& C, const Cfg& cfg, const SimStep& S, int
 // the sums and adds dt_pred at once.
 // MOVING: the context holds moving meshes (the fixed ones' kernel carries no drift registers).
 template <bool MOVING>
-__global__ void __launch_bounds__(HFV_BLOCK) k_mask(Batch B, int mode) {
+__global__ void __launch_bounds__(HFV_BLOCK) k_mask(Batch B, V2Bufs V, int mode) {
   if (blockIdx.x == 0 && threadIdx.x == 0) B.cnt->nfall = 0;
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
@@ -929,6 +1010,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mask(Batch B, int mode) {
       G.min_bin = S.min_bin;
       G.n_down = S.n_down;
       G.nf_tmp = S.nf_tmp;
+      G.n_over = S.n_over;
     }
     if (!S.stepping) return;
   }
@@ -949,6 +1031,9 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mask(Batch B, int mode) {
       }
     });
     if (!fits) ev.fail(E_UNSUPPORTED);
+  }
+  if constexpr (MOVING) {
+    if (mode == 0 && valid && B.sims[s].vmesh) v_count_bin(B, V, B.sims[s], s, i);
   }
   if (valid) {
     if (mode != 1) {
@@ -1365,7 +1450,8 @@ __device__ __forceinline__ void store_rec(double* rec, int64_t f, const double* 
   dst[3] = make_double2(outv[6], 0.);
 }
 
-// Faces with an active cell get their record (zero when gated off) and cur = 1; the others cur = 0.
+// Faces with an active cell get their record (zero when gated off); the others keep an old one, which
+// nothing reads.
 // With SOLVER == AIRS, faces that need the exact solver are queued for k_flux_fallback.
 // STATIC: when the chunk has a staging list and a face with an active cell, the block stages its
 // distinct cells' flux records and extrapolations in LDS by whole lines (each cell is read once per
@@ -1398,18 +1484,14 @@ __device__ __forceinline__ void flux_chunk(const Batch& B, const BlockJob J) {
   bool la = false, ra = false;
   int32_t myc = 0;
   if (STATIC && (int)threadIdx.x < ns) myc = B.F.scell[(uint64_t)J.chunk * HFV_STAGE_MAX + threadIdx.x];
-  if (f < J.hi) {
+  // a device-rebuilt mesh (dynamic geometry only) ends before the range that the grid covers
+  const int64_t fhi = !STATIC && B.sims[s].vmesh ? B.sims[s].face_base + B.eng[s].nf_mesh : J.hi;
+  if (f < J.hi && f < fhi) {
     l = B.F.left[f];
     r = B.F.right[f];
-    if (!STATIC && l < 0) {  // past a device-rebuilt mesh's faces (dynamic geometry only): no cells
-      l = 0;
-      r = -1;
-    } else {
-      la = B.C.act[l];
-      ra = r >= 0 && B.C.act[r];
-      cur = la || ra;
-    }
-    B.F.cur[f] = cur ? 1 : 0;
+    la = B.C.act[l];
+    ra = r >= 0 && B.C.act[r];
+    cur = la || ra;
   }
   if (STATIC) {
     if ((int)threadIdx.x < ns) scl[threadIdx.x] = myc;
@@ -1637,16 +1719,18 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_apply(Batch B, int mode) {
   bool have_prim = false;
   St<double> prim;
   if (mode & 1) {
-    St<double> acc = vacuum<double>();
+    St<double> acc = vacuum<double>(), cons0 = vacuum<double>();
     bool have = false;
-    double msv = 0., maor = 0.;
-    if (a) {
+    double msv = 0., maor = 0., vol = 0.;
+    const int32_t k0 = F.off[i], k1 = F.off[i + 1];
+    if (a) {  // all in flight with the first CSR values
       acc = ld5(C.facc, n, i);
-      have = true;
+      cons0 = ld5(C.cons, n, i);
       msv = C.msv[i];
       maor = C.maor[i];
+      vol = C.vol[i];
+      have = true;
     }
-    const int32_t k0 = F.off[i], k1 = F.off[i + 1];
     // a face's record: its five fluxes, v_max and a_over_r
     auto load_rec = [&](uint32_t f, St<double>& r, double& vmx, double& aor) {
       if (f32) {
@@ -1663,23 +1747,41 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_apply(Batch B, int mode) {
         aor = r67.x;
       }
     };
-    // Entries in chunks: a chunk's CSR values, then its faces' flags, then the records of its current
-    // faces, all in flight together before the chunk's entries are applied in CSR order.
+    // Entries in chunks: the records of a chunk's current faces with the next chunk's CSR values, all in
+    // flight together before the chunk's entries are applied in CSR order.  Every face of an active cell is
+    // current; an inactive cell's where its other cell is active (the face kernel's gate, from one byte of
+    // the neighbour, so that no flag per face is written or read: a cell waits for its CSR values and its
+    // records only).
+    int32_t cv[HFV_APPLY_CHUNK];
+#pragma unroll
+    for (int u = 0; u < HFV_APPLY_CHUNK; ++u) cv[u] = k0 + u < k1 ? F.conn[k0 + u] : -1;
     for (int32_t kb = k0; kb < k1; kb += HFV_APPLY_CHUNK) {
-      int32_t cv[HFV_APPLY_CHUNK];
+      bool cf[HFV_APPLY_CHUNK];
 #pragma unroll
-      for (int u = 0; u < HFV_APPLY_CHUNK; ++u) cv[u] = kb + u < k1 ? F.conn[kb + u] : 0;
-      uint32_t cf[HFV_APPLY_CHUNK];
+      for (int u = 0; u < HFV_APPLY_CHUNK; ++u) cf[u] = cv[u] >= 0;
+      if (!a) {
+        int32_t o[HFV_APPLY_CHUNK];
 #pragma unroll
-      for (int u = 0; u < HFV_APPLY_CHUNK; ++u) cf[u] = kb + u < k1 ? (uint32_t)F.cur[(uint32_t)(cv[u] >> 1)] : 0u;
+        for (int u = 0; u < HFV_APPLY_CHUNK; ++u) o[u] = cf[u] ? F.nbr[kb + u] : -1;
+#pragma unroll
+        for (int u = 0; u < HFV_APPLY_CHUNK; ++u) cf[u] = o[u] >= 0 && C.act[o[u]];
+      }
       St<double> rc[HFV_APPLY_CHUNK];
       double vm[HFV_APPLY_CHUNK], ao[HFV_APPLY_CHUNK];
+      uint32_t side = 0;
+      int32_t nx[HFV_APPLY_CHUNK];
 #pragma unroll
       for (int u = 0; u < HFV_APPLY_CHUNK; ++u) {
         rc[u] = vacuum<double>();
         vm[u] = 0.;
         ao[u] = 0.;
         if (cf[u]) load_rec((uint32_t)(cv[u] >> 1), rc[u], vm[u], ao[u]);
+        side |= (uint32_t)(cv[u] & 1) << u;
+      }
+#pragma unroll
+      for (int u = 0; u < HFV_APPLY_CHUNK; ++u) {
+        const int32_t k = kb + HFV_APPLY_CHUNK + u;
+        nx[u] = k < k1 ? F.conn[k] : -1;
       }
 #pragma unroll
       for (int u = 0; u < HFV_APPLY_CHUNK; ++u) {
@@ -1688,7 +1790,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_apply(Batch B, int mode) {
           acc = ld5(C.facc, n, i);
           have = true;
         }
-        if ((cv[u] & 1) == 0)
+        if (((side >> u) & 1u) == 0)
           acc = acc - rc[u];
         else
           acc = acc + rc[u];
@@ -1697,10 +1799,12 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_apply(Batch B, int mode) {
           maor = hmax(maor, ao[u]);
         }
       }
+#pragma unroll
+      for (int u = 0; u < HFV_APPLY_CHUNK; ++u) cv[u] = nx[u];
     }
     if (have) {
       if (a) {
-        St<double> cc = ld5(C.cons, n, i) + acc;  // apply_flux (part.rs:178-193)
+        St<double> cc = cons0 + acc;  // apply_flux (part.rs:178-193)
 #pragma unroll
         for (int q = 0; q < 5; ++q)
           if (!hfinite(cc.c[q])) ev.fail(E_NONFINITE);
@@ -1721,7 +1825,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_apply(Batch B, int mode) {
         C.msv[i] = msv;
         C.maor[i] = maor;
         if (mode & 2) {
-          prim = c2p(cc, C.vol[i], cfg.gd, ev);
+          prim = c2p(cc, vol, cfg.gd, ev);
           st5(C.prim, n, i, prim);
           have_prim = true;
         }
@@ -1838,13 +1942,16 @@ __device__ __forceinline__ void boundary_neighbour(const Faces& F, const Cfg& cf
 // fused with compute_timesteps (euler_eqns_fvs.rs:50-61, part.rs:42-84, 328-372) and timesteps_apply
 // (hydrodynamics.rs:145-158, timeline.rs:103-139) for an active cell.  The limiter's neighbour min/max
 // is gathered in the estimate sweep (same values, same order); the second sweep only extrapolates.
-// STATIC (fixed 3D mesh): the per-entry weight w, offset ds and face offset dxf, and the inverse of the
-// gradient matrix, are the values k_geom_cells computed once with the same expressions and order.  (On
-// 1D/2D meshes recomputing them reads fewer bytes than the precomputed lines, so those stay dynamic.)
+// STATIC (fixed mesh): the per-entry weight w and face offset dxf, and the inverse of the gradient matrix, are
+// the values k_geom_cells computed once with the same expressions and order; sb is the base of the wave's
+// slice of them.  Whole lines per load and no dependent address: KH 128^3 (FP32 flux, LDS-staged
+// neighbours) 796 -> 572 us against the per-step geometry and 861 -> 572 against the geometry as one 64-byte
+// line per entry; in 1D and 2D the neighbours' gathers dominate and the per-step geometry stays the default
+// (509^2 vortex 70 us per step against 76 with slices).
 template <bool STATIC>
 __device__ __forceinline__ void grad_cell(const Batch& B, const Cfg& cfg, const SimStep& S, int64_t i, int do_grad,
                                           int do_ts, bool pack_fr, double* frv, bool v_zero, const double4* gst,
-                                          uint64_t* dti_out, Events& ev) {
+                                          int64_t sb, uint64_t* dti_out, Events& ev) {
   const Cells& C = B.C;
   const Faces& F = B.F;
   const int64_t n = C.n, nf = F.nf;
@@ -1878,46 +1985,51 @@ __device__ __forceinline__ void grad_cell(const Batch& B, const Cfg& cfg, const 
       __builtin_amdgcn_sched_barrier(0);
     };
     if (STATIC) {
-      // entries in chunks of HFV_GRAD_CHUNK: a chunk's neighbour references (LDS stage slot when staged,
-      // else its cell; -1 at a wall) and geometry lines in flight together, then its entries in order
-      for (int32_t kb = k0; kb < k1; kb += HFV_GRAD_CHUNK) {
-        int32_t rr[HFV_GRAD_CHUNK];
-        double4 ag[HFV_GRAD_CHUNK];
+      // the next chunk's slice entries are in flight while a chunk's are accumulated in order
+      const uint32_t cnt = (uint32_t)(k1 - k0);
+      const int32_t* R = F.seref + sb;
+      const uint8_t* Q = F.secode + sb;
+      const double* W = F.sew + sb;
+      int32_t rr[HFV_GRAD_CHUNK];
+      uint32_t cc[HFV_GRAD_CHUNK];
+      double ww[HFV_GRAD_CHUNK];
+      auto load = [&](uint32_t kb) {
 #pragma unroll
-        for (int u = 0; u < HFV_GRAD_CHUNK; ++u) {
-          const int32_t k = kb + u;
-          if (k < k1) {
-            if (gst) {
-              const uint32_t li = F.nloc[k];
-              rr[u] = li == 0xFFFFu ? -1 : (int32_t)li;
-            } else {
-              rr[u] = F.nbr[k];
-            }
-            ag[u] = ((const double4*)(F.eg + 8 * (uint64_t)(uint32_t)k))[0];
-          } else {
-            rr[u] = -1;
-            ag[u] = make_double4(0., 0., 0., 0.);
-          }
+        for (uint32_t u = 0; u < HFV_GRAD_CHUNK; ++u) {
+          const bool in = kb + u < cnt;
+          const uint32_t e = 64u * (kb + u) + __lane_id();
+          rr[u] = in ? R[e] : -1;
+          cc[u] = in ? (uint32_t)Q[e] : 0u;
+          ww[u] = in ? W[e] : 0.;
         }
+      };
+      load(0);
+      for (uint32_t kb = 0; kb < cnt; kb += HFV_GRAD_CHUNK) {
+        int32_t rc[HFV_GRAD_CHUNK];
+        uint32_t qc[HFV_GRAD_CHUNK];
+        double wc[HFV_GRAD_CHUNK];
 #pragma unroll
         for (int u = 0; u < HFV_GRAD_CHUNK; ++u) {
-          const int32_t k = kb + u;
-          if (k >= k1) break;
-          const int32_t other = rr[u];
-          const double4 a = ag[u];
-          const double w = a.x;
-          const V3<double> ds = mk3(a.y, a.z, a.w);
-          St<double> op;
+          rc[u] = rr[u];
+          qc[u] = cc[u];
+          wc[u] = ww[u];
+        }
+        load(kb + HFV_GRAD_CHUNK);
+#pragma unroll
+        for (int u = 0; u < HFV_GRAD_CHUNK; ++u) {
+          if (kb + u >= cnt) break;
+          const int32_t other = rc[u];
+          St<double> op = prim;
+          V3<double> oc = cen;
           if (other >= 0) {
-            V3<double> oc;
             if (gst) load_pc((const double*)(gst + 2 * (uint32_t)other), 0, op, oc);
             else load_pc(C.pc, (uint32_t)other, op, oc);
           } else {
-            op = prim;  // Space::get_boundary_part (space.rs:213-229)
-            if (cfg.boundary == BND_REFLECTIVE) op = reflect(prim, ld3(F.nrm, nf, (uint32_t)(F.conn[k] >> 1)));
-            else if (cfg.boundary == BND_VACUUM) op = vacuum<double>();
+            boundary_neighbour(F, cfg, (uint32_t)(F.conn[k0 + kb + u] >> 1), cen, prim, oc, op);
           }
-          accumulate(op, ds, w);
+          const V3<double> sh = decode_shift((uint8_t)(qc[u] & 63u), cfg.box);
+          const V3<double> shift = (qc[u] & 64u) == 0 ? sh : -sh;
+          accumulate(op, (oc + shift) - cen, wc[u]);
         }
       }
     } else {
@@ -1982,9 +2094,12 @@ __device__ __forceinline__ void grad_cell(const Batch& B, const Cfg& cfg, const 
     {
       M3 inv;
       if (STATIC) {
-        inv.x = mk3(ldo(C.minv, (uint32_t)i), ldo(C.minv + n, (uint32_t)i), ldo(C.minv + 2 * n, (uint32_t)i));
-        inv.y = mk3(ldo(C.minv + 3 * n, (uint32_t)i), ldo(C.minv + 4 * n, (uint32_t)i), ldo(C.minv + 5 * n, (uint32_t)i));
-        inv.z = mk3(ldo(C.minv + 6 * n, (uint32_t)i), ldo(C.minv + 7 * n, (uint32_t)i), ldo(C.minv + 8 * n, (uint32_t)i));
+        const double xx = ldo(C.minv, (uint32_t)i), xy = ldo(C.minv + n, (uint32_t)i), xz = ldo(C.minv + 2 * n, (uint32_t)i),
+                     yy = ldo(C.minv + 3 * n, (uint32_t)i), yz = ldo(C.minv + 4 * n, (uint32_t)i),
+                     zz = ldo(C.minv + 5 * n, (uint32_t)i);
+        inv.x = mk3(xx, xy, xz);
+        inv.y = mk3(xy, yy, yz);
+        inv.z = mk3(xz, yz, zz);
       } else {
         M3 m;
         m.x = mk3(mxx, mxy, mxz);
@@ -2025,15 +2140,26 @@ __device__ __forceinline__ void grad_cell(const Batch& B, const Cfg& cfg, const 
       }
     };
     if (STATIC) {
-      for (int32_t kb = k0; kb < k1; kb += HFV_GRAD_CHUNK) {  // chunks of lines in flight together
-        double4 bg[HFV_GRAD_CHUNK];
+      const uint32_t cnt = (uint32_t)(k1 - k0);
+      const double *X = F.sedx + sb, *Y = X + F.nse, *Z = Y + F.nse;
+      V3<double> bg[HFV_GRAD_CHUNK];
+      auto load = [&](uint32_t kb) {
 #pragma unroll
-        for (int u = 0; u < HFV_GRAD_CHUNK; ++u)
-          bg[u] = kb + u < k1 ? ((const double4*)(F.eg + 8 * (uint64_t)(uint32_t)(kb + u)))[1] : make_double4(0., 0., 0., 0.);
+        for (uint32_t u = 0; u < HFV_GRAD_CHUNK; ++u) {
+          const uint32_t e = 64u * (kb + u) + __lane_id();
+          bg[u] = kb + u < cnt ? mk3(X[e], Y[e], Z[e]) : mk3(0., 0., 0.);
+        }
+      };
+      load(0);
+      for (uint32_t kb = 0; kb < cnt; kb += HFV_GRAD_CHUNK) {
+        V3<double> bc[HFV_GRAD_CHUNK];
+#pragma unroll
+        for (int u = 0; u < HFV_GRAD_CHUNK; ++u) bc[u] = bg[u];
+        load(kb + HFV_GRAD_CHUNK);
 #pragma unroll
         for (int u = 0; u < HFV_GRAD_CHUNK; ++u) {
-          if (kb + u >= k1) break;
-          extrema(mk3(bg[u].x, bg[u].y, bg[u].z));
+          if (kb + u >= cnt) break;
+          extrema(bc[u]);
         }
       }
     } else {
@@ -2218,7 +2344,7 @@ __global__ void __launch_bounds__(HFV_BLOCK, HFV_GRAD_WAVES) k_grad(Batch B, int
   double frv[HFV_FR_W];
   if (a)
     grad_cell<STATIC>(B, cfg, S, i, do_grad, do_ts, pack, frv, B.sims[s].static_geom != 0, staged ? lds4 : nullptr,
-                      &my, ev);
+                      STATIC ? B.F.soff[4 * (int64_t)J.chunk + (threadIdx.x >> 6)] : 0, &my, ev);
   if (pack) {
     if (staged) __syncthreads();  // the staged lines are dead from here on
     double* wbuf = (double*)lds4 + (threadIdx.x >> 6) * (64 * 17);
@@ -2322,7 +2448,8 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_geom_cells(Batch B, int s, int64_
   if (i >= hi) return;
   const Cells& C = B.C;
   const Faces& F = B.F;
-  const Cfg& cfg = B.sims[s].cfg;
+  const SimDesc& D = B.sims[s];
+  const Cfg& cfg = D.cfg;
   const int64_t n = C.n, nf = F.nf;
   const V3<double> cen = ld3(C.cen, n, i);
   const St<double> prim = ld5(C.prim, n, i);
@@ -2336,11 +2463,15 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_geom_cells(Batch B, int s, int64_
   } else if (cfg.dim == 2) {
     m.z.z = 1.;
   }
+  const int32_t chunk = D.cchunk0 + (int32_t)((i - lo) / HFV_BLOCK);
+  const bool slots = D.gstaged && F.gcnt[chunk] > 0;  // the gradient kernel's own test
+  const int64_t e0 = F.soff[4 * (int64_t)chunk + (threadIdx.x >> 6)] + (threadIdx.x & 63);
   const int32_t k0 = F.off[i], k1 = F.off[i + 1];
   for (int32_t k = k0; k < k1; ++k) {
     const int32_t e = F.conn[k];
     const uint32_t f = (uint32_t)(e >> 1);
-    const V3<double> sh = decode_shift(F.shc[f], cfg.box);
+    const uint8_t code = F.shc[f];
+    const V3<double> sh = decode_shift(code, cfg.box);
     const V3<double> shift = (e & 1) == 0 ? sh : -sh;
     const int32_t other = F.nbr[k];
     V3<double> oc;
@@ -2353,14 +2484,20 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_geom_cells(Batch B, int s, int64_
     m.y = m.y + (w * (ds.y * ds));
     m.z = m.z + (w * (ds.z * ds));
     const V3<double> dxf = (ld3(F.fcen, nf, f) - cen) - shift;
-    double4* eg = (double4*)(F.eg + 8 * (uint64_t)(uint32_t)k);
-    eg[0] = make_double4(w, ds.x, ds.y, ds.z);
-    eg[1] = make_double4(dxf.x, dxf.y, dxf.z, 0.);
+    const int64_t q = e0 + 64 * (int64_t)(k - k0);
+    F.seref[q] = slots && other >= 0 ? (int32_t)F.nloc[k] : other;
+    F.secode[q] = (uint8_t)(code | ((e & 1) << 6));
+    F.sew[q] = w;
+    F.sedx[q] = dxf.x;
+    F.sedx[F.nse + q] = dxf.y;
+    F.sedx[2 * F.nse + q] = dxf.z;
   }
+  // the matrix is symmetric bit for bit (w (a b) == w (b a), summed in the same order), and its cofactor
+  // inverse too: six distinct entries
   const M3 inv = inverse_cols(m);
-  const double v[9] = {inv.x.x, inv.x.y, inv.x.z, inv.y.x, inv.y.y, inv.y.z, inv.z.x, inv.z.y, inv.z.z};
+  const double v[6] = {inv.x.x, inv.x.y, inv.x.z, inv.y.y, inv.y.z, inv.z.z};
 #pragma unroll
-  for (int q = 0; q < 9; ++q) C.minv[q * n + i] = v[q];
+  for (int q = 0; q < 6; ++q) C.minv[q * n + i] = v[q];
 }
 __global__ void __launch_bounds__(HFV_BLOCK) k_geom_faces(Batch B, int s, int64_t flo, int64_t fhi) {
   const int64_t f = flo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2456,7 +2593,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_limit(Batch B, int phase) {
     dt = C.dt[i];
     const uint64_t ti_current = S.ti_current;
     const double time_base = S.time_base;
-    if (bin <= get_max_active_bin(ti_current)) {
+    if (bin <= S.mab) {
       bin = (int8_t)wakeup;
       dt = (double)get_integer_timestep(bin) * time_base;
     } else {

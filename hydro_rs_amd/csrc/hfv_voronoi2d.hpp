@@ -14,14 +14,20 @@
 // CSR lists its faces in ascending face index.
 //
 // Per step (simulations with vmesh = 2, while stepping; 3D: hfv_voronoi3d.hpp), after the drift and the predict:
-//   k_v2_clear, k_v2_bin, scan<0>, k_v2_place          the bin grid (counting sort of the generators)
-//   k_v2_cells<0>, k_v2_cells<1>                       the active cells' polygons, volume,
-//                                                      centroid and search radius (Particle::
-//                                                      update_geometry, part.rs:151-158); the cell's
-//                                                      emitted faces in a provisional order
-//   scan<1>, k_v2_faces                                face indices in cell order, the face arrays
-//   scan<2>, k_v2_csr_fill, k_v2_csr_sort              offsets and CSR entries in ascending face order
-// (scan<A>: k_v2_scan_up, k_v2_scan_mid, k_v2_scan_down)
+//   k_mask (v_count_bin)        bin counts of the generators
+//   k_v2_sum<0>, k_v2_bins,
+//   k_v2_place                  bin starts; the generators grouped by bin (a counting sort)
+//   k_v2_cells (3D: k_v3_cells) the active cells' polygons, volume, centroid and search radius
+//                               (Particle::update_geometry, part.rs:151-158); the cell's emitted faces in a
+//                               provisional order, and the chunk sums of their counts
+//   k_v2_faces                  face indices in cell order, the face arrays, each cell's CSR entries in its
+//                               bucket
+//   k_v2_sum<1>, k_v2_conn      CSR offsets; the entries in ascending face order
+// Each prefix sum over cells (or bins) is two levels: a kernel before leaves the sums of the chunks of
+// HFV_BLOCK elements, and every block of the kernel that needs the sum adds up the chunks before its own
+// (chunks_before) and scans its chunk.  The rebuild was 18 launches of 4-5 us each (counts, sums,
+// scans, fill and sort apart) and is 7 in 2D: a 125^2 vortex with steered generators 218 -> 202 us a step,
+// a Sedov 256^2 run to t = 0.004 121 -> 111.5 ms.
 // Inactive cells keep their geometry and get new CSR ranges (the reference's note at space.rs:233-235).
 #pragma once
 
@@ -31,33 +37,6 @@ namespace hfv {
 // A clip removes the vertices beyond a plane by more than this fraction of its offset (the host
 // tessellator's threshold): vertices on it test as beyond by a rounding error on exact lattices.
 #define HFV_CLIP_TOL 1e-12
-
-// A face in the provisional order: area (length in 2D), centroid and unit normal relative to the emitting
-// generator, the neighbour's local index (< 0: a wall) and periodic image code.
-struct V2Face {
-  double area, cx, cy, cz, nx, ny, nz;
-  int32_t nb, code;
-};
-
-struct V2Bufs {
-  int32_t* gcnt;   // [N + S + 1], simulation s at cell_base + s: bin counts, then bin starts (nbins + 1)
-  int32_t* gfill;  // same layout: placement cursors
-  int32_t* gord;   // [N] at cell_base: local cell indices grouped by bin
-  int32_t* gkey;   // [N] bin of each cell
-  int32_t* femit;  // [N + S + 1]: faces a cell emits, then their exclusive offsets (the total at [n])
-  int32_t* vst;    // [N] start of a cell's faces in vf
-  int32_t* ccnt;   // [N + S + 1]: CSR entries per cell, then exclusive offsets
-  int32_t* cfill;  // [N] CSR fill cursors (global entry index)
-  V2Face* vf;      // [F] at face_base: faces in provisional order
-  int32_t* part;   // [cell chunks] chunk sums, then chunk offsets, of the prefix sums
-};
-
-__device__ __forceinline__ int v2_bin(double x, double w, int nb) {
-  int b = (int)floor(x / w);
-  if (b < 0) b = 0;
-  if (b >= nb) b = nb - 1;
-  return b;
-}
 
 // (squared distance, index, image code) order; the code compares as the host's memcmp of int8 codes
 __device__ __forceinline__ bool v2_less(double ad2, int32_t aj, int32_t ak, double bd2, int32_t bj, int32_t bk) {
@@ -70,55 +49,7 @@ __device__ __forceinline__ int32_t v2_shift_code(int s0, int s1) {
   return (s0 == 1 ? 1 : s0 == -1 ? 2 : 0) | ((s1 == 1 ? 1 : s1 == -1 ? 2 : 0) << 2);
 }
 
-// ---------------------------------------------------------------- bin grid
-__global__ void __launch_bounds__(HFV_BLOCK) k_v2_clear(Batch B, V2Bufs V) {
-  const BlockJob J = B.cjobs[blockIdx.x];
-  if (J.sim < 0) return;
-  const int s = J.sim;
-  const SimDesc& D = B.sims[s];
-  if (!D.vmesh || !B.st[s].stepping) return;
-  const int64_t gi = (int64_t)J.lo + threadIdx.x;
-  if (gi >= J.hi) return;
-  const int64_t k = D.cell_base + s + (gi - D.cell_base);
-  V.gcnt[k] = 0;
-  V.ccnt[k] = 0;
-  V.femit[k] = 0;
-  if (gi == D.cell_base) {  // entry n (bins: nbins <= n)
-    V.gcnt[D.cell_base + s + D.n] = 0;
-    V.ccnt[D.cell_base + s + D.n] = 0;
-    V.femit[D.cell_base + s + D.n] = 0;
-  }
-}
-
-__global__ void __launch_bounds__(HFV_BLOCK) k_v2_bin(Batch B, V2Bufs V) {
-  const BlockJob J = B.cjobs[blockIdx.x];
-  if (J.sim < 0) return;
-  const int s = J.sim;
-  const SimDesc& D = B.sims[s];
-  if (!D.vmesh || !B.st[s].stepping) return;
-  const int64_t gi = (int64_t)J.lo + threadIdx.x;
-  if (gi >= J.hi) return;
-  const int64_t N = B.C.n;
-  const int key = (v2_bin(B.C.loc[gi], D.vw[0], D.vnb[0]) * D.vnb[1] + v2_bin(B.C.loc[N + gi], D.vw[1], D.vnb[1])) *
-                      D.vnb[2] +
-                  (D.vmesh == 3 ? v2_bin(B.C.loc[2 * N + gi], D.vw[2], D.vnb[2]) : 0);
-  V.gkey[gi] = key;
-  atomicAdd(&V.gcnt[D.cell_base + s + key], 1);
-}
-
 // ---------------------------------------------------------------- prefix sums
-// Exclusive prefix sums over a simulation's region of one of three arrays, in three launches over the
-// cell block table (chunks of HFV_BLOCK elements): k_v2_scan_up sums each chunk, k_v2_scan_mid (one block
-// per simulation) scans the chunk sums and stores the total after the region, k_v2_scan_down scans each
-// chunk from its offset.  A: 0 bin counts (length nbins; the bin starts, copied to the placement
-// cursors), 1 emitted faces per cell (length n; the face offsets, the total is the mesh's face count),
-// 2 CSR entries per cell (length n; the CSR offsets of the cells).
-template <int A>
-__device__ __forceinline__ int32_t* v2_scan_region(const V2Bufs& V, const SimDesc& D, int s, int64_t& len) {
-  len = A == 0 ? (int64_t)D.vnb[0] * D.vnb[1] * D.vnb[2] : D.n;
-  return (A == 0 ? V.gcnt : A == 1 ? V.femit : V.ccnt) + D.cell_base + s;
-}
-
 // exclusive scan of one value per thread over a block of HFV_BLOCK threads; *total receives the sum
 __device__ __forceinline__ int32_t block_excl_scan(int32_t v, int32_t* total) {
   __shared__ int32_t ws[HFV_BLOCK / 64];
@@ -140,90 +71,75 @@ __device__ __forceinline__ int32_t block_excl_scan(int32_t v, int32_t* total) {
   return before + x - v;
 }
 
-template <int A>
-__global__ void __launch_bounds__(HFV_BLOCK) k_v2_scan_up(Batch B, V2Bufs V) {
+// The sum of the simulation's chunk sums before chunk `chunk`, and of all of them (every thread gets both).
+// Each block reads every chunk sum: at most a few thousand words that the L2 holds, where a launch of its
+// own to scan them costs 4-5 us.
+__device__ __forceinline__ int32_t chunks_before(const int32_t* part, const SimDesc& D, int32_t chunk, int32_t* total) {
+  __shared__ int32_t wb[HFV_BLOCK / 64], wt[HFV_BLOCK / 64];
+  int32_t b = 0, t = 0;
+  for (int32_t c = D.cchunk0 + (int32_t)threadIdx.x; c < D.cchunk1; c += HFV_BLOCK) {
+    const int32_t v = part[c];
+    t += v;
+    if (c < chunk) b += v;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    b += __shfl_xor(b, o);
+    t += __shfl_xor(t, o);
+  }
+  if (__lane_id() == 0) {
+    wb[threadIdx.x >> 6] = b;
+    wt[threadIdx.x >> 6] = t;
+  }
+  __syncthreads();
+  b = 0;
+  t = 0;
+#pragma unroll
+  for (int w = 0; w < HFV_BLOCK / 64; ++w) {
+    b += wb[w];
+    t += wt[w];
+  }
+  __syncthreads();
+  *total = t;
+  return b;
+}
+
+// Chunk sums of the bin counts (CSR 0) or of the cells' CSR entries (CSR 1).  (Added up by the counting
+// atomics instead, they put hundreds of atomics on one address: 10-100 us.)
+template <int CSR>
+__global__ void __launch_bounds__(HFV_BLOCK) k_v2_sum(Batch B, V2Bufs V) {
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
   if (!D.vmesh || !B.st[s].stepping) return;
-  int64_t len;
-  const int32_t* a = v2_scan_region<A>(V, D, s, len);
   const int64_t k = (int64_t)J.lo - D.cell_base + threadIdx.x;
-  int32_t tot;
-  block_excl_scan(k < len ? a[k] : 0, &tot);
-  if (threadIdx.x == 0) V.part[J.chunk] = tot;
+  const int64_t len = CSR ? D.n : (int64_t)D.vnb[0] * D.vnb[1] * D.vnb[2];
+  const int32_t* a = CSR ? V.ccnt + D.cell_base : V.gcnt + D.cell_base + s;
+  const uint32_t t = block_sum_u32(k < len ? (uint32_t)a[k] : 0u);
+  if (threadIdx.x == 0) (CSR ? V.part2 : V.part0)[J.chunk] = (int32_t)t;
 }
 
-template <int A>
-__global__ void __launch_bounds__(HFV_SCAN_BLOCK) k_v2_scan_mid(Batch B, V2Bufs V) {
-  const int s = blockIdx.x;
-  const SimDesc& D = B.sims[s];
-  SimStep& S = B.st[s];
-  if (!D.vmesh || !S.stepping) return;
-  int64_t len;
-  int32_t* a = v2_scan_region<A>(V, D, s, len);
-  __shared__ int32_t wsum[HFV_SCAN_BLOCK / 64];
-  __shared__ int32_t tot_s;
-  // the chunk sums, HFV_SCAN_BLOCK at a time: wave scans, then the waves' totals
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  int32_t carry = 0;
-  for (int32_t c0 = D.cchunk0; c0 < D.cchunk1; c0 += blockDim.x) {
-    const int32_t c = c0 + (int32_t)threadIdx.x;
-    const int32_t v = c < D.cchunk1 ? V.part[c] : 0;
-    int32_t x = v;
-    for (int o = 1; o < 64; o <<= 1) {
-      const int32_t y = __shfl_up(x, o, 64);
-      if (lane >= o) x += y;
-    }
-    if (lane == 63) wsum[wid] = x;
-    __syncthreads();
-    int32_t before = 0, tot = 0;
-    for (int w = 0; w < nw; ++w) {
-      if (w < wid) before += wsum[w];
-      tot += wsum[w];
-    }
-    if (c < D.cchunk1) V.part[c] = carry + before + x - v;
-    carry += tot;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    a[len] = carry;
-    tot_s = carry;
-    if (A == 1) B.eng[s].nf_mesh = S.err ? 0 : carry;  // a failed cell emitted nothing: the simulation stops
-    if (A == 2 && carry > D.conn_cap) {
-      atomicCAS(&B.cnt->err, 0, E_MESH);
-      atomicCAS(&S.err, 0, E_MESH);
-    }
-  }
-  __syncthreads();
-  if (A == 2) {  // offsets past the last cell: the slot's end of the CSR
-    const int32_t end = (int32_t)D.conn_base + (S.err ? 0 : tot_s);
-    for (int64_t k = D.n + threadIdx.x; k < D.noff; k += blockDim.x) B.F.off[D.cell_base + k] = end;
-  }
-}
-
-template <int A>
-__global__ void __launch_bounds__(HFV_BLOCK) k_v2_scan_down(Batch B, V2Bufs V) {
+// Bin starts and placement cursors; the chunk sums of the emitted faces restart at zero.
+__global__ void __launch_bounds__(HFV_BLOCK) k_v2_bins(Batch B, V2Bufs V) {
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
-  const SimStep& S = B.st[s];
-  if (!D.vmesh || !S.stepping) return;
-  int64_t len;
-  int32_t* a = v2_scan_region<A>(V, D, s, len);
+  if (!D.vmesh || !B.st[s].stepping) return;
+  if (threadIdx.x == 0) V.part1[J.chunk] = 0;
+  const int64_t nbins = (int64_t)D.vnb[0] * D.vnb[1] * D.vnb[2];  // <= n
   const int64_t k = (int64_t)J.lo - D.cell_base + threadIdx.x;
-  int32_t tot;
-  const int32_t x = V.part[J.chunk] + block_excl_scan(k < len ? a[k] : 0, &tot);
-  if (k >= len) return;
-  a[k] = x;
-  if (A == 0) V.gfill[D.cell_base + s + k] = x;
-  if (A == 2) {
-    const int32_t o = (int32_t)D.conn_base + (S.err ? 0 : x);
-    B.F.off[D.cell_base + k] = o;
-    V.cfill[D.cell_base + k] = o;
+  int32_t* a = V.gcnt + D.cell_base + s;
+  const int32_t v = k < nbins ? a[k] : 0;
+  int32_t all, tot;
+  const int32_t base = chunks_before(V.part0, D, J.chunk, &all);
+  const int32_t x = base + block_excl_scan(v, &tot);
+  if (k < nbins) {
+    a[k] = x;
+    V.gfill[D.cell_base + s + k] = x;
   }
+  if (J.chunk == D.cchunk1 - 1 && threadIdx.x == 0) a[nbins] = all;
 }
 
 __global__ void __launch_bounds__(HFV_BLOCK) k_v2_place(Batch B, V2Bufs V) {
@@ -243,9 +159,9 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_place(Batch B, V2Bufs V) {
 // testing, moving and intersecting every TEAM-th edge; the next candidate in (squared distance, index,
 // image code) order is a team minimum over the lanes' smallest keys above the last one, each lane taking
 // every TEAM-th bin of the (2K+1)^2 block.  k_v2_cells keeps each lane's candidates in registers (at most
-// HFV_V2_TC) and polygons of up to HFV_V2_TL edges; cells that outgrow either go to k_v2_cells_wide,
-// which rescans the bins for every candidate and holds polygons of up to HFV_V2_TLW edges.  Both make the
-// host tessellator's operations in its order, so the same bits.
+// HFV_V2_TC) and polygons of up to HFV_V2_TL edges; cells that outgrow either are built again, rescanning
+// the bins for every candidate, with polygons of up to HFV_V2_TLW edges.  Both make the host tessellator's
+// operations in its order, so the same bits.
 // 16 lanes per cell: 205 us per step on Sedov 256^2 with steered generators, against 325 with 8 and 217
 // with 32 (the rebuild is latency-bound: few active cells per step, each team's chain of clips)
 #ifndef HFV_V2_TEAM
@@ -261,7 +177,6 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_place(Batch B, V2Bufs V) {
 #define HFV_V2_TC 8
 #endif
 #define HFV_V2_SUB HFV_V2_TEAM  // blocks per cell chunk
-#define HFV_V2_WIDE (-1)         // femit mark: the cell goes to k_v2_cells_wide
 
 template <int TL>
 struct V2TeamPoly {
@@ -279,7 +194,7 @@ __device__ __forceinline__ bool v2_emits(const Batch& B, int64_t cb, int32_t nb,
 // Cell2::finish), the emitted faces appended to vf in edge order, and the cell's geometry
 // (Particle::update_geometry, part.rs:151-158).
 template <int TL>
-__device__ void v2_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int s, int64_t gi,
+__device__ void v2_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int chunk, int64_t gi,
                           int32_t i, double xi, double yi, double zi, const V2TeamPoly<TL>& P, int m) {
   const int64_t N = B.C.n, cb = D.cell_base;
   double area = 0., cx = 0., cy = 0., r2 = 0.;
@@ -298,13 +213,14 @@ __device__ void v2_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, Sim
   }
   const int32_t start = atomicAdd(&S.nf_tmp, cnt);
   if ((int64_t)start + cnt > D.face_cap) {
-    V.femit[cb + s + i] = 0;
+    V.femit[gi] = 0;
     atomicCAS(&B.cnt->err, 0, E_MESH);
     atomicCAS(&S.err, 0, E_MESH);
     return;
   }
   V.vst[gi] = start;
-  V.femit[cb + s + i] = cnt;
+  V.femit[gi] = cnt;
+  if (cnt) atomicAdd(&V.part1[chunk], cnt);
   V2Face* out = V.vf + D.face_base + start;
   int q = 0;
   for (int k = 0; k < m; ++k) {
@@ -616,12 +532,14 @@ __device__ int v2_team_build(const Batch& B, const SimDesc& D, const V2Bufs& V, 
   return 0;
 }
 
-// grid: HFV_V2_SUB blocks per cell chunk, HFV_BLOCK / HFV_V2_TEAM cells per block.  WIDE: only the cells
-// that the first pass marked.
-template <bool WIDE>
+// grid: HFV_V2_SUB blocks per cell chunk, HFV_BLOCK / HFV_V2_TEAM cells per block.  A cell whose candidates
+// or edges outgrow the registers and the small polygon is built again by the same team in the wide one.
 __global__ void __launch_bounds__(HFV_BLOCK) k_v2_cells(Batch B, V2Bufs V) {
-  constexpr int TL = WIDE ? HFV_V2_TLW : HFV_V2_TL;
-  __shared__ V2TeamPoly<TL> polys[HFV_BLOCK / HFV_V2_TEAM];
+  union Poly {
+    V2TeamPoly<HFV_V2_TL> a;
+    V2TeamPoly<HFV_V2_TLW> b;
+  };
+  __shared__ Poly polys[HFV_BLOCK / HFV_V2_TEAM];
   const BlockJob J = B.cjobs[blockIdx.x / HFV_V2_SUB];
   if (J.sim < 0) return;
   const int s = J.sim;
@@ -634,134 +552,164 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_cells(Batch B, V2Bufs V) {
   if (gi >= J.hi) return;  // whole teams; no block barrier follows
   const int64_t N = B.C.n, cb = D.cell_base;
   const int32_t i = (int32_t)(gi - cb);
-  if (!B.C.act[gi]) return;  // unbuilt in a partial build (femit stays 0)
-  if (WIDE && V.femit[cb + s + i] != HFV_V2_WIDE) return;
+  if (lane == 0) V.ccnt[gi] = 0;
+  if (!B.C.act[gi]) {  // unbuilt in a partial build
+    if (lane == 0) V.femit[gi] = 0;
+    return;
+  }
   const double xi = B.C.loc[gi], yi = B.C.loc[N + gi], zi = B.C.loc[2 * N + gi];
-  V2TeamPoly<TL>& P = polys[team];
+  Poly& P = polys[team];
   int m = 0, r = 1;
   double r2 = 0.;
   const int kmax = max(6, max(D.vnb[0], D.vnb[1]));
   for (int K = 2; K <= kmax && r == 1; ++K)
-    r = v2_team_build<!WIDE, TL>(B, D, V, s, i, xi, yi, zi, K, P, m, r2, lane, tiw);
+    r = v2_team_build<true, HFV_V2_TL>(B, D, V, s, i, xi, yi, zi, K, P.a, m, r2, lane, tiw);
+  const bool wide = r == 2;
+  if (wide) {
+    r = 1;
+    for (int K = 2; K <= kmax && r == 1; ++K)
+      r = v2_team_build<false, HFV_V2_TLW>(B, D, V, s, i, xi, yi, zi, K, P.b, m, r2, lane, tiw);
+  }
   if (lane != 0) return;
-  if (r == 2 && !WIDE) {
-    V.femit[cb + s + i] = HFV_V2_WIDE;
-  } else if (r != 0) {
-    V.femit[cb + s + i] = 0;
+  if (r != 0) {
+    V.femit[gi] = 0;
     atomicCAS(&B.cnt->err, 0, E_MESH);
     atomicCAS(&S.err, 0, E_MESH);
+  } else if (wide) {
+    v2_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, P.b, m);
   } else {
-    v2_finish(B, V, D, S, s, gi, i, xi, yi, zi, P, m);
+    v2_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, P.a, m);
   }
 }
 
 // ---------------------------------------------------------------- faces and CSR
+// The faces of a chunk's cells, in cell order after the faces of the chunks before: face arrays, and the
+// entries of both cells into their buckets.  The block's threads take its faces in turn, whichever cell
+// emitted them (a binary search of the cells' offsets in LDS).
 __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
-  const BlockJob J = B.fjobs[blockIdx.x];
-  if (J.sim < 0) return;
-  const int s = J.sim;
-  const SimDesc& D = B.sims[s];
-  const SimStep& S = B.st[s];
-  if (!D.vmesh || !S.stepping) return;
-  const int64_t f = (int64_t)J.lo + threadIdx.x;
-  if (f >= J.hi) return;
-  Faces& F = B.F;
-  const int64_t fl = f - D.face_base, cb = D.cell_base, NF = F.nf, N = B.C.n;
-  if (fl >= B.eng[s].nf_mesh) {
-    F.left[f] = -1;
-    F.right[f] = -1;
-    return;
-  }
-  const int32_t* off = V.femit + cb + s;
-  int64_t lo = 0, hi = D.n;  // off[lo] <= fl < off[hi]
-  while (hi - lo > 1) {
-    const int64_t mid = (lo + hi) >> 1;
-    if (off[mid] <= fl) lo = mid;
-    else hi = mid;
-  }
-  const int64_t gi = cb + lo;
-  const V2Face r = V.vf[D.face_base + V.vst[gi] + (fl - off[lo])];
-  F.area[f] = r.area;
-  F.nrm[f] = r.nx;
-  F.nrm[NF + f] = r.ny;
-  F.nrm[2 * NF + f] = D.vmesh == 3 ? r.nz : 0.;
-  F.fcen[f] = B.C.loc[gi] + r.cx;
-  F.fcen[NF + f] = B.C.loc[N + gi] + r.cy;
-  F.fcen[2 * NF + f] = D.vmesh == 3 ? B.C.loc[2 * N + gi] + r.cz : B.C.loc[2 * N + gi];
-  F.left[f] = (int32_t)gi;
-  F.right[f] = r.nb < 0 ? -1 : (int32_t)(cb + r.nb);
-  F.shc[f] = (uint8_t)r.code;
-  atomicAdd(&V.ccnt[cb + s + lo], 1);
-  if (r.nb >= 0) atomicAdd(&V.ccnt[cb + s + r.nb], 1);
-}
-
-__global__ void __launch_bounds__(HFV_BLOCK) k_v2_csr_fill(Batch B, V2Bufs V) {
-  const BlockJob J = B.fjobs[blockIdx.x];
-  if (J.sim < 0) return;
-  const int s = J.sim;
-  const SimDesc& D = B.sims[s];
-  const SimStep& S = B.st[s];
-  if (!D.vmesh || !S.stepping || S.err) return;
-  const int64_t f = (int64_t)J.lo + threadIdx.x;
-  if (f >= J.hi || f - D.face_base >= B.eng[s].nf_mesh) return;
-  const int32_t l = B.F.left[f], r = B.F.right[f];
-  int32_t p = atomicAdd(&V.cfill[l], 1);
-  B.F.conn[p] = (int32_t)(f << 1);
-  B.F.nbr[p] = r;
-  if (r >= 0) {
-    p = atomicAdd(&V.cfill[r], 1);
-    B.F.conn[p] = (int32_t)((f << 1) | 1);
-    B.F.nbr[p] = l;
-  }
-}
-
-#define HFV_CSR_SORT_LDS 24  // a cell's CSR entries sorted in LDS (more: in place in memory)
-
-__global__ void __launch_bounds__(HFV_BLOCK) k_v2_csr_sort(Batch B, V2Bufs V) {
-  __shared__ uint64_t ent[HFV_CSR_SORT_LDS][HFV_BLOCK];  // [slot][thread]: (CSR value << 32) | neighbour
+  __shared__ int32_t offs[HFV_BLOCK], starts[HFV_BLOCK];
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
   SimStep& S = B.st[s];
-  if (!D.vmesh || !S.stepping || S.err) return;
-  const int64_t gi = (int64_t)J.lo + threadIdx.x;
-  if (gi >= J.hi) return;  // (no block barrier follows)
-  const int32_t e0 = B.F.off[gi], e1 = B.F.off[gi + 1];
+  if (!D.vmesh || !S.stepping) return;
+  const int64_t cb = D.cell_base, NF = B.F.nf, N = B.C.n;
+  const int64_t gi0 = (int64_t)J.lo + threadIdx.x;
+  const bool in = gi0 < J.hi;
+  int32_t all, tot;
+  const int32_t base = chunks_before(V.part1, D, J.chunk, &all);
+  offs[threadIdx.x] = block_excl_scan(in ? V.femit[gi0] : 0, &tot);
+  starts[threadIdx.x] = in ? V.vst[gi0] : 0;
+  const bool bad = S.err != 0;  // a failed cell emitted nothing: the simulation stops
+  if (J.chunk == D.cchunk0 && threadIdx.x == 0) B.eng[s].nf_mesh = bad ? 0 : all;
+  __syncthreads();
+  if (bad) return;
+  const Faces& F = B.F;
+  for (int32_t t = threadIdx.x; t < tot; t += HFV_BLOCK) {
+    int lo = 0;  // the last cell whose offset is <= t (later cells of the same offset emit nothing)
+#pragma unroll
+    for (int h = HFV_BLOCK / 2; h > 0; h >>= 1)
+      if (offs[lo + h] <= t) lo += h;
+    const int64_t gi = (int64_t)J.lo + lo;
+    const int64_t f = D.face_base + base + t;
+    const V2Face r = V.vf[D.face_base + starts[lo] + (t - offs[lo])];
+    F.area[f] = r.area;
+    F.nrm[f] = r.nx;
+    F.nrm[NF + f] = r.ny;
+    F.nrm[2 * NF + f] = D.vmesh == 3 ? r.nz : 0.;
+    F.fcen[f] = B.C.loc[gi] + r.cx;
+    F.fcen[NF + f] = B.C.loc[N + gi] + r.cy;
+    F.fcen[2 * NF + f] = D.vmesh == 3 ? B.C.loc[2 * N + gi] + r.cz : B.C.loc[2 * N + gi];
+    const int32_t right = r.nb < 0 ? -1 : (int32_t)(cb + r.nb);
+    F.left[f] = (int32_t)gi;
+    F.right[f] = right;
+    F.shc[f] = (uint8_t)r.code;
+    auto put = [&](int32_t cell, int32_t conn, int32_t nbr) {
+      const int32_t q = atomicAdd(&V.ccnt[cell], 1);
+      if (q < HFV_BUCKET) {
+        V.bkt[(int64_t)q * N + cell] = ((uint64_t)(uint32_t)conn << 32) | (uint32_t)nbr;
+        return;
+      }
+      const int32_t o = atomicAdd(&S.n_over, 1);
+      if (o < D.conn_cap) V.over[D.conn_base + o] = V2Over{cell, conn, nbr};  // (more: refused by k_v2_conn)
+    };
+    put((int32_t)gi, (int32_t)(f << 1), right);
+    if (right >= 0) put(right, (int32_t)((f << 1) | 1), (int32_t)gi);
+  }
+}
+
+// CSR offsets, and every cell's entries in ascending face order (then side): CSR values are distinct and
+// non-negative, so the packed words order as they do.  The bin counts restart at zero.
+__global__ void __launch_bounds__(HFV_BLOCK) k_v2_conn(Batch B, V2Bufs V) {
+  __shared__ uint64_t ent[HFV_BUCKET][HFV_BLOCK];  // [slot][thread]
+  const BlockJob J = B.cjobs[blockIdx.x];
+  if (J.sim < 0) return;
+  const int s = J.sim;
+  const SimDesc& D = B.sims[s];
+  SimStep& S = B.st[s];
+  if (!D.vmesh || !S.stepping) return;
+  const int64_t gi = (int64_t)J.lo + threadIdx.x, N = B.C.n;
+  const bool in = gi < J.hi;
+  const int64_t bin = gi - D.cell_base;
+  if (bin < (int64_t)D.vnb[0] * D.vnb[1] * D.vnb[2]) V.gcnt[D.cell_base + s + bin] = 0;
+  const int m = in ? V.ccnt[gi] : 0;
+  int32_t all, tot;
+  const int32_t base = chunks_before(V.part2, D, J.chunk, &all);
+  const int32_t x = base + block_excl_scan(m, &tot);
+  const bool full = all > D.conn_cap;
+  const bool bad = full || S.err != 0;
+  if (full && J.chunk == D.cchunk0 && threadIdx.x == 0) {
+    atomicCAS(&B.cnt->err, 0, E_MESH);
+    atomicCAS(&S.err, 0, E_MESH);
+  }
+  const int32_t e0 = (int32_t)D.conn_base + (bad ? 0 : x);
+  if (in) B.F.off[gi] = e0;
+  if (J.chunk == D.cchunk1 - 1) {  // offsets past the last cell: the slot's end of the CSR
+    const int32_t end = (int32_t)D.conn_base + (bad ? 0 : all);
+    for (int64_t k = D.n + threadIdx.x; k < D.noff; k += HFV_BLOCK) B.F.off[D.cell_base + k] = end;
+  }
+  if (bad || !in) return;  // (no block barrier follows)
   int32_t* c = B.F.conn;
   int32_t* nb = B.F.nbr;
-  const int m = e1 - e0;
-  if (m <= HFV_CSR_SORT_LDS) {
-    // insertion sort of the cell's entries by face index (then side): CSR values are distinct and
-    // non-negative, so the packed words order as they do
+  if (m <= HFV_BUCKET) {
     uint64_t* v = &ent[0][threadIdx.x];
-    for (int k = 0; k < m; ++k) v[k * HFV_BLOCK] = ((uint64_t)(uint32_t)c[e0 + k] << 32) | (uint32_t)nb[e0 + k];
+    for (int k = 0; k < m; ++k) v[k * HFV_BLOCK] = V.bkt[(int64_t)k * N + gi];
     for (int k = 1; k < m; ++k) {
-      const uint64_t x = v[k * HFV_BLOCK];
+      const uint64_t w = v[k * HFV_BLOCK];
       int j = k - 1;
-      while (j >= 0 && v[j * HFV_BLOCK] > x) {
+      while (j >= 0 && v[j * HFV_BLOCK] > w) {
         v[(j + 1) * HFV_BLOCK] = v[j * HFV_BLOCK];
         --j;
       }
-      v[(j + 1) * HFV_BLOCK] = x;
+      v[(j + 1) * HFV_BLOCK] = w;
     }
     for (int k = 0; k < m; ++k) {
-      const uint64_t x = v[k * HFV_BLOCK];
-      c[e0 + k] = (int32_t)(x >> 32);
-      nb[e0 + k] = (int32_t)(uint32_t)x;
+      const uint64_t w = v[k * HFV_BLOCK];
+      c[e0 + k] = (int32_t)(w >> 32);
+      nb[e0 + k] = (int32_t)(uint32_t)w;
     }
     return;
   }
-  for (int32_t k = e0 + 1; k < e1; ++k) {  // insertion sort in place
-    const int32_t x = c[k], y = nb[k];
-    int32_t j = k - 1;
-    while (j >= e0 && c[j] > x) {
+  // more than the bucket holds: its entries and the list's, sorted in place in memory
+  auto insert = [&](int32_t at, int32_t conn, int32_t nbr) {
+    int32_t j = e0 + at - 1;
+    while (j >= e0 && c[j] > conn) {
       c[j + 1] = c[j];
       nb[j + 1] = nb[j];
       --j;
     }
-    c[j + 1] = x;
-    nb[j + 1] = y;
+    c[j + 1] = conn;
+    nb[j + 1] = nbr;
+  };
+  int32_t at = 0;
+  for (; at < HFV_BUCKET; ++at) {
+    const uint64_t w = V.bkt[(int64_t)at * N + gi];
+    insert(at, (int32_t)(w >> 32), (int32_t)(uint32_t)w);
+  }
+  for (int32_t o = 0; o < S.n_over && at < m; ++o) {
+    const V2Over w = V.over[D.conn_base + o];
+    if (w.cell == (int32_t)gi) insert(at++, w.conn, w.nbr);
   }
 }
 

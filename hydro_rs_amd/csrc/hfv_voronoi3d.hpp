@@ -667,7 +667,7 @@ __device__ int v3_build(const Batch& B, const SimDesc& D, const V2Bufs& V, int s
 // Cell3::finish on the clipped cell.  Returns 0, 1 (a periodic cell touching the initial region: retry
 // with a larger K) or 3 (a face of more than HFV_V3_FAN vertices); on 0 the faces and the geometry are
 // written.
-__device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int s, int64_t gi, int32_t i,
+__device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int chunk, int64_t gi, int32_t i,
                          double xi, double yi, double zi, V3Cell& C, int np, int nt, double r2) {
   const int lane = __lane_id();
   const int p = lane;
@@ -787,7 +787,7 @@ __device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimS
   start = __shfl(start, 0, 64);
   if ((int64_t)start + cnt > D.face_cap) {
     if (lane == 0) {
-      V.femit[cb + s + i] = 0;
+      V.femit[gi] = 0;
       atomicCAS(&B.cnt->err, 0, E_MESH);
       atomicCAS(&S.err, 0, E_MESH);
     }
@@ -810,7 +810,8 @@ __device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimS
   wave_sync();
   if (lane != 0) return 0;
   V.vst[gi] = start;
-  V.femit[cb + s + i] = cnt;
+  V.femit[gi] = cnt;
+  if (cnt) atomicAdd(&V.part1[chunk], cnt);
   // the cell's volume and centroid: the tetrahedron terms added in the host's order
   double vol = 0., cenx = 0., ceny = 0., cenz = 0.;
   for (int q = 0; q < ntri; ++q) {
@@ -841,7 +842,11 @@ __global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V) {
   if (D.vmesh != 3 || !S.stepping) return;
   const int64_t gi = (int64_t)J.lo + blockIdx.x % HFV_BLOCK;
   if (gi >= J.hi) return;
-  if (!B.C.act[gi]) return;  // unbuilt in a partial build (femit stays 0)
+  if (__lane_id() == 0) V.ccnt[gi] = 0;
+  if (!B.C.act[gi]) {  // unbuilt in a partial build
+    if (__lane_id() == 0) V.femit[gi] = 0;
+    return;
+  }
   const int64_t N = B.C.n, cb = D.cell_base;
   const int32_t i = (int32_t)(gi - cb);
   const double xi = B.C.loc[gi], yi = B.C.loc[N + gi], zi = B.C.loc[2 * N + gi];
@@ -850,10 +855,10 @@ __global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V) {
   double r2 = 0.;
   for (int K = 2; K <= kmax && r == 1; ++K) {
     r = v3_build(B, D, V, s, i, xi, yi, zi, K, C, np, nt, r2);
-    if (r == 0) r = v3_finish(B, V, D, S, s, gi, i, xi, yi, zi, C, np, nt, r2);
+    if (r == 0) r = v3_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, C, np, nt, r2);
   }
   if (r != 0 && __lane_id() == 0) {
-    V.femit[cb + s + i] = 0;
+    V.femit[gi] = 0;
     atomicCAS(&B.cnt->err, 0, E_MESH);
     atomicCAS(&S.err, 0, E_MESH);
   }
