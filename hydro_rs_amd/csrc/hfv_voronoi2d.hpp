@@ -155,27 +155,21 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_place(Batch B, V2Bufs V) {
 }
 
 // ---------------------------------------------------------------- cells, a team of lanes per cell
-// HFV_V2_TEAM lanes of one wavefront build one cell together.  The polygon lives in LDS, each lane
-// testing, moving and intersecting every TEAM-th edge; the next candidate in (squared distance, index,
-// image code) order is a team minimum over the lanes' smallest keys above the last one, each lane taking
-// every TEAM-th bin of the (2K+1)^2 block.  k_v2_cells keeps each lane's candidates in registers (at most
-// HFV_V2_TC) and polygons of up to HFV_V2_TL edges; cells that outgrow either are built again, rescanning
-// the bins for every candidate, with polygons of up to HFV_V2_TLW edges.  Both make the host tessellator's
+// 16 lanes, a DPP row, build one cell together.  The candidates of the (2K+1)^2 block are gathered into LDS
+// once, ranked by (squared distance, index, image code) (each lane ranks every 16th against all), and clip
+// the polygon in rank order.  The polygon lies in registers, lane k holding edge k and the vertex after it: a
+// clip is one ballot, and where it cuts, one permute that closes the edges up, one for the next edge's plane,
+// the lanes' vertices and a row maximum.  The finish takes each edge's terms on its own lane and adds them in
+// order.  (A team's chain of candidates is what bounds the rebuild, most of all where few cells are
+// active: with the next candidate a 4-stage team minimum over whole candidates and the polygon in LDS the
+// kernel took 65 us on Sedov 256^2 with steered generators and 98 us on a 125^2 vortex, now 35 and 71.)
+// Cells of more than HFV_V2_CAP candidates or 16 edges are built by v2_team_build, which rescans the bins for
+// every candidate and keeps polygons of up to HFV_V2_TLW edges in LDS.  Both make the host tessellator's
 // operations in its order, so the same bits.
-// 16 lanes per cell: 205 us per step on Sedov 256^2 with steered generators, against 325 with 8 and 217
-// with 32 (the rebuild is latency-bound: few active cells per step, each team's chain of clips)
-#ifndef HFV_V2_TEAM
 #define HFV_V2_TEAM 16
-#endif
-#ifndef HFV_V2_TL
-#define HFV_V2_TL 32
-#endif
-#ifndef HFV_V2_TLW
 #define HFV_V2_TLW 48
-#endif
-#ifndef HFV_V2_TC
-#define HFV_V2_TC 8
-#endif
+#define HFV_V2_CAP 96           // 3 blocks a CU; a 9 x 9-bin block (K = 4) at one generator per bin mostly fits
+#define HFV_V2_OWN (HFV_V2_CAP / HFV_V2_TEAM)
 #define HFV_V2_SUB HFV_V2_TEAM  // blocks per cell chunk
 
 template <int TL>
@@ -449,9 +443,9 @@ __device__ __forceinline__ void team_min(bool& have, V2Cand& b) {
   }
 }
 
-// The cell of generator i with candidate bins within K: 0 built, 1 retry with a larger K, 2 too many
-// candidates or edges for this variant (LIST: candidates kept in registers; otherwise rescanned).
-template <bool LIST, int TL>
+// The cell of generator i with candidate bins within K, any number of candidates: 0 built, 1 retry with a
+// larger K, 2 more than TL edges.
+template <int TL>
 __device__ int v2_team_build(const Batch& B, const SimDesc& D, const V2Bufs& V, int s, int32_t i, double xi,
                              double yi, double zi, int K, V2TeamPoly<TL>& P, int& m, double& r2, int lane, int tiw) {
   const double w0 = D.vw[0], w1 = D.vw[1];
@@ -473,17 +467,6 @@ __device__ int v2_team_build(const Batch& B, const SimDesc& D, const V2Bufs& V, 
   m = 4;
   team_recompute(P, m, lane);
   r2 = team_rmax2(P, m, lane);
-  V2Cand cl[LIST ? HFV_V2_TC : 1];
-  int cnt = 0;
-  if (LIST) {
-    v2_lane_candidates(B, D, V, s, i, xi, yi, zi, K, lane, [&](const V2Cand& c) {
-#pragma unroll
-      for (int q = 0; q < (LIST ? HFV_V2_TC : 1); ++q)
-        if (q == cnt) cl[q] = c;
-      ++cnt;
-    });
-    if (team_ballot(cnt > HFV_V2_TC, tiw)) return 2;
-  }
   bool have_last = false;
   V2Cand last{};
   while (true) {
@@ -496,13 +479,7 @@ __device__ int v2_team_build(const Batch& B, const SimDesc& D, const V2Bufs& V, 
         best = c;
       }
     };
-    if (LIST) {
-#pragma unroll
-      for (int q = 0; q < (LIST ? HFV_V2_TC : 1); ++q)
-        if (q < cnt) consider(cl[q]);
-    } else {
-      v2_lane_candidates(B, D, V, s, i, xi, yi, zi, K, lane, consider);
-    }
+    v2_lane_candidates(B, D, V, s, i, xi, yi, zi, K, lane, consider);
     team_min(have, best);
     if (!have || 0.25 * best.d2 > r2) break;  // security radius: the bisector lies beyond every vertex
     const int c = team_clip(P, m, best.rx, best.ry, 0.5 * best.d2, best.j, best.code, lane, tiw);
@@ -532,14 +509,297 @@ __device__ int v2_team_build(const Batch& B, const SimDesc& D, const V2Bufs& V, 
   return 0;
 }
 
-// grid: HFV_V2_SUB blocks per cell chunk, HFV_BLOCK / HFV_V2_TEAM cells per block.  A cell whose candidates
-// or edges outgrow the registers and the small polygon is built again by the same team in the wide one.
+struct V2TeamCands {
+  double d2[HFV_V2_CAP], rx[HFV_V2_CAP], ry[HFV_V2_CAP];
+  int32_t j[HFV_V2_CAP], k[HFV_V2_CAP];
+  uint8_t ord[HFV_V2_CAP];  // candidate of each rank
+  int32_t n;
+};
+
+// A team's polygon: this lane's edge (plane, neighbour, image code) and the vertex between it and the next.
+struct V2RegPoly {
+  double nx, ny, d, vx, vy;
+  int32_t nb, code;
+};
+
+template <int CTRL>
+__device__ __forceinline__ double row_max_step(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  const double t = __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false),
+                                    __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false));
+  return v < t ? t : v;
+}
+// maximum over the team (a DPP row: row_ror 8, 4, 2, 1), in every lane
+__device__ __forceinline__ double team_max(double v) {
+  static_assert(HFV_V2_TEAM == 16, "a team is a DPP row");
+  v = row_max_step<0x128>(v);
+  v = row_max_step<0x124>(v);
+  v = row_max_step<0x122>(v);
+  return row_max_step<0x121>(v);
+}
+
+// every vertex from its edge and the next one (0 where they are parallel); the largest squared radius
+__device__ __forceinline__ double v2_vertices(V2RegPoly& P, int m, int lane) {
+  const int k1 = lane + 1 == m ? 0 : lane + 1;
+  const double nx1 = __shfl(P.nx, k1, HFV_V2_TEAM), ny1 = __shfl(P.ny, k1, HFV_V2_TEAM), d1 = __shfl(P.d, k1, HFV_V2_TEAM);
+  double r = 0.;
+  if (lane < m) {
+    const double det = P.nx * ny1 - P.ny * nx1;
+    P.vx = 0.;
+    P.vy = 0.;
+    if (det != 0.0) {
+      P.vx = (P.d * ny1 - d1 * P.ny) / det;
+      P.vy = (P.nx * d1 - nx1 * P.d) / det;
+    }
+    const double q = P.vx * P.vx + P.vy * P.vy;
+    r = r < q ? q : r;
+  }
+  return team_max(r);
+}
+
+// The candidates of the (2K+1)^2 block into LDS (any order: the rank orders them), each lane taking every 16th
+// bin, four candidates' loads in flight: their count, or -1 beyond HFV_V2_CAP.
+__device__ __forceinline__ int v2_gather(const Batch& B, const SimDesc& D, const V2Bufs& V, int s, int32_t i, double xi,
+                                         double yi, double zi, int K, V2TeamCands& Q, int lane, int tiw) {
+  const int64_t N = B.C.n, cb = D.cell_base;
+  const double* L = B.C.loc;
+  const double bx = D.cfg.box[0], by = D.cfg.box[1], bz = D.cfg.box[2];
+  const int nb0 = D.vnb[0], nb1 = D.vnb[1];
+  const bool per = D.periodic != 0;
+  const int bi0 = v2_bin(xi, D.vw[0], nb0), bi1 = v2_bin(yi, D.vw[1], nb1);
+  const int32_t* gst = V.gcnt + cb + s;
+  const int32_t* gord = V.gord + cb;
+  const int side = 2 * K + 1;
+  if (lane == 0) Q.n = 0;
+  team_sync();
+  for (int bb = lane; bb < side * side; bb += HFV_V2_TEAM) {
+    int b0 = bi0 + bb / side - K, b1 = bi1 + bb % side - K, s0 = 0, s1 = 0;
+    bool skip = false;
+    if (b0 < 0 || b0 >= nb0) {
+      s0 = b0 < 0 ? -1 : 1;
+      b0 -= s0 * nb0;
+      skip = !per || b0 < 0 || b0 >= nb0;
+    }
+    if (b1 < 0 || b1 >= nb1) {
+      s1 = b1 < 0 ? -1 : 1;
+      b1 -= s1 * nb1;
+      skip = skip || !per || b1 < 0 || b1 >= nb1;
+    }
+    if (skip) continue;
+    const int key = b0 * nb1 + b1;
+    const int32_t kk = ((s0 & 0xFF) << 16) | ((s1 & 0xFF) << 8);  // the host's memcmp order of the int8 codes
+    const int32_t g0 = gst[key], g1 = gst[key + 1];
+    for (int32_t q0 = g0; q0 < g1; q0 += 4) {
+      int32_t jj[4];
+      double x[4], y[4], z[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) jj[u] = q0 + u < g1 ? gord[q0 + u] : -1;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t gj = cb + (jj[u] < 0 ? 0 : jj[u]);
+        x[u] = L[gj];
+        y[u] = L[N + gj];
+        z[u] = L[2 * N + gj];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (jj[u] < 0 || (jj[u] == i && s0 == 0 && s1 == 0)) continue;
+        const double xj = x[u] + (double)s0 * bx, yj = y[u] + (double)s1 * by, zj = z[u] + 0.0 * bz;
+        const double rx = xj - xi, ry = yj - yi, rz = zj - zi;
+        const int at = atomicAdd(&Q.n, 1);
+        if (at >= HFV_V2_CAP) continue;
+        Q.d2[at] = rx * rx + ry * ry + rz * rz;
+        Q.rx[at] = rx;
+        Q.ry[at] = ry;
+        Q.j[at] = jj[u];
+        Q.k[at] = kk;
+      }
+    }
+  }
+  team_sync();
+  const int n = Q.n;
+  return n > HFV_V2_CAP ? -1 : n;
+}
+
+// ord[rank] = candidate, by squared distance (a non-negative double orders as its bits), and by the whole key
+// where two squared distances are equal.
+__device__ __forceinline__ void v2_rank(V2TeamCands& Q, int n, int lane, int tiw) {
+  const int nown = (n + HFV_V2_TEAM - 1) / HFV_V2_TEAM;
+  const uint64_t* D2 = reinterpret_cast<const uint64_t*>(Q.d2);
+  for (int h = 0; h < nown; ++h) {
+    const int a = lane + HFV_V2_TEAM * h;
+    const int aa = a < n ? a : 0;
+    const uint64_t od = D2[aa];
+    int rk = 0, le = 0;
+    for (int b = 0; b < n; b += 8) {
+      uint64_t db[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) db[u] = b + u < n ? D2[b + u] : ~0ull;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        rk += db[u] < od ? 1 : 0;
+        le += db[u] <= od ? 1 : 0;
+      }
+    }
+    if (a < n && le - rk > 1) {  // (rare)
+      const int32_t oj = Q.j[a], ok = Q.k[a];
+      for (int b = 0; b < n; ++b)
+        rk += D2[b] == od && (Q.j[b] < oj || (Q.j[b] == oj && Q.k[b] < ok)) ? 1 : 0;
+    }
+    if (a < n) Q.ord[rk] = (uint8_t)a;
+  }
+  team_sync();
+}
+
+// The cell of generator i with candidate bins within K: 0 built, 1 retry with a larger K, 2 too many
+// candidates or edges.
+__device__ __forceinline__ int v2_reg_build(const Batch& B, const SimDesc& D, const V2Bufs& V, int s, int32_t i,
+                                            double xi, double yi, double zi, int K, V2TeamCands& Q, V2RegPoly& P, int& m,
+                                            double& r2, int lane, int tiw) {
+  const double w0 = D.vw[0], w1 = D.vw[1];
+  const bool per = D.periodic != 0;
+  // initial region: the box, or K bin widths around the generator on a periodic box
+  double reach = 0.;
+  reach = reach < K * w0 ? K * w0 : reach;
+  reach = reach < K * w1 ? K * w1 : reach;
+  const double lox = per ? -reach : -xi, loy = per ? -reach : -yi;
+  const double hix = per ? reach : D.cfg.box[0] - xi, hiy = per ? reach : D.cfg.box[1] - yi;
+  // counter-clockwise: bottom, right, top, left (walls -3, -2, -4, -1)
+  P.nx = lane == 1 ? 1. : lane == 3 ? -1. : 0.;
+  P.ny = lane == 0 ? -1. : lane == 2 ? 1. : 0.;
+  P.d = lane == 0 ? -loy : lane == 1 ? hix : lane == 2 ? hiy : -lox;
+  P.nb = lane == 0 ? -3 : lane == 1 ? -2 : lane == 2 ? -4 : -1;
+  P.code = 0;
+  P.vx = 0.;
+  P.vy = 0.;
+  m = 4;
+  r2 = v2_vertices(P, m, lane);
+  const int n = v2_gather(B, D, V, s, i, xi, yi, zi, K, Q, lane, tiw);
+  if (n < 0) return 2;
+  v2_rank(Q, n, lane, tiw);
+  int a = n > 0 ? Q.ord[0] : 0;
+  double cd2 = Q.d2[a], cx = Q.rx[a], cy = Q.ry[a];
+  for (int q = 0; q < n; ++q) {
+    if (0.25 * cd2 > r2) break;  // security radius: the bisector lies beyond every vertex
+    const int now = a;
+    const double ca = cx, cbb = cy, dd = 0.5 * cd2;
+    a = Q.ord[q + 1 < n ? q + 1 : q];  // the next candidate, in flight during the clip
+    cd2 = Q.d2[a];
+    cx = Q.rx[a];
+    cy = Q.ry[a];
+    // clip by the half-plane (ca, cbb).y <= dd: the run of outside vertices start .. start+nout-1 is contiguous;
+    // edges start+1 .. start+nout-1 go, the new edge follows edge start, and the list restarts at the first
+    // kept edge after the removed run
+    const bool out = lane < m && (ca * P.vx + cbb * P.vy) > dd + HFV_CLIP_TOL * dd;
+    const uint32_t om = team_ballot(out, tiw);
+    const int nout = __popc(om);
+    if (nout == 0 || nout == m) continue;
+    const int mq = m - nout + 2;
+    if (mq > HFV_V2_TEAM) return 2;
+    const uint32_t full = (1u << m) - 1u;
+    const uint32_t prev = ((om << 1) | (om >> (m - 1))) & full;  // bit k: vertex k-1 is outside
+    const uint32_t sm = om & ~prev;
+    const int start = sm ? __builtin_ctz(sm) : 0;
+    int src = start + nout;
+    src = src >= m ? src - m : src;
+    src += lane;
+    src = src >= m ? src - m : src;  // (lanes past the kept edges read any lane)
+    const double ex = __shfl(P.nx, src, HFV_V2_TEAM), ey = __shfl(P.ny, src, HFV_V2_TEAM), ed = __shfl(P.d, src, HFV_V2_TEAM);
+    const int32_t en = __shfl(P.nb, src, HFV_V2_TEAM), ec = __shfl(P.code, src, HFV_V2_TEAM);
+    const bool fresh = lane == mq - 1;
+    const int32_t ck = Q.k[now];
+    P.nx = fresh ? ca : ex;
+    P.ny = fresh ? cbb : ey;
+    P.d = fresh ? dd : ed;
+    P.nb = fresh ? Q.j[now] : en;
+    P.code = fresh ? v2_shift_code((int8_t)((ck >> 16) & 0xFF), (int8_t)((ck >> 8) & 0xFF)) : ec;
+    m = mq;
+    r2 = v2_vertices(P, m, lane);
+  }
+  // completeness: every unvisited generator lies farther than K bin widths
+  double minw = 1e300;
+  minw = K * w0 < minw ? K * w0 : minw;
+  minw = K * w1 < minw ? K * w1 : minw;
+  if (4.0 * r2 > minw * minw) return 1;
+  if (per) {  // a periodic cell must not touch the initial region
+    const int km = lane == 0 ? m - 1 : lane - 1;
+    const double ex = P.vx - __shfl(P.vx, km, HFV_V2_TEAM), ey = P.vy - __shfl(P.vy, km, HFV_V2_TEAM);
+    if (team_ballot(lane < m && P.nb < 0 && sqrt(ex * ex + ey * ey) > 0., tiw)) return 1;
+  }
+  return 0;
+}
+
+// v2_finish of a team's register polygon, each edge on its lane; the sums are added in edge order.
+__device__ __forceinline__ void v2_reg_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int chunk,
+                                              int64_t gi, int32_t i, double xi, double yi, double zi, const V2RegPoly& P,
+                                              int m, int lane, int tiw) {
+  const int64_t N = B.C.n, cb = D.cell_base;
+  const int km = lane == 0 ? m - 1 : lane - 1;
+  const double ax = __shfl(P.vx, km, HFV_V2_TEAM), ay = __shfl(P.vy, km, HFV_V2_TEAM), bxx = P.vx, byy = P.vy;
+  const double cr = ax * byy - bxx * ay;
+  const double ta = 0.5 * cr, tx = (cr / 6.0) * (ax + bxx), ty = (cr / 6.0) * (ay + byy);
+  const double len = sqrt((bxx - ax) * (bxx - ax) + (byy - ay) * (byy - ay));
+  const bool emit = lane < m && len > 0. && v2_emits(B, cb, P.nb, i);
+  double q = 0.;
+  if (lane < m) {
+    const double qq = bxx * bxx + byy * byy;
+    q = q < qq ? qq : q;
+  }
+  const double r2 = team_max(q);
+  double area = 0., cx = 0., cy = 0.;
+  for (int k = 0; k < m; ++k) {
+    area += __shfl(ta, k, HFV_V2_TEAM);
+    cx = cx + __shfl(tx, k, HFV_V2_TEAM);
+    cy = cy + __shfl(ty, k, HFV_V2_TEAM);
+  }
+  const uint32_t em = team_ballot(emit, tiw);
+  const int cnt = __popc(em);
+  int32_t start = 0;
+  if (lane == 0) start = atomicAdd(&S.nf_tmp, cnt);
+  start = __shfl(start, 0, HFV_V2_TEAM);
+  if ((int64_t)start + cnt > D.face_cap) {
+    if (lane == 0) {
+      V.femit[gi] = 0;
+      atomicCAS(&B.cnt->err, 0, E_MESH);
+      atomicCAS(&S.err, 0, E_MESH);
+    }
+    return;
+  }
+  if (emit) {
+    const double inv = 1.0 / sqrt(P.nx * P.nx + P.ny * P.ny);
+    V2Face f;
+    f.area = len;
+    f.cx = 0.5 * (ax + bxx);
+    f.cy = 0.5 * (ay + byy);
+    f.cz = 0.;
+    f.nx = inv * P.nx;
+    f.ny = inv * P.ny;
+    f.nz = 0.;
+    f.nb = P.nb < 0 ? -1 : P.nb;
+    f.code = P.code;
+    V.vf[D.face_base + start + __popc(em & ((1u << lane) - 1u))] = f;
+  }
+  if (lane != 0) return;
+  V.vst[gi] = start;
+  V.femit[gi] = cnt;
+  if (cnt) atomicAdd(&V.part1[chunk], cnt);
+  if (B.C.act[gi]) {
+    B.C.vol[gi] = area;
+    const double ia = area > 0. ? 1.0 / area : 0.;
+    B.C.cen[gi] = xi + (area > 0. ? ia * cx : 0.);
+    B.C.cen[N + gi] = yi + (area > 0. ? ia * cy : 0.);
+    B.C.cen[2 * N + gi] = zi;
+    B.C.srad[gi] = 1.5 * 2.0 * sqrt(r2);
+  }
+}
+
+// grid: HFV_V2_SUB blocks per cell chunk, HFV_BLOCK / HFV_V2_TEAM cells per block.
 __global__ void __launch_bounds__(HFV_BLOCK) k_v2_cells(Batch B, V2Bufs V) {
-  union Poly {
-    V2TeamPoly<HFV_V2_TL> a;
-    V2TeamPoly<HFV_V2_TLW> b;
+  union Team {
+    V2TeamCands q;
+    V2TeamPoly<HFV_V2_TLW> wide;
   };
-  __shared__ Poly polys[HFV_BLOCK / HFV_V2_TEAM];
+  __shared__ Team teams[HFV_BLOCK / HFV_V2_TEAM];
   const BlockJob J = B.cjobs[blockIdx.x / HFV_V2_SUB];
   if (J.sim < 0) return;
   const int s = J.sim;
@@ -558,27 +818,31 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_cells(Batch B, V2Bufs V) {
     return;
   }
   const double xi = B.C.loc[gi], yi = B.C.loc[N + gi], zi = B.C.loc[2 * N + gi];
-  Poly& P = polys[team];
+  Team& T = teams[team];
   int m = 0, r = 1;
   double r2 = 0.;
   const int kmax = max(6, max(D.vnb[0], D.vnb[1]));
-  for (int K = 2; K <= kmax && r == 1; ++K)
-    r = v2_team_build<true, HFV_V2_TL>(B, D, V, s, i, xi, yi, zi, K, P.a, m, r2, lane, tiw);
-  const bool wide = r == 2;
-  if (wide) {
+  {
+    V2RegPoly P;
+    for (int K = 2; K <= kmax && r == 1; ++K)
+      r = v2_reg_build(B, D, V, s, i, xi, yi, zi, K, T.q, P, m, r2, lane, tiw);
+    if (r == 0) {
+      v2_reg_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, P, m, lane, tiw);
+      return;
+    }
+  }
+  if (r == 2) {
     r = 1;
     for (int K = 2; K <= kmax && r == 1; ++K)
-      r = v2_team_build<false, HFV_V2_TLW>(B, D, V, s, i, xi, yi, zi, K, P.b, m, r2, lane, tiw);
+      r = v2_team_build<HFV_V2_TLW>(B, D, V, s, i, xi, yi, zi, K, T.wide, m, r2, lane, tiw);
   }
   if (lane != 0) return;
   if (r != 0) {
     V.femit[gi] = 0;
     atomicCAS(&B.cnt->err, 0, E_MESH);
     atomicCAS(&S.err, 0, E_MESH);
-  } else if (wide) {
-    v2_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, P.b, m);
   } else {
-    v2_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, P.a, m);
+    v2_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, T.wide, m);
   }
 }
 
