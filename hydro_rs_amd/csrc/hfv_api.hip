@@ -301,7 +301,7 @@ int ensure_v2(hfv_ctx* c) {
   v.gord = dalloc<int32_t>(c, c->n);
   v.gkey = dalloc<int32_t>(c, c->n);
   v.vst = dalloc<int32_t>(c, c->n);
-  v.vf = dalloc<V2Face>(c, c->nf);
+  v.vf = dalloc<V2Face>(c, 2 * c->nf);
   v.bkt = dalloc<uint64_t>(c, HFV_BUCKET * c->n);
   v.over = dalloc<V2Over>(c, c->nconn);
   v.part0 = dalloc<int32_t>(c, c->ncchunk);

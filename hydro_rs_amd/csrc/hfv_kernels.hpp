@@ -187,7 +187,7 @@ struct SimStep {
   int err;       // the first hard error that a kernel of this step raised (merged into the engine's at the end)
   int min_bin;   // sync_all: the smallest new bin
   int n_down;    // 1D periodic moving meshes: faces of this step's rebuild where the generator order steps down
-  int nf_tmp;    // 2D/3D moving meshes: the rebuild's provisional face cursor
+  int nf_tmp;    // 2D/3D moving meshes: the rebuild's provisional faces beyond their chunks' shares
   int n_over;    // 2D/3D moving meshes: CSR entries beyond their cells' buckets in this step's rebuild
 };
 
@@ -946,11 +946,11 @@ struct V2Bufs {
   int32_t* femit;  // [N] faces a cell emits
   int32_t* vst;    // [N] start of a cell's faces in vf
   int32_t* ccnt;   // [N] CSR entries per cell
-  V2Face* vf;      // [F] at face_base: faces in provisional order
+  V2Face* vf;      // [2 F] faces in provisional order: shares of the chunks at face_base, the rest at F + face_base
   uint64_t* bkt;   // [HFV_BUCKET][N] entries of a cell: (CSR value << 32) | neighbour
   V2Over* over;    // [CSR capacity] at conn_base: entries beyond their cells' buckets
   int32_t* part0;  // [cell chunks] sums of gcnt over the chunk's bins
-  int32_t* part1;  // [cell chunks] sums of femit over the chunk's cells
+  int32_t* part1;  // [cell chunks] sums of femit over the chunk's cells (their cursors while they are built)
   int32_t* part2;  // [cell chunks] sums of ccnt
 };
 

@@ -184,6 +184,19 @@ __device__ __forceinline__ bool v2_emits(const Batch& B, int64_t cb, int32_t nb,
   return nb < 0 || nb > i || !B.C.act[cb + nb];
 }
 
+// Place of a cell's cnt emitted faces in the provisional order (an index into vf): after those that its chunk
+// has placed, in the chunk's share of the simulation's face capacity, or in the common second half where the
+// chunk's share is full.  -1 beyond the capacity.  (One cursor for the whole simulation instead is an atomic
+// on one address per cell, about 20 ns each: it alone bounded the 3D cell kernel.)
+__device__ __forceinline__ int32_t v_place_faces(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int chunk,
+                                                 int cnt) {
+  const int32_t share = (int32_t)(D.face_cap / (D.cchunk1 - D.cchunk0));
+  const int32_t p = atomicAdd(&V.part1[chunk], cnt);
+  if (p + cnt <= share) return (int32_t)(D.face_base + (int64_t)(chunk - D.cchunk0) * share + p);
+  const int32_t o = atomicAdd(&S.nf_tmp, cnt);
+  return (int64_t)o + cnt <= D.face_cap ? (int32_t)(B.F.nf + D.face_base + o) : -1;
+}
+
 // The finished cell: area and centroid summed over the edges in order (the host tessellator's
 // Cell2::finish), the emitted faces appended to vf in edge order, and the cell's geometry
 // (Particle::update_geometry, part.rs:151-158).
@@ -205,8 +218,8 @@ __device__ void v2_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, Sim
     const double q = bxx * bxx + byy * byy;
     r2 = r2 < q ? q : r2;
   }
-  const int32_t start = atomicAdd(&S.nf_tmp, cnt);
-  if ((int64_t)start + cnt > D.face_cap) {
+  const int32_t start = v_place_faces(B, V, D, S, chunk, cnt);
+  if (start < 0) {
     V.femit[gi] = 0;
     atomicCAS(&B.cnt->err, 0, E_MESH);
     atomicCAS(&S.err, 0, E_MESH);
@@ -214,8 +227,7 @@ __device__ void v2_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, Sim
   }
   V.vst[gi] = start;
   V.femit[gi] = cnt;
-  if (cnt) atomicAdd(&V.part1[chunk], cnt);
-  V2Face* out = V.vf + D.face_base + start;
+  V2Face* out = V.vf + start;
   int q = 0;
   for (int k = 0; k < m; ++k) {
     const int km = k == 0 ? m - 1 : k - 1;
@@ -755,9 +767,9 @@ __device__ __forceinline__ void v2_reg_finish(const Batch& B, const V2Bufs& V, c
   const uint32_t em = team_ballot(emit, tiw);
   const int cnt = __popc(em);
   int32_t start = 0;
-  if (lane == 0) start = atomicAdd(&S.nf_tmp, cnt);
+  if (lane == 0) start = v_place_faces(B, V, D, S, chunk, cnt);
   start = __shfl(start, 0, HFV_V2_TEAM);
-  if ((int64_t)start + cnt > D.face_cap) {
+  if (start < 0) {
     if (lane == 0) {
       V.femit[gi] = 0;
       atomicCAS(&B.cnt->err, 0, E_MESH);
@@ -777,12 +789,11 @@ __device__ __forceinline__ void v2_reg_finish(const Batch& B, const V2Bufs& V, c
     f.nz = 0.;
     f.nb = P.nb < 0 ? -1 : P.nb;
     f.code = P.code;
-    V.vf[D.face_base + start + __popc(em & ((1u << lane) - 1u))] = f;
+    V.vf[start + __popc(em & ((1u << lane) - 1u))] = f;
   }
   if (lane != 0) return;
   V.vst[gi] = start;
   V.femit[gi] = cnt;
-  if (cnt) atomicAdd(&V.part1[chunk], cnt);
   if (B.C.act[gi]) {
     B.C.vol[gi] = area;
     const double ia = area > 0. ? 1.0 / area : 0.;
@@ -865,8 +876,15 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
   const int32_t base = chunks_before(V.part1, D, J.chunk, &all);
   offs[threadIdx.x] = block_excl_scan(in ? V.femit[gi0] : 0, &tot);
   starts[threadIdx.x] = in ? V.vst[gi0] : 0;
-  const bool bad = S.err != 0;  // a failed cell emitted nothing: the simulation stops
-  if (J.chunk == D.cchunk0 && threadIdx.x == 0) B.eng[s].nf_mesh = bad ? 0 : all;
+  const bool full = all > D.face_cap;
+  const bool bad = full || S.err != 0;  // a failed cell emitted nothing: the simulation stops
+  if (J.chunk == D.cchunk0 && threadIdx.x == 0) {
+    B.eng[s].nf_mesh = bad ? 0 : all;
+    if (full) {
+      atomicCAS(&B.cnt->err, 0, E_MESH);
+      atomicCAS(&S.err, 0, E_MESH);
+    }
+  }
   __syncthreads();
   if (bad) return;
   const Faces& F = B.F;
@@ -877,7 +895,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
       if (offs[lo + h] <= t) lo += h;
     const int64_t gi = (int64_t)J.lo + lo;
     const int64_t f = D.face_base + base + t;
-    const V2Face r = V.vf[D.face_base + starts[lo] + (t - offs[lo])];
+    const V2Face r = V.vf[starts[lo] + (t - offs[lo])];
     F.area[f] = r.area;
     F.nrm[f] = r.nx;
     F.nrm[NF + f] = r.ny;

@@ -783,9 +783,9 @@ __device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimS
   const uint64_t me = __ballot(emit);
   const int cnt = __popcll(me);
   int start = 0;
-  if (lane == 0) start = atomicAdd(&S.nf_tmp, cnt);
+  if (lane == 0) start = v_place_faces(B, V, D, S, chunk, cnt);
   start = __shfl(start, 0, 64);
-  if ((int64_t)start + cnt > D.face_cap) {
+  if (start < 0) {
     if (lane == 0) {
       V.femit[gi] = 0;
       atomicCAS(&B.cnt->err, 0, E_MESH);
@@ -805,13 +805,12 @@ __device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimS
     f.nz = inv * C.pz[p];
     f.nb = pnb < 0 ? -1 : pnb;
     f.code = C.pcode[p];
-    V.vf[D.face_base + start + __popcll(me & ((1ull << lane) - 1ull))] = f;
+    V.vf[start + __popcll(me & ((1ull << lane) - 1ull))] = f;
   }
   wave_sync();
   if (lane != 0) return 0;
   V.vst[gi] = start;
   V.femit[gi] = cnt;
-  if (cnt) atomicAdd(&V.part1[chunk], cnt);
   // the cell's volume and centroid: the tetrahedron terms added in the host's order
   double vol = 0., cenx = 0., ceny = 0., cenz = 0.;
   for (int q = 0; q < ntri; ++q) {
