@@ -1138,7 +1138,10 @@ void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
     hipLaunchKernelGGL(k_v2_bins, gc, gb, 0, st, B, V);
     hipLaunchKernelGGL(k_v2_place, gc, gb, 0, st, B, V);
     if (c->any_vmesh2) hipLaunchKernelGGL(k_v2_cells, dim3((unsigned)(c->ncg * HFV_V2_SUB)), gb, 0, st, B, V);
-    if (c->any_vmesh3) hipLaunchKernelGGL(k_v3_cells, dim3((unsigned)(c->ncg * BLOCK)), dim3(64), 0, st, B, V);
+    if (c->any_vmesh3) {
+      hipLaunchKernelGGL(k_v3_cells_reg, dim3((unsigned)(c->ncg * HFV_V3R_SUB)), dim3(256), 0, st, B, V);
+      hipLaunchKernelGGL(k_v3_cells, dim3((unsigned)(c->ncg * HFV_V3_SUB)), dim3(64), 0, st, B, V);
+    }
     hipLaunchKernelGGL(k_v2_faces, gc, gb, 0, st, B, V);
     hipLaunchKernelGGL(k_v2_sum<1>, gc, gb, 0, st, B, V);
     hipLaunchKernelGGL(k_v2_conn, gc, gb, 0, st, B, V);

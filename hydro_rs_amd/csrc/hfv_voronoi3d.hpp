@@ -12,15 +12,15 @@
 // others in order and appends the new ones.  The faces are the planes' vertex fans chained into polygons;
 // area vector, centroid and the cell's volume and centroid are the host's triangle-fan sums in its order.
 //
-// One wavefront (a block of its own) builds one cell, everything in LDS: the block's candidates are
-// gathered once per K and ranked by their key (each lane ranks every 64th candidate against all), then
-// taken in rank order; a clip reads each vertex once (two per lane), lists the removed ones with two
-// ballots, compacts the kept ones from registers and makes the new ones one boundary edge per lane; the
-// largest vertex radius is a DPP reduction over the lanes' kept and new vertices.  The finish builds each
-// plane's fan and polygon on its own lane, with the face sums and the cell's tetrahedron terms, which one
-// lane then adds in the host's order.  Blocks of more than HFV_V3_CAP candidates are taken in bands of
-// squared distance that fit (chosen from an LDS histogram); only a band that cannot be narrowed enough
-// takes each next candidate as a wave minimum over a rescan of the bins.
+// One wavefront builds one cell: k_v3_cells_reg with the vertices in registers, and the few cells that outgrow
+// it k_v3_cells with everything in LDS: the block's candidates are gathered once per K and ranked by their key
+// (each lane ranks every 64th candidate against all), then taken in rank order; a clip reads each vertex once
+// (two per lane), lists the removed ones with two ballots, compacts the kept ones from registers and makes the
+// new ones one boundary edge per lane; the largest vertex radius is a DPP reduction over the lanes' kept and new
+// vertices.  The finish builds each plane's fan and polygon on its own lane, with the face sums and the cell's
+// tetrahedron terms, which one lane then adds in the host's order.  Blocks of more than HFV_V3_CAP candidates
+// are taken in bands of squared distance that fit (chosen from an LDS histogram); only a band that cannot be
+// narrowed enough takes each next candidate as a wave minimum over a rescan of the bins.
 #pragma once
 
 namespace hfv {
@@ -90,7 +90,8 @@ __device__ __forceinline__ double v3dot(double ax, double ay, double az, double 
 }
 
 // intersect3 of planes a, b and (cn, cd): false where they meet in no point
-__device__ __forceinline__ bool v3_intersect(const V3Cell& C, int a, int b, double cnx, double cny, double cnz,
+template <class Cell>
+__device__ __forceinline__ bool v3_intersect(const Cell& C, int a, int b, double cnx, double cny, double cnz,
                                              double cd, double& ox, double& oy, double& oz) {
   const double anx = C.px[a], any = C.py[a], anz = C.pz[a], ad = C.pd[a];
   const double bnx = C.px[b], bny = C.py[b], bnz = C.pz[b], bd = C.pd[b];
@@ -830,36 +831,573 @@ __device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimS
   return 0;
 }
 
-// grid: HFV_BLOCK one-wavefront blocks per cell chunk, one cell each
-__global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V) {
-  __shared__ V3Cell C;
-  const BlockJob J = B.cjobs[blockIdx.x / HFV_BLOCK];
+// ---------------------------------------------------------------- cells with their vertices in registers
+// The same cell by one wavefront with vertex t on lane t, which the ordinary cell fits (a cell of 15 faces has
+// 27 vertices).  A clip is a ballot of the vertices beyond the plane; where it cuts, the removed triangles are
+// read as scalars, each of their edges is tested on a lane of its own, one permute sends the boundary edges to
+// the next free lanes, and those become the new vertices: kept vertices stay where they are (their order is
+// the host's), and close up only when the lanes run out.  Candidates come in bands of squared distance that
+// hold about 45 generators each (the first is enough for most cells), so that a band is ranked with one key a
+// lane.  A cell that outgrows this (64 live vertices, 64 candidates in a band, a face of more than 12 vertices)
+// is left to k_v3_cells.
+// What bounds it: instruction issue, FP64 and integer alike at 4 cycles a wave (about 250 instructions a cutting
+// clip, 16 of them a cell).  7 KB of LDS and 128 VGPRs let 16 waves a CU hide each other's latencies, where
+// the LDS cell has 15 KB (10 waves) and spends 66k of its 126k cycles a cell on clips (LDS round trips), 30k on
+// the finish and 14k on ranking 124 candidates.  KH 48^3, steered generators (8 steps and the state's copy):
+// 16.3 -> 12.2 ms, the rebuild 1.73 -> 1.25 ms a step.
+#define HFV_V3R_CAP 64  // candidates of a band: one a lane
+#define HFV_V3R_FAN 12  // vertices of a face
+#define HFV_V3R_TRI 96  // fan triangles of a cell
+#define HFV_V3_LEFT (-1)  // femit mark: the cell is left to k_v3_cells
+
+struct V3RCands {
+  V3Key key[HFV_V3R_CAP];
+  double rx[HFV_V3R_CAP], ry[HFV_V3R_CAP], rz[HFV_V3R_CAP];
+  uint8_t ord[HFV_V3R_CAP];
+  int32_t n;
+};
+struct V3RFin {
+  double tx[64], ty[64], tz[64];
+  union {
+    uint32_t fan[HFV_V3_MAXP][HFV_V3R_FAN];  // u | v << 8 | vertex << 16, in vertex order
+    double q[4][HFV_V3R_TRI];                // tetrahedron terms: volume, centroid numerators
+  } u;
+};
+struct V3RCell {
+  double px[HFV_V3_MAXP], py[HFV_V3_MAXP], pz[HFV_V3_MAXP], pd[HFV_V3_MAXP];
+  int32_t pnb[HFV_V3_MAXP], pcode[HFV_V3_MAXP];
+  union {
+    V3RCands q;
+    V3RFin f;
+  } u;
+};
+
+// This lane's vertex (at the generator where there is none: no plane cuts it off), and the wave's: which lanes
+// hold one (live), the first lane never used (top).
+struct V3RVerts {
+  double x, y, z, q;  // q = its squared radius
+  uint32_t tp;        // plane ids a | b << 8 | c << 16
+  uint64_t live;
+  int top;
+};
+
+template <int CTRL, int ROW>
+__device__ __forceinline__ uint32_t dpp_umax_step(uint32_t v) {
+  const uint32_t t = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROW, 0xf, false);
+  return v < t ? t : v;
+}
+__device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
+  v = dpp_umax_step<0x111, 0xf>(v);
+  v = dpp_umax_step<0x112, 0xf>(v);
+  v = dpp_umax_step<0x114, 0xf>(v);
+  v = dpp_umax_step<0x118, 0xf>(v);
+  v = dpp_umax_step<0x142, 0xa>(v);
+  v = dpp_umax_step<0x143, 0xc>(v);
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// maximum of non-negative doubles (which order as their bits) over the wavefront
+__device__ __forceinline__ double wave_max_nonneg(double v) {
+  const uint32_t hi = (uint32_t)__double2hiint(v), top = wave_umax(hi);
+  const uint32_t lo = wave_umax(hi == top ? (uint32_t)__double2loint(v) : 0u);
+  return __hiloint2double((int)top, (int)lo);
+}
+__device__ __forceinline__ double readlane_f64(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l), __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+__device__ __forceinline__ double permute_f64(int addr, double v) {
+  return __hiloint2double(__builtin_amdgcn_ds_permute(addr, __double2hiint(v)),
+                          __builtin_amdgcn_ds_permute(addr, __double2loint(v)));
+}
+
+// Live vertices close up to the lowest lanes, in order.
+__device__ __forceinline__ void v3r_close(V3RVerts& T) {
+  const int lane = __lane_id();
+  const bool mine = (T.live >> lane) & 1ull;
+  const int n = __popcll(T.live);
+  // (lanes without a vertex send to the last lane: it is not a target unless every lane is live)
+  const int to = (mine ? __popcll(T.live & ((1ull << lane) - 1ull)) : 63) << 2;
+  T.x = permute_f64(to, T.x);
+  T.y = permute_f64(to, T.y);
+  T.z = permute_f64(to, T.z);
+  T.q = permute_f64(to, T.q);
+  T.tp = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)T.tp);
+  T.live = n == 64 ? ~0ull : (1ull << n) - 1ull;
+  if (lane >= n) T.x = T.y = T.z = T.q = 0.;
+  T.top = n;
+}
+
+// Cell3::clip by plane (n, d, nb, code): 0 no cut, 1 cut, -1 more than the lanes hold.
+__device__ __forceinline__ int v3r_clip(V3RCell& C, V3RVerts& T, int& np, double nx, double ny, double nz, double d,
+                                        int32_t nb, int32_t code) {
+  const int lane = __lane_id();
+  const double dth = d + HFV_CLIP_TOL * d;  // (beyond by more than a rounding error)
+  uint64_t mr = __ballot(v3dot(nx, ny, nz, T.x, T.y, T.z) > dth);  // (d > 0: lanes without a vertex are inside)
+  if (mr == 0 || mr == T.live) return 0;
+  const int nrem = __popcll(mr);
+  if (np + 1 > HFV_V3_MAXP || 3 * nrem > 64) return -1;
+  if (T.top + nrem + 2 > 64) {  // (a closed cell's removed region has nrem + 2 boundary edges)
+    v3r_close(T);
+    mr = __ballot(v3dot(nx, ny, nz, T.x, T.y, T.z) > dth);
+  }
+  // lane e: edge e % 3 of the removed vertex e / 3, in (removed vertex, edge) order
+  const int rq = lane / 3, e = lane - 3 * rq;
+  uint32_t w = 0;
+  int idx = 0;
+  for (uint64_t m = mr; m; m &= m - 1, ++idx) {
+    const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)T.tp, __builtin_ctzll(m));
+    w = rq == idx ? t : w;
+  }
+  const uint32_t a0 = w & 0xFF, a1 = (w >> 8) & 0xFF, a2 = w >> 16;
+  const uint32_t ex = e == 0 ? a0 : e == 1 ? a1 : a2, ey = e == 0 ? a1 : e == 1 ? a2 : a0;
+  const uint32_t back = ey | (ex << 8);  // internal: another removed vertex has the edge (y, x)
+  bool internal = lane >= 3 * nrem;
+  for (uint64_t m = mr; m; m &= m - 1) {
+    const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)T.tp, __builtin_ctzll(m));
+    const uint32_t t01 = t & 0xFFFF, t12 = t >> 8, t20 = (t >> 16) | ((t & 0xFF) << 8);
+    internal = internal | (back == t01) | (back == t12) | (back == t20);
+  }
+  const uint64_t mb = __ballot(!internal);
+  const int nnew = __popcll(mb);
+  if (T.top + nnew > 64) return -1;
+  // boundary edges to the next free lanes, in order (the others send to lane 0, which is in use)
+  const int to = internal ? 0 : T.top + __popcll(mb & ((1ull << lane) - 1ull));
+  const uint32_t got = (uint32_t)__builtin_amdgcn_ds_permute(to << 2, (int)(ex | (ey << 8)));
+  const bool fresh = lane >= T.top && lane < T.top + nnew;
+  const int x = got & 0xFF, y = (got >> 8) & 0xFF;
+  double ox = 0., oy = 0., oz = 0.;
+  const bool fb = fresh && !v3_intersect(C, x, y, nx, ny, nz, d, ox, oy, oz);
+  // (rare) the three planes meet in no point: where the edge (x, y) from the removed vertex to the vertex
+  // across it (the first with the edge (y, x), a kept one) crosses the plane; the removed vertex's
+  // position where that is no crossing
+  for (uint64_t todo = __ballot(fb); todo; todo &= todo - 1) {
+    const int L = __builtin_ctzll(todo);
+    const uint32_t g = (uint32_t)__builtin_amdgcn_readlane((int)got, L);
+    const uint32_t bk = ((g >> 8) & 0xFF) | ((g & 0xFF) << 8);
+    const uint32_t t = T.tp, t01 = t & 0xFFFF, t12 = t >> 8, t20 = (t >> 16) | ((t & 0xFF) << 8);
+    const uint64_t k = __ballot((bk == t01) | (bk == t12) | (bk == t20)) & T.live;
+    const int rl = __builtin_ctzll(__ballot((g == t01) | (g == t12) | (g == t20)) & mr);  // the removed one with (x, y)
+    const double tx = readlane_f64(T.x, rl), ty = readlane_f64(T.y, rl), tz = readlane_f64(T.z, rl);
+    double cx = tx, cy = ty, cz = tz;
+    if (k) {
+      const int us = __builtin_ctzll(k);
+      const double ux = readlane_f64(T.x, us), uy = readlane_f64(T.y, us), uz = readlane_f64(T.z, us);
+      const double a = v3dot(nx, ny, nz, ux, uy, uz) - d, b = v3dot(nx, ny, nz, tx, ty, tz) - d;
+      if (a <= 0.0 && b > a) {
+        const double sc = a / (a - b);
+        cx = ux + sc * (tx - ux);
+        cy = uy + sc * (ty - uy);
+        cz = uz + sc * (tz - uz);
+      }
+    }
+    if (lane == L) {
+      ox = cx;
+      oy = cy;
+      oz = cz;
+    }
+  }
+  if ((mr >> lane) & 1ull) T.x = T.y = T.z = T.q = 0.;
+  if (fresh) {
+    T.x = ox;
+    T.y = oy;
+    T.z = oz;
+    T.tp = (uint32_t)x | ((uint32_t)y << 8) | ((uint32_t)np << 16);
+    T.q = v3dot(ox, oy, oz, ox, oy, oz);
+  }
+  if (lane == 0) {
+    C.px[np] = nx;
+    C.py[np] = ny;
+    C.pz[np] = nz;
+    C.pd[np] = d;
+    C.pnb[np] = nb;
+    C.pcode[np] = code;
+  }
+  wave_sync();
+  T.live = (T.live & ~mr) | ((nnew == 64 ? ~0ull : (1ull << nnew) - 1ull) << T.top);
+  T.top += nnew;
+  np += 1;
+  return 1;
+}
+
+// The block's candidates of squared distance in [lo, hi) into LDS and ranked: their count, -1 beyond HFV_V3R_CAP.
+__device__ __forceinline__ int v3r_band(const Batch& B, const SimDesc& D, const V2Bufs& V, int s, int32_t i, double xi,
+                                        double yi, double zi, int K, V3RCell& C, double lo, double hi) {
+  const int lane = __lane_id();
+  V3RCands& Q = C.u.q;
+  const int64_t N = B.C.n, cb = D.cell_base;
+  const double* L = B.C.loc;
+  const int32_t* gst = V.gcnt + cb + s;
+  const int32_t* gord = V.gord + cb;
+  wave_sync();
+  if (lane == 0) Q.n = 0;
+  wave_sync();
+  v3_lane_bins(D, xi, yi, zi, K, [&](int key, int s0, int s1, int s2, bool) {
+    const int32_t kk = ((s0 & 0xFF) << 16) | ((s1 & 0xFF) << 8) | (s2 & 0xFF);  // the host's memcmp order
+    const int32_t g0 = gst[key], g1 = gst[key + 1];
+    for (int32_t q0 = g0; q0 < g1; q0 += 2) {  // (two candidates' loads in flight)
+      int32_t jj[2];
+      double x[2], y[2], z[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) jj[u] = q0 + u < g1 ? gord[q0 + u] : -1;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int64_t gj = cb + (jj[u] < 0 ? 0 : jj[u]);
+        x[u] = L[gj];
+        y[u] = L[N + gj];
+        z[u] = L[2 * N + gj];
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (jj[u] < 0 || (jj[u] == i && s0 == 0 && s1 == 0 && s2 == 0)) continue;
+        const double rx = (x[u] + (double)s0 * D.cfg.box[0]) - xi, ry = (y[u] + (double)s1 * D.cfg.box[1]) - yi,
+                     rz = (z[u] + (double)s2 * D.cfg.box[2]) - zi;
+        const double d2 = v3dot(rx, ry, rz, rx, ry, rz);
+        if (!(d2 >= lo && d2 < hi)) continue;
+        const int at = atomicAdd(&Q.n, 1);  // (any order: the rank orders them)
+        if (at >= HFV_V3R_CAP) continue;
+        V3Key key3;
+        key3.d2 = d2;
+        key3.j = jj[u];
+        key3.k = kk;
+        Q.key[at] = key3;
+        Q.rx[at] = rx;
+        Q.ry[at] = ry;
+        Q.rz[at] = rz;
+      }
+    }
+  });
+  wave_sync();
+  const int n = __builtin_amdgcn_readfirstlane(Q.n);
+  if (n > HFV_V3R_CAP) return -1;
+  // the rank of this lane's candidate: the number of keys below it, by the squared distance (a non-negative
+  // double orders as its bits), by the whole key where two squared distances are equal
+  const V3Key own = Q.key[lane < n ? lane : 0];
+  const uint64_t od = (uint64_t)__double_as_longlong(own.d2);
+  int rk = 0, le = 0;
+  for (int b = 0; b < n; b += 8) {
+    uint64_t db[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) db[u] = b + u < n ? (uint64_t)__double_as_longlong(Q.key[b + u].d2) : ~0ull;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      rk += db[u] < od ? 1 : 0;
+      le += db[u] <= od ? 1 : 0;
+    }
+  }
+  if (__ballot(lane < n && le - rk > 1)) {
+    for (int b = 0; b < n; ++b) {
+      const V3Key kb = Q.key[b];
+      rk += (uint64_t)__double_as_longlong(kb.d2) == od && (kb.j < own.j || (kb.j == own.j && kb.k < own.k)) ? 1 : 0;
+    }
+  }
+  if (lane < n) Q.ord[rk] = (uint8_t)lane;
+  wave_sync();
+  return n;
+}
+
+// The cell for candidate bins within K: 0 clipped (finish next), 1 retry with a larger K, 2 left to k_v3_cells.
+__device__ __forceinline__ int v3r_build(const Batch& B, const SimDesc& D, const V2Bufs& V, int s, int32_t i, double xi,
+                                         double yi, double zi, int K, V3RCell& C, V3RVerts& T, int& np, double& r2) {
+  const int lane = __lane_id();
+  const double w0 = D.vw[0], w1 = D.vw[1], w2 = D.vw[2];
+  const bool per = D.periodic != 0;
+  double reach = 0.;
+  reach = reach < K * w0 ? K * w0 : reach;
+  reach = reach < K * w1 ? K * w1 : reach;
+  reach = reach < K * w2 ? K * w2 : reach;
+  const double lo[3] = {per ? -reach : -xi, per ? -reach : -yi, per ? -reach : -zi};
+  const double hi[3] = {per ? reach : D.cfg.box[0] - xi, per ? reach : D.cfg.box[1] - yi,
+                        per ? reach : D.cfg.box[2] - zi};
+  wave_sync();
+  if (lane < 6) {  // walls 0:-x 1:+x 2:-y 3:+y 4:-z 5:+z
+    const int a = lane >> 1;
+    const bool up = lane & 1;
+    C.px[lane] = a == 0 ? (up ? 1. : -1.) : 0.;
+    C.py[lane] = a == 1 ? (up ? 1. : -1.) : 0.;
+    C.pz[lane] = a == 2 ? (up ? 1. : -1.) : 0.;
+    C.pd[lane] = up ? (a == 0 ? hi[0] : a == 1 ? hi[1] : hi[2]) : -(a == 0 ? lo[0] : a == 1 ? lo[1] : lo[2]);
+    C.pnb[lane] = -1 - lane;
+    C.pcode[lane] = 0;
+  }
+  wave_sync();
+  T.x = T.y = T.z = T.q = 0.;
+  T.tp = 0;
+  if (lane < 8) {  // the cube's corners (sx, sy, sz), oriented so that det(n_a, n_b, n_c) > 0
+    const int a = lane >> 2, b = 2 + ((lane >> 1) & 1), c = 4 + (lane & 1);
+    const double cx = C.py[b] * C.pz[c] - C.pz[b] * C.py[c], cy = C.pz[b] * C.px[c] - C.px[b] * C.pz[c],
+                 cz = C.px[b] * C.py[c] - C.py[b] * C.px[c];
+    const double det = v3dot(C.px[a], C.py[a], C.pz[a], cx, cy, cz);
+    const int t0 = det > 0 ? a : b, t1 = det > 0 ? b : a;
+    T.tp = (uint32_t)t0 | ((uint32_t)t1 << 8) | ((uint32_t)c << 16);
+    v3_intersect(C, t0, t1, C.px[c], C.py[c], C.pz[c], C.pd[c], T.x, T.y, T.z);
+    T.q = v3dot(T.x, T.y, T.z, T.x, T.y, T.z);
+  }
+  T.live = 0xFFull;
+  T.top = 8;
+  np = 6;
+  const V3RCands& Q = C.u.q;
+  // bands of equal volume: radii 2.2 mean bin widths times the cube roots of 1, 2, 3, 4, then all the rest
+  const double t0 = 4.84 * ((w0 * w0 + w1 * w1 + w2 * w2) / 3.);
+  double blo = 0.;
+  bool stop = false;
+  for (int band = 0; band < 5 && !stop; ++band) {
+    const double bhi = band == 0 ? t0 : band == 1 ? 1.5874 * t0 : band == 2 ? 2.0801 * t0 : band == 3 ? 2.5198 * t0
+                                                                                                   : (double)INFINITY;
+    const int n = v3r_band(B, D, V, s, i, xi, yi, zi, K, C, blo, bhi);
+    if (n < 0) return 2;
+    for (int q = 0; q < n; ++q) {
+      const int a = __builtin_amdgcn_readfirstlane(Q.ord[q]);
+      const V3Key key = Q.key[a];
+      if (!__ballot(T.q >= 0.25 * key.d2)) {  // security radius: the bisector lies beyond every vertex
+        stop = true;
+        break;
+      }
+      if (v3r_clip(C, T, np, Q.rx[a], Q.ry[a], Q.rz[a], 0.5 * key.d2, key.j, v3_code_of(key.k)) < 0) return 2;
+    }
+    // every later candidate is at least this band's end away
+    if (!__ballot(T.q >= 0.25 * bhi)) stop = true;
+    blo = bhi;
+  }
+  r2 = wave_max_nonneg(T.q);
+  // completeness: every unvisited generator lies farther than K bin widths
+  double minw = 1e300;
+  minw = K * w0 < minw ? K * w0 : minw;
+  minw = K * w1 < minw ? K * w1 : minw;
+  minw = K * w2 < minw ? K * w2 : minw;
+  return 4.0 * r2 > minw * minw ? 1 : 0;
+}
+
+// v3_finish of a register cell: 0, 1 (retry with a larger K) or 2 (left to k_v3_cells).
+__device__ __forceinline__ int v3r_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int chunk,
+                                          int64_t gi, int32_t i, double xi, double yi, double zi, V3RCell& C,
+                                          const V3RVerts& T, int np, double r2) {
+  const int lane = __lane_id();
+  const int p = lane;
+  V3RFin& F = C.u.f;  // over the candidates, read for the last time before
+  wave_sync();
+  if ((T.live >> lane) & 1ull) {
+    const int t = __popcll(T.live & ((1ull << lane) - 1ull));
+    F.tx[t] = T.x;
+    F.ty[t] = T.y;
+    F.tz[t] = T.z;
+  }
+  // plane p's fan: its vertices rotated to (p, u, v), in vertex order
+  int f = 0;
+  {
+    uint32_t t = 0;
+    for (uint64_t m = T.live; m; m &= m - 1, ++t) {
+      const uint32_t w = (uint32_t)__builtin_amdgcn_readlane((int)T.tp, __builtin_ctzll(m));
+      const uint32_t a = w & 0xFF, b = (w >> 8) & 0xFF, c = w >> 16;
+      const bool ia = a == (uint32_t)p, ib = b == (uint32_t)p, ic = c == (uint32_t)p;
+      const uint32_t uv = ia ? (b | (c << 8)) : ib ? (c | (a << 8)) : (a | (b << 8));
+      if (ia | ib | ic) {
+        if (f < HFV_V3R_FAN) F.u.fan[p][f] = uv | (t << 16);
+        ++f;
+      }
+    }
+  }
+  if (p >= np) f = 0;
+  if (__ballot(f > HFV_V3R_FAN)) return 2;
+  // chained into a polygon: from (u, v) the next entry around p is the first one whose u is this v
+  uint32_t ent[HFV_V3R_FAN];
+#pragma unroll
+  for (int k = 0; k < HFV_V3R_FAN; ++k) ent[k] = k < f ? F.u.fan[p][k] : 0xFFu;  // (no plane id)
+  uint32_t poly[HFV_V3R_FAN];
+  int m = 0;
+  if (f >= 3) {
+    uint32_t cur = ent[0];
+    bool on = true;
+#pragma unroll
+    for (int k = 0; k < HFV_V3R_FAN; ++k) {
+      poly[k] = cur >> 16;
+      if (on && k < f) m = k + 1;
+      const uint32_t want = (cur >> 8) & 0xFF;
+      uint32_t nxt = 0xFFFFFFFFu;
+#pragma unroll
+      for (int e = HFV_V3R_FAN - 1; e >= 0; --e) nxt = (ent[e] & 0xFF) == want ? ent[e] : nxt;
+      // the chain ends where no entry follows, at the first entry again, or after f of them
+      on = on && k + 1 < f && nxt != 0xFFFFFFFFu && nxt != ent[0];
+      cur = on ? nxt : cur;
+    }
+  }
+  if (m < 3) m = 0;
+  // the plane's fan triangles: their place among the cell's (planes in order), by a wave prefix sum
+  const int nq = m >= 3 ? m - 2 : 0;
+  int incl = nq;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += t;
+  }
+  const int ntri = __builtin_amdgcn_readlane(incl, 63);
+  if (ntri > HFV_V3R_TRI) return 2;
+  const int q0 = incl - nq;
+  wave_sync();  // the fans are read no more: their place takes the terms
+  // the face's area vector and centroid; the cell's tetrahedron terms (vertex fan with the generator)
+  double area = 0., fcx = 0., fcy = 0., fcz = 0.;
+  if (m >= 3) {
+    const double p0x = F.tx[poly[0]], p0y = F.ty[poly[0]], p0z = F.tz[poly[0]];
+    double avx = 0., avy = 0., avz = 0., acx = 0., acy = 0., acz = 0., asum = 0.;
+    double Ax = F.tx[poly[1]], Ay = F.ty[poly[1]], Az = F.tz[poly[1]];
+#pragma unroll
+    for (int k = 1; k + 1 < HFV_V3R_FAN; ++k) {
+      if (k + 1 >= m) break;
+      const double Bx = F.tx[poly[k + 1]], By = F.ty[poly[k + 1]], Bz = F.tz[poly[k + 1]];
+      const double ax = Ax - p0x, ay = Ay - p0y, az = Az - p0z, bx = Bx - p0x, by = By - p0y, bz = Bz - p0z;
+      const double crx = ay * bz - az * by, cry = az * bx - ax * bz, crz = ax * by - ay * bx;
+      const double a = 0.5 * sqrt(v3dot(crx, cry, crz, crx, cry, crz));
+      avx = avx + 0.5 * crx;
+      avy = avy + 0.5 * cry;
+      avz = avz + 0.5 * crz;
+      asum += a;
+      const double s3 = a / 3.0;
+      acx = acx + s3 * ((p0x + Ax) + Bx);
+      acy = acy + s3 * ((p0y + Ay) + By);
+      acz = acz + s3 * ((p0z + Az) + Bz);
+      const double ux = Ay * Bz - Az * By, uy = Az * Bx - Ax * Bz, uz = Ax * By - Ay * Bx;
+      const double tv = fabs(v3dot(p0x, p0y, p0z, ux, uy, uz)) / 6.0;
+      const double s4 = tv / 4.0;
+      const int qi = q0 + k - 1;
+      F.u.q[0][qi] = tv;
+      F.u.q[1][qi] = s4 * ((p0x + Ax) + Bx);
+      F.u.q[2][qi] = s4 * ((p0y + Ay) + By);
+      F.u.q[3][qi] = s4 * ((p0z + Az) + Bz);
+      Ax = Bx;
+      Ay = By;
+      Az = Bz;
+    }
+    area = sqrt(v3dot(avx, avy, avz, avx, avy, avz));
+    if (asum > 0) {
+      const double inv = 1.0 / asum;
+      fcx = inv * acx;
+      fcy = inv * acy;
+      fcz = inv * acz;
+    } else {
+      fcx = p0x;
+      fcy = p0y;
+      fcz = p0z;
+    }
+  }
+  const int32_t pnb = p < np ? C.pnb[p] : 0;
+  // a periodic cell must not touch the initial region (a wall face of positive area)
+  if (D.periodic && __ballot(p < np && pnb < 0 && area > 0.)) return 1;
+  const int64_t cb = D.cell_base, N = B.C.n;
+  const bool emit = p < np && area > 0. && v2_emits(B, cb, pnb, i);
+  const uint64_t me = __ballot(emit);
+  const int cnt = __popcll(me);
+  int start = 0;
+  if (lane == 0) start = v_place_faces(B, V, D, S, chunk, cnt);
+  start = __builtin_amdgcn_readfirstlane(start);
+  if (start < 0) {
+    if (lane == 0) {
+      V.femit[gi] = 0;
+      atomicCAS(&B.cnt->err, 0, E_MESH);
+      atomicCAS(&S.err, 0, E_MESH);
+    }
+    return 0;
+  }
+  if (emit) {
+    const double inv = 1.0 / sqrt(v3dot(C.px[p], C.py[p], C.pz[p], C.px[p], C.py[p], C.pz[p]));
+    V2Face o;
+    o.area = area;
+    o.cx = fcx;
+    o.cy = fcy;
+    o.cz = fcz;
+    o.nx = inv * C.px[p];
+    o.ny = inv * C.py[p];
+    o.nz = inv * C.pz[p];
+    o.nb = pnb < 0 ? -1 : pnb;
+    o.code = C.pcode[p];
+    V.vf[start + __popcll(me & ((1ull << lane) - 1ull))] = o;
+  }
+  wave_sync();
+  // the cell's volume and centroid: the tetrahedron terms added in the host's order, one sum a lane
+  double sum = 0.;
+  for (int q = 0; q < ntri; ++q) sum = sum + F.u.q[lane & 3][q];
+  const double vol = readlane_f64(sum, 0), cenx = readlane_f64(sum, 1), ceny = readlane_f64(sum, 2),
+               cenz = readlane_f64(sum, 3);
+  if (lane != 0) return 0;
+  V.vst[gi] = start;
+  V.femit[gi] = cnt;
+  if (B.C.act[gi]) {  // Particle::update_geometry (part.rs:151-158)
+    B.C.vol[gi] = vol;
+    const double iv = vol > 0. ? 1.0 / vol : 0.;
+    B.C.cen[gi] = xi + (vol > 0. ? iv * cenx : 0.);
+    B.C.cen[N + gi] = yi + (vol > 0. ? iv * ceny : 0.);
+    B.C.cen[2 * N + gi] = zi + (vol > 0. ? iv * cenz : 0.);
+    B.C.srad[gi] = 1.5 * 2.0 * sqrt(r2);
+  }
+  return 0;
+}
+
+// grid: HFV_BLOCK / 4 blocks per cell chunk, a wavefront a cell
+#define HFV_V3R_SUB (HFV_BLOCK / 4)
+__global__ void __launch_bounds__(256, 4) k_v3_cells_reg(Batch B, V2Bufs V) {
+  __shared__ V3RCell cells[4];
+  const BlockJob J = B.cjobs[blockIdx.x / HFV_V3R_SUB];
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
   SimStep& S = B.st[s];
   if (D.vmesh != 3 || !S.stepping) return;
-  const int64_t gi = (int64_t)J.lo + blockIdx.x % HFV_BLOCK;
-  if (gi >= J.hi) return;
-  if (__lane_id() == 0) V.ccnt[gi] = 0;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t gi = (int64_t)J.lo + (blockIdx.x % HFV_V3R_SUB) * 4 + wave;
+  if (gi >= J.hi) return;  // (no block barrier follows)
+  const int lane = __lane_id();
+  if (lane == 0) V.ccnt[gi] = 0;
   if (!B.C.act[gi]) {  // unbuilt in a partial build
-    if (__lane_id() == 0) V.femit[gi] = 0;
+    if (lane == 0) V.femit[gi] = 0;
     return;
   }
+  V3RCell& C = cells[wave];
   const int64_t N = B.C.n, cb = D.cell_base;
   const int32_t i = (int32_t)(gi - cb);
   const double xi = B.C.loc[gi], yi = B.C.loc[N + gi], zi = B.C.loc[2 * N + gi];
   const int kmax = max(6, max(D.vnb[0], max(D.vnb[1], D.vnb[2])));
-  int np = 0, nt = 0, r = 1;
+  V3RVerts T;
+  int np = 0, r = 1;
   double r2 = 0.;
   for (int K = 2; K <= kmax && r == 1; ++K) {
-    r = v3_build(B, D, V, s, i, xi, yi, zi, K, C, np, nt, r2);
-    if (r == 0) r = v3_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, C, np, nt, r2);
+    r = v3r_build(B, D, V, s, i, xi, yi, zi, K, C, T, np, r2);
+    if (r == 0) r = v3r_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, C, T, np, r2);
   }
-  if (r != 0 && __lane_id() == 0) {
-    V.femit[gi] = 0;
-    atomicCAS(&B.cnt->err, 0, E_MESH);
-    atomicCAS(&S.err, 0, E_MESH);
+  if (r != 0 && lane == 0) V.femit[gi] = HFV_V3_LEFT;
+}
+
+// The cells that k_v3_cells_reg left.  Grid: HFV_V3_SUB one-wavefront blocks per cell chunk, each looking
+// through HFV_BLOCK / HFV_V3_SUB cells and building those marked, one after another (a block per cell, nearly
+// all of which only look, took 75 us on KH 48^3).
+#define HFV_V3_SUB 8
+__global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V) {
+  __shared__ V3Cell C;
+  const BlockJob J = B.cjobs[blockIdx.x / HFV_V3_SUB];
+  if (J.sim < 0) return;
+  const int s = J.sim;
+  const SimDesc& D = B.sims[s];
+  SimStep& S = B.st[s];
+  if (D.vmesh != 3 || !S.stepping) return;
+  constexpr int CELLS = HFV_BLOCK / HFV_V3_SUB;
+  static_assert(CELLS <= 64, "a lane per cell looked at");
+  const int64_t g0 = (int64_t)J.lo + (blockIdx.x % HFV_V3_SUB) * CELLS;
+  const int lane = __lane_id();
+  const int64_t N = B.C.n, cb = D.cell_base;
+  const int kmax = max(6, max(D.vnb[0], max(D.vnb[1], D.vnb[2])));
+  uint64_t todo = __ballot(lane < CELLS && g0 + lane < J.hi && V.femit[g0 + lane] == HFV_V3_LEFT);
+  for (; todo; todo &= todo - 1) {
+    const int64_t gi = g0 + __builtin_ctzll(todo);
+    const int32_t i = (int32_t)(gi - cb);
+    const double xi = B.C.loc[gi], yi = B.C.loc[N + gi], zi = B.C.loc[2 * N + gi];
+    int np = 0, nt = 0, r = 1;
+    double r2 = 0.;
+    wave_sync();
+    for (int K = 2; K <= kmax && r == 1; ++K) {
+      r = v3_build(B, D, V, s, i, xi, yi, zi, K, C, np, nt, r2);
+      if (r == 0) r = v3_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, C, np, nt, r2);
+    }
+    if (r != 0 && lane == 0) {
+      V.femit[gi] = 0;
+      atomicCAS(&B.cnt->err, 0, E_MESH);
+      atomicCAS(&S.err, 0, E_MESH);
+    }
   }
 }
 
