@@ -1064,22 +1064,29 @@ void prof_next(hfv_ctx* c) {
 template <class T, bool STATIC, int FPT>
 void launch_flux_fpt(hfv_ctx* c, const Batch& B, unsigned g) {
   switch (c->solver) {
+    case HFV_EXACT:
+      hipLaunchKernelGGL((k_flux<T, SOLVER_EXACT, STATIC, FPT>), dim3(g), dim3(BLOCK), 0, c->stream, B);
+      break;
     case HFV_HLLC:
       hipLaunchKernelGGL((k_flux<T, SOLVER_HLLC, STATIC, FPT>), dim3(g), dim3(BLOCK), 0, c->stream, B);
       break;
     case HFV_AIRS:
       hipLaunchKernelGGL((k_flux<T, SOLVER_AIRS, STATIC, FPT>), dim3(g), dim3(BLOCK), 0, c->stream, B);
       break;
-    case HFV_EXACT:
-      hipLaunchKernelGGL((k_flux<T, SOLVER_EXACT, STATIC, FPT>), dim3(g), dim3(BLOCK), 0, c->stream, B);
-      break;
     default:
       hipLaunchKernelGGL((k_flux<T, -1, STATIC, FPT>), dim3(g), dim3(BLOCK), 0, c->stream, B);
   }
 }
+constexpr int64_t kPairGrid = 128;  // face chunks
 template <class T, bool STATIC>
 void launch_flux_ts(hfv_ctx* c, const Batch& B, unsigned g) {
-  if (c->flux_fpt == 4) launch_flux_fpt<T, STATIC, 4>(c, B, g);
+  // The exact solver with two lanes a face (a chunk a block, whatever the launch shape) while a step waits for one
+  // face's chain of pow calls, and not for throughput: face kernel with one lane / two on tubes of 1000 cells 72 / 46
+  // us (FP64, moving) and of 20,000 67 / 54 us (79 chunks), on vortices of 100^2 cells 70 / 69 us (117 chunks), of
+  // 144^2 74 / 84 us (243 chunks) and of 256^2 148 / 214 us.
+  if (c->solver == HFV_EXACT && c->nfg <= kPairGrid)
+    hipLaunchKernelGGL((k_flux_exact<T, STATIC>), dim3((unsigned)c->nfg), dim3(2 * BLOCK), 0, c->stream, B);
+  else if (c->flux_fpt == 4) launch_flux_fpt<T, STATIC, 4>(c, B, g);
   else if (c->flux_fpt == 2) launch_flux_fpt<T, STATIC, 2>(c, B, g);
   else launch_flux_fpt<T, STATIC, 1>(c, B, g);
 }

@@ -1305,7 +1305,8 @@ __device__ __forceinline__ St<T> face_side(const Acc& X, const St<T>& pT, V3<T> 
 // STATIC (fixed mesh, zero particle velocities): the centroid offset and a_over_r come from the face's
 // precomputed line (same expressions, evaluated once by k_geom_faces) and the face velocity is the
 // value the formula yields for v = 0, namely +0 in every component.
-template <class T, int SOLVER, bool DEFER, bool STATIC, class Acc>
+// PAIR: the two lanes of a pair hold the same face (for the exact solver's both_sides).
+template <class T, int SOLVER, bool DEFER, bool STATIC, class Acc, bool PAIR = false>
 __device__ __forceinline__ bool face_flux(const Batch& B, const Cfg& cfg, int64_t f, const Acc& L, const Acc& R,
                                           int32_t r, bool la, bool ra, double* outv, Events& ev) {
   const Faces& F = B.F;
@@ -1425,7 +1426,7 @@ __device__ __forceinline__ bool face_flux(const Batch& B, const Cfg& cfg, int64_
   // ---- Riemann problem in the face frame (the wall problem has no boost: v_face = 0)
   const V3<double> nrm = ld3(F.nrm, nf, f);
   const double area = F.area[f];
-  const St<T> Fl = riemann_flux<T, DEFER>(sc, WL, WR, vfT, cvt3<T>(nrm), g, cfg.gd, ev);
+  const St<T> Fl = riemann_flux<T, DEFER, PAIR>(sc, WL, WR, vfT, cvt3<T>(nrm), g, cfg.gd, ev);
   const St<double> rec = dt * (area * cvtst<double>(Fl));
 #pragma unroll
   for (int k = 0; k < 5; ++k) outv[k] = rec.c[k];
@@ -1633,6 +1634,43 @@ __global__ void __launch_bounds__(HFV_BLOCK, !STATIC || sizeof(T) != 4 ? HFV_FLU
     flux_chunk<T, SOLVER, STATIC>(B, B.fjobs[blockIdx.x + q * gridDim.x]);
     if (q + 1 < FPT) __syncthreads();  // the chunk's LDS is dead before the next chunk stages
   }
+}
+
+// The face kernel of the exact solver: two lanes a face, each evaluating one side's functions of the pressure
+// iteration (both_sides); everything else they compute alike.  The iteration (Newton, then Brent's method from
+// zero) is a chain of some tens of FP64 pow calls, which is what a step of a small exact-solver mesh waits for:
+// on a moving 1000-cell tube the kernel took 72 us with a lane a face (both sides in turn), 46 with two.  Meshes
+// whose faces fill the chip keep k_flux (the launch rule has both sides' times).  Cells are gathered (the same bits
+// as staged).
+template <class T, bool STATIC>
+__global__ void __launch_bounds__(2 * HFV_BLOCK) k_flux_exact(Batch B) {
+  const BlockJob J = B.fjobs[blockIdx.x];
+  if (J.sim < 0) return;
+  const int s = J.sim;
+  if (!B.st[s].stepping || B.sims[s].static_geom != (STATIC ? 1 : 0)) return;
+  const Cfg& cfg = B.sims[s].cfg;
+  const int64_t f = (int64_t)J.lo + (threadIdx.x >> 1);
+  const int64_t fhi = !STATIC && B.sims[s].vmesh ? B.sims[s].face_base + B.eng[s].nf_mesh : J.hi;
+  const bool first = !(threadIdx.x & 1);
+  bool computed = false;
+  Events ev;
+  if (f < J.hi && f < fhi) {
+    const int32_t l = B.F.left[f], r = B.F.right[f];
+    const bool la = B.C.act[l], ra = r >= 0 && B.C.act[r];
+    if (la || ra) {
+      double outv[7];
+      computed = face_flux<T, SOLVER_EXACT, false, STATIC, SoaCell<T>, true>(
+          B, cfg, f, SoaCell<T>(B.C, cfg.gd, B.st[s], l), SoaCell<T>(B.C, cfg.gd, B.st[s], r), r, la, ra, outv, ev);
+      if (first) store_rec(B.F.rec, f, outv, sizeof(T) == 4);
+    }
+  }
+  const int cnt = __syncthreads_count(computed && first);
+  if (threadIdx.x == 0) B.P.face[J.chunk] = (uint32_t)cnt;
+  // one atomic a wave for the Brent calls (most faces of a smooth flow make one)
+  const uint64_t br = __ballot(first && ev.brent);
+  if (br && __lane_id() == 0) atomicAdd(&B.cnt->brent, (unsigned long long)__popcll(br));
+  ev.brent = 0;
+  if (first) flush_events(ev, B.cnt, &B.st[s].err);
 }
 
 // The queued faces of this step with the full AIRS solver (exact fallback), grid-stride.

@@ -387,6 +387,41 @@ __device__ __noinline__ St<T> vacuum_sample(St<T> left, St<T> right, T v_l, T v_
 }
 
 // ------------------------------------------------------------------ exact.rs
+// The solver's functions of a side are evaluated for both sides by one lane, or (PAIR) by a lane each: the two
+// lanes of a pair hold the same face, take the same steps, and each evaluates its own side and receives the
+// other's.  The iteration is a serial chain of FP64 pow calls, so this halves it; the sums are formed in the
+// same order, so the results are the same bits.
+template <class T>
+struct Sides {
+  T l, r;
+};
+__device__ __forceinline__ double pair_other(double v) {  // DPP quad_perm 1, 0, 3, 2
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0xB1, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(lo, lo, 0xB1, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float pair_other(float v) {
+  const int w = __float_as_int(v);
+  return __int_as_float(__builtin_amdgcn_update_dpp(w, w, 0xB1, 0xf, 0xf, false));
+}
+// f(state, sound speed) of both sides
+template <bool PAIR, class T, class Fn>
+__device__ __forceinline__ Sides<T> both_sides(const St<T>& l, const St<T>& r, T a_l, T a_r, Fn&& f) {
+  Sides<T> o;
+  if constexpr (PAIR) {
+    const bool right = __lane_id() & 1;
+    St<T> s;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) s.c[q] = right ? r.c[q] : l.c[q];
+    const T mine = f(s, right ? a_r : a_l), other = pair_other(mine);
+    o.l = right ? other : mine;
+    o.r = right ? mine : other;
+  } else {
+    o.l = f(l, a_l);
+    o.r = f(r, a_r);
+  }
+  return o;
+}
 template <class T>
 __device__ __forceinline__ T ex_fb(T p, const St<T>& s, T a, const Gas<T>& g) {
   if (p > s.c[4]) {
@@ -396,9 +431,10 @@ __device__ __forceinline__ T ex_fb(T p, const St<T>& s, T a, const Gas<T>& g) {
   }
   return g.tdgm1 * a * (hpow(p / s.c[4], g.gm1d2g) - T(1));
 }
-template <class T>
+template <bool PAIR, class T>
 __device__ __forceinline__ T ex_f(T p, const St<T>& l, const St<T>& r, T v_l, T v_r, T a_l, T a_r, const Gas<T>& g) {
-  return ex_fb(p, l, a_l, g) + ex_fb(p, r, a_r, g) + (v_r - v_l);
+  const Sides<T> f = both_sides<PAIR>(l, r, a_l, a_r, [&](const St<T>& s, T a) { return ex_fb(p, s, a, g); });
+  return f.l + f.r + (v_r - v_l);
 }
 // exact.rs:37-45 (rarefaction branch exponent -(gamma-1)/(2 gamma), as in the reference)
 template <class T>
@@ -416,7 +452,7 @@ __device__ __forceinline__ T ex_gb(T p, const St<T>& s, const Gas<T>& g) {
   T cap_b = g.gm1dgp1 * s.c[4];
   return hsqrt(cap_a / (p + cap_b));
 }
-template <class T>
+template <bool PAIR, class T>
 __device__ __forceinline__ T ex_guess_p(const St<T>& l, const St<T>& r, T v_l, T v_r, T a_l, T a_r, const Gas<T>& g) {
   T p_min = hmin(l.c[4], r.c[4]);
   T p_max = hmax(l.c[4], r.c[4]);
@@ -427,15 +463,17 @@ __device__ __forceinline__ T ex_guess_p(const St<T>& l, const St<T>& r, T v_l, T
   if (q_max <= T(2) && p_min <= ppv && ppv <= p_max) {
     p_guess = ppv;
   } else if (ppv < p_min) {
-    T base = (a_l + a_r - g.half_gm1 * (v_r - v_l)) / (a_l / hpow(l.c[4], g.gm1d2g) + a_r / hpow(r.c[4], g.gm1d2g));
+    const Sides<T> d = both_sides<PAIR>(l, r, a_l, a_r, [&](const St<T>& s, T a) { return a / hpow(s.c[4], g.gm1d2g); });
+    T base = (a_l + a_r - g.half_gm1 * (v_r - v_l)) / (d.l + d.r);
     p_guess = hpow(base, g.gamma_tdgm1);
   } else {
-    T gl = ex_gb(ppv, l, g), gr = ex_gb(ppv, r, g);
+    const Sides<T> b = both_sides<PAIR>(l, r, a_l, a_r, [&](const St<T>& s, T) { return ex_gb(ppv, s, g); });
+    T gl = b.l, gr = b.r;
     p_guess = (gl * l.c[4] + gr * r.c[4] - v_r + v_l) / (gl + gr);
   }
   return hmax(p_guess, T(1e-8));
 }
-template <class T>
+template <bool PAIR, class T>
 __device__ __noinline__ T ex_solve_brent(T lower, T upper, T low_f, T up_f, T tol, St<T> l, St<T> r, T v_l, T v_r,
                                          T a_l, T a_r, const Gas<T>& g, Events& ev) {
   T a = lower, b = upper, c, d = T(INFINITY);
@@ -468,7 +506,7 @@ __device__ __noinline__ T ex_solve_brent(T lower, T upper, T low_f, T up_f, T to
     } else {
       mflag = false;
     }
-    fs = ex_f(s, l, r, v_l, v_r, a_l, a_r, g);
+    fs = ex_f<PAIR>(s, l, r, v_l, v_r, a_l, a_r, g);
     d = c;
     c = b;
     fc = fb;
@@ -498,31 +536,34 @@ __device__ __forceinline__ T middle_density(T p, const St<T>& s, const Gas<T>& g
   if (pdps > T(1)) return s.c[0] * (pdps + g.gm1dgp1) / (g.gm1dgp1 * pdps + T(1));
   return s.c[0] * hpow(pdps, g.one_over_gamma);
 }
-template <class T>
+template <bool PAIR, class T>
 __device__ __forceinline__ Star<T> star_from_pstar(T pstar, const St<T>& l, const St<T>& r, T v_l, T v_r, T a_l,
                                                    T a_r, const Gas<T>& g) {
   Star<T> sv;
-  sv.u = T(0.5) * (v_l + v_r) + T(0.5) * (ex_fb(pstar, r, a_r, g) - ex_fb(pstar, l, a_l, g));
-  sv.rho_l = middle_density(pstar, l, g);
-  sv.rho_r = middle_density(pstar, r, g);
+  const Sides<T> f = both_sides<PAIR>(l, r, a_l, a_r, [&](const St<T>& s, T a) { return ex_fb(pstar, s, a, g); });
+  const Sides<T> m = both_sides<PAIR>(l, r, a_l, a_r, [&](const St<T>& s, T) { return middle_density(pstar, s, g); });
+  sv.u = T(0.5) * (v_l + v_r) + T(0.5) * (f.r - f.l);
+  sv.rho_l = m.l;
+  sv.rho_r = m.r;
   sv.p = pstar;
   return sv;
 }
 // exact.rs:242-290
-template <class T>
+template <bool PAIR, class T>
 __device__ __noinline__ Star<T> exact_star(St<T> l, St<T> r, T v_l, T v_r, T a_l, T a_r, const Gas<T>& g,
                                            Events& ev) {
   T p = T(0);
-  T p_guess = ex_guess_p(l, r, v_l, v_r, a_l, a_r, g);
-  T fp = ex_f(p, l, r, v_l, v_r, a_l, a_r, g);
-  T fp_guess = ex_f(p_guess, l, r, v_l, v_r, a_l, a_r, g);
+  T p_guess = ex_guess_p<PAIR>(l, r, v_l, v_r, a_l, a_r, g);
+  T fp = ex_f<PAIR>(p, l, r, v_l, v_r, a_l, a_r, g);
+  T fp_guess = ex_f<PAIR>(p_guess, l, r, v_l, v_r, a_l, a_r, g);
   if (fp * fp_guess >= T(0)) {
     int counter = 0;
     while (habs(p - p_guess) > T(1e-6) * T(0.5) * (p + p_guess) && fp_guess < T(0)) {
       p = p_guess;
-      T fpr = ex_fprimeb(p_guess, l, a_l, g) + ex_fprimeb(p_guess, r, a_r, g);
+      const Sides<T> d = both_sides<PAIR>(l, r, a_l, a_r, [&](const St<T>& s, T a) { return ex_fprimeb(p_guess, s, a, g); });
+      T fpr = d.l + d.r;
       p_guess = p_guess - fp_guess / fpr;
-      fp_guess = ex_f(p_guess, l, r, v_l, v_r, a_l, a_r, g);
+      fp_guess = ex_f<PAIR>(p_guess, l, r, v_l, v_r, a_l, a_r, g);
       counter += 1;
       if (counter > 1000) {
         ev.fail(E_NEWTON);
@@ -532,13 +573,13 @@ __device__ __noinline__ Star<T> exact_star(St<T> l, St<T> r, T v_l, T v_r, T a_l
   }
   if (habs(p - p_guess) > T(1e-6) * T(0.5) * (p + p_guess) && fp_guess > T(0)) {
     p = T(0);
-    fp = ex_f(p, l, r, v_l, v_r, a_l, a_r, g);
+    fp = ex_f<PAIR>(p, l, r, v_l, v_r, a_l, a_r, g);
     ev.brent++;
-    p = ex_solve_brent(p, p_guess, fp, fp_guess, T(1e-6), l, r, v_l, v_r, a_l, a_r, g, ev);
+    p = ex_solve_brent<PAIR>(p, p_guess, fp, fp_guess, T(1e-6), l, r, v_l, v_r, a_l, a_r, g, ev);
   } else {
     p = p_guess;
   }
-  return star_from_pstar(p, l, r, v_l, v_r, a_l, a_r, g);
+  return star_from_pstar<PAIR>(p, l, r, v_l, v_r, a_l, a_r, g);
 }
 
 // ------------------------------------------------------------------ pvrs.rs / tsrs.rs / trrs.rs
@@ -565,7 +606,7 @@ __device__ __forceinline__ Star<T> tsrs_star(const St<T>& l, const St<T>& r, T v
   T g_l = hsqrt((g.tdgp1 / l.c[0]) / (p_guess + g.gm1dgp1 * l.c[4]));
   T g_r = hsqrt((g.tdgp1 / r.c[0]) / (p_guess + g.gm1dgp1 * r.c[4]));
   T pstar = (g_l * l.c[4] + g_r * r.c[4] - (v_r - v_l)) / (g_l + g_r);
-  return star_from_pstar(pstar, l, r, v_l, v_r, a_l, a_r, g);
+  return star_from_pstar<false>(pstar, l, r, v_l, v_r, a_l, a_r, g);
 }
 template <class T>
 __device__ __forceinline__ Star<T> trrs_star(const St<T>& l, const St<T>& r, T v_l, T v_r, T a_l, T a_r,
@@ -574,7 +615,7 @@ __device__ __forceinline__ Star<T> trrs_star(const St<T>& l, const St<T>& r, T v
   T num = a_l + a_r - g.half_gm1 * (v_r - v_l);
   T denom = a_l * hpow(l.c[4], -beta) + a_r * hpow(r.c[4], -beta);
   T pstar = hpow(num / denom, T(1) / beta);
-  return star_from_pstar(pstar, l, r, v_l, v_r, a_l, a_r, g);
+  return star_from_pstar<false>(pstar, l, r, v_l, v_r, a_l, a_r, g);
 }
 
 // ------------------------------------------------------------------ hllc.rs
@@ -603,7 +644,7 @@ struct SolverCfg {
 };
 
 // FP64 star state for any star solver (exact/PVRS/AIRS/TSRS/TRRS).
-template <class T>
+template <bool PAIR, class T>
 __device__ __forceinline__ Star<T> star_for(int kind, double threshold, const St<T>& l, const St<T>& r, T v_l, T v_r,
                                             T a_l, T a_r, const Gas<T>& g, Events& ev) {
   switch (kind) {
@@ -614,14 +655,14 @@ __device__ __forceinline__ Star<T> star_for(int kind, double threshold, const St
       T p_max = hmax(l.c[4], r.c[4]);
       T p_min = hmin(l.c[4], r.c[4]);
       if (fdiv(p_max, p_min) < (T)threshold) return st;
-      return exact_star(l, r, v_l, v_r, a_l, a_r, g, ev);
+      return exact_star<PAIR>(l, r, v_l, v_r, a_l, a_r, g, ev);
     }
     case SOLVER_TSRS:
       return tsrs_star(l, r, v_l, v_r, a_l, a_r, g);
     case SOLVER_TRRS:
       return trrs_star(l, r, v_l, v_r, a_l, a_r, g);
     default:
-      return exact_star(l, r, v_l, v_r, a_l, a_r, g, ev);
+      return exact_star<PAIR>(l, r, v_l, v_r, a_l, a_r, g, ev);
   }
 }
 
@@ -630,7 +671,8 @@ __device__ __forceinline__ Star<T> star_for(int kind, double threshold, const St
 // DEFER (AIRS only): a face whose pressure ratio calls for the exact solver is not solved here
 // (ev.deferred is set); the caller hands it to a separate pass, so that this code path carries no
 // exact-solver registers.
-template <class T, bool DEFER = false>
+// PAIR: the two lanes of a pair hold the same face (both_sides).
+template <class T, bool DEFER = false, bool PAIR = false>
 __device__ __forceinline__ St<T> riemann_flux(const SolverCfg& sc, const St<T>& left, const St<T>& right, V3<T> iv, V3<T> n,
                               const Gas<T>& g, const Gas<double>& gd, Events& ev) {
   if (sc.kind == SOLVER_LINADV) {  // linear_advection.rs:17-33
@@ -700,13 +742,13 @@ __device__ __forceinline__ St<T> riemann_flux(const SolverCfg& sc, const St<T>& 
                                                    (T)sc.threshold)));
     if (need_fp64) {
       St<double> ld = cvtst<double>(left), rd = cvtst<double>(right);
-      Star<double> sd = exact_star(ld, rd, (double)v_l, (double)v_r, (double)a_l, (double)a_r, gd, ev);
+      Star<double> sd = exact_star<PAIR>(ld, rd, (double)v_l, (double)v_r, (double)a_l, (double)a_r, gd, ev);
       star.rho_l = (T)sd.rho_l;
       star.rho_r = (T)sd.rho_r;
       star.u = (T)sd.u;
       star.p = (T)sd.p;
     } else {
-      star = star_for(sc.kind, sc.threshold, left, right, v_l, v_r, a_l, a_r, g, ev);
+      star = star_for<PAIR>(sc.kind, sc.threshold, left, right, v_l, v_r, a_l, a_r, g, ev);
     }
     w = sample_from_star(star, left, right, v_l, v_r, a_l, a_r, n, g);
   }
