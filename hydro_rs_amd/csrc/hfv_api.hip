@@ -963,7 +963,8 @@ int reset_slot(hfv_ctx* c, int s) {
   HIP_OK(hipMemsetAsync(C.nbin + cb, HFV_NO_BIN, cap, st));
   HIP_OK(hipMemsetAsync(c->dst + s, 0, sizeof(SimStep), st));
   HIP_OK(hipMemsetAsync(C.act + cb, 0, cap, st));
-  (void)n;
+  if (n > 0)  // the new mesh's centroids (a step of a fixed mesh renews the primitives only)
+    hipLaunchKernelGGL(k_pack_pc, dim3(grid_full(n)), dim3(BLOCK), 0, st, c->batch_args(), cb, cb + n);
   c->v_zero[s] = 1;
   c->fr_dirty = true;
   c->heng[s] = fresh_engine(c->params[s]);
