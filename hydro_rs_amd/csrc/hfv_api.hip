@@ -944,27 +944,11 @@ int upload_mesh(hfv_ctx* c, int s, const hfv_mesh_arrays* m, const uint8_t* upda
 // Reset a slot's per-cell state (Particle::default) and its engine; set the cell -> slot map.
 int reset_slot(hfv_ctx* c, int s) {
   hipStream_t st = c->stream;
-  const int64_t N = c->n, cb = c->cbase[s], cap = icap(c, s), n = c->nused[s];
-  Cells& C = c->C;
-  struct {
-    double* p;
-    int w;
-  } fl[] = {{C.prim, 5}, {C.gc, 3}, {C.cons, 5}, {C.facc, 5}, {C.loc, 3}, {C.v, 3},
-            {C.vrel, 3}, {C.maor, 1}, {C.msv, 1}, {C.dt, 1}};
-  for (auto& f : fl)
-    for (int k = 0; k < f.w; ++k) HIP_OK(hipMemsetAsync(f.p + k * N + cb, 0, sizeof(double) * cap, st));
-  // extrapolations and kept rates: doubles, or floats in FP32-flux contexts (one precision per batch)
-  const size_t es = c->params[s].precision == HFV_FP32_FLUX ? sizeof(float) : sizeof(double);
-  HIP_OK(hipMemsetAsync((char*)C.extrap + es * HFV_EX_W * cb, 0, es * HFV_EX_W * cap, st));
-  for (int k = 0; k < 5; ++k) HIP_OK(hipMemsetAsync((char*)C.tex + es * (k * N + cb), 0, es * cap, st));
-  for (int k = 0; k < 15; ++k) HIP_OK(hipMemsetAsync((char*)C.grad + es * (k * N + cb), 0, es * cap, st));
-  HIP_OK(hipMemsetAsync(C.tiex + cb, 0, sizeof(uint64_t) * cap, st));  // = the fresh engine's ti_pred
-  HIP_OK(hipMemsetAsync(C.bin + cb, 0, cap, st));
-  HIP_OK(hipMemsetAsync(C.nbin + cb, HFV_NO_BIN, cap, st));
+  const int64_t cb = c->cbase[s], cap = icap(c, s), n = c->nused[s];
   HIP_OK(hipMemsetAsync(c->dst + s, 0, sizeof(SimStep), st));
-  HIP_OK(hipMemsetAsync(C.act + cb, 0, cap, st));
-  if (n > 0)  // the new mesh's centroids (a step of a fixed mesh renews the primitives only)
-    hipLaunchKernelGGL(k_pack_pc, dim3(grid_full(n)), dim3(BLOCK), 0, st, c->batch_args(), cb, cb + n);
+  hipLaunchKernelGGL(k_reset, dim3(grid_full(cap)), dim3(BLOCK), 0, st, c->batch_args(), cb, cb + n, cb + cap,
+                     c->params[s].precision == HFV_FP32_FLUX ? 1 : 0);
+  HIP_OK(hipGetLastError());
   c->v_zero[s] = 1;
   c->fr_dirty = true;
   c->heng[s] = fresh_engine(c->params[s]);

@@ -1907,6 +1907,40 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_pack_pc(Batch B, int64_t lo, int6
   store_pc(B.C.pc, i, ld5(B.C.prim, B.C.n, i), ld3(B.C.cen, B.C.n, i));
 }
 
+// The default particle (Particle::default) in the cells [lo, hi) of a slot, of which those below `used` have a
+// mesh: their pc lines get its centroids (a step of a fixed mesh renews the primitives only).  One launch: as a
+// clearing of each field and component it was 43, 10 us apart, which twelve small jobs that a server admits
+// together waited for (5.7 of 37 ms).
+__global__ void __launch_bounds__(HFV_BLOCK) k_reset(Batch B, int64_t lo, int64_t used, int64_t hi, int f32) {
+  const int64_t i = lo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= hi) return;
+  const Cells& C = B.C;
+  const int64_t n = C.n;
+  const V3<double> zero = mk3(0., 0., 0.);
+  st5(C.prim, n, i, vacuum<double>());
+  st5(C.cons, n, i, vacuum<double>());
+  st5(C.facc, n, i, vacuum<double>());
+  st3(C.gc, n, i, zero);
+  st3(C.loc, n, i, zero);
+  st3(C.v, n, i, zero);
+  st3(C.vrel, n, i, zero);
+  C.maor[i] = 0.;
+  C.msv[i] = 0.;
+  C.dt[i] = 0.;
+  Gr<double> g;
+#pragma unroll
+  for (int q = 0; q < 5; ++q) g.g[q] = zero;
+  // doubles, or floats in FP32-flux contexts (one precision per batch)
+  st_grad(C, i, f32 != 0, g);
+  st_ex(C, i, f32 != 0, vacuum<double>());
+  st_tex(C, i, f32 != 0, vacuum<double>());
+  C.tiex[i] = 0;  // = the fresh engine's ti_pred
+  C.bin[i] = 0;
+  C.nbin[i] = HFV_NO_BIN;
+  C.act[i] = 0;
+  if (i < used) store_pc(C.pc, i, vacuum<double>(), ld3(C.cen, n, i));
+}
+
 // The time-extrapolation rates of every loaded simulation's cells, and the flux records of the staged
 // ones, from the SoA fields (after the host changed the state or the mesh, or a phase call changed
 // fields on its own).
