@@ -527,6 +527,8 @@ int alloc_batch(hfv_ctx* c) {
   }
   F.nse = nse;
   F.soff = dalloc<int64_t>(c, 4 * ncc);
+  F.seconn = dalloc<int32_t>(c, nse);
+  F.senbr = dalloc<int32_t>(c, nse);
   F.seref = dalloc<int32_t>(c, nse);
   F.secode = dalloc<uint8_t>(c, nse);
   F.sew = dalloc<double>(c, nse);
