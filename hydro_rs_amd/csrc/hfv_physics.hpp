@@ -310,34 +310,41 @@ template <class T>
 __device__ __forceinline__ St<T> sample_middle_state(T rho, T u, T p, const St<T>& s, T v, V3<T> n) {
   return mkst(rho, vel(s) + ((u - v) * n), p);
 }
+// |v| < |a| y with room for every rounding, for a factor y that is known to be at least num / den: the sign of
+// v - a y is then the sign of -a, and y need not be evaluated.  The factors are roots and powers whose computed
+// values are a few ulp (below 1e-6, FP32) off; the band is 1e-4.  NaN, zero and extreme operands are not certain.
+template <class T>
+__device__ __host__ __forceinline__ bool surely_below(T v, T a, T num, T den) {
+  const T lim = habs(a) * num, x = habs(v) * den;
+  return x < T(0.9999) * lim && lim > T(1e-30) && lim < T(1e30) && x < T(1e30);
+}
+// The state at x/t = 0.  The wave's faces have their contact on either side of it, so the side is chosen first
+// and one copy of the tests runs for both (a = a_l on the left, -a_r on the right: the same expressions, ahead and
+// behind the ones of each side).  Where the flow is subsonic with respect to the wave, as most of it is, the signs
+// of a shock's speed (its root is >= 1, as star.p > p) and of a rarefaction's tail (its power is >= star.p / p, as
+// star.p <= p and the exponent is below 1) are known without the root, the division and the FP32 or FP64 pow.
+// The kernel is bound by the instructions it issues: face kernel with AIRS on KH 128^3 (FP32 flux) 603 -> 542 us, on
+// KH 96^3 (FP64) 402 -> 352; exact solver on a moving 1000-cell tube 47.4 -> 45 us.
 template <class T>
 __device__ __forceinline__ St<T> sample_from_star(const Star<T>& star, const St<T>& left, const St<T>& right, T v_l,
                                                T v_r, T a_l, T a_r, V3<T> n, const Gas<T>& g) {
-  if (star.u < T(0)) {
-    if (star.p > right.c[4]) {  // right shock
-      if (shock_speed(v_r, -a_r, fdiv(star.p, right.c[4]), g) > T(0))
-        return sample_middle_state(star.rho_r, star.u, star.p, right, v_r, n);
-      return right;
+  const bool rt = star.u < T(0);
+  St<T> s;
+#pragma unroll
+  for (int q = 0; q < 5; ++q) s.c[q] = rt ? right.c[q] : left.c[q];
+  const T v = rt ? v_r : v_l, a = rt ? -a_r : a_l, rho = rt ? star.rho_r : star.rho_l;
+  auto ahead = [&](T x) { return rt ? x > T(0) : x < T(0); };  // moving away from the contact
+  bool middle;
+  if (star.p > s.c[4]) {  // shock
+    middle = surely_below(v, a, T(1), T(1)) || ahead(shock_speed(v, a, fdiv(star.p, s.c[4]), g));
+  } else {  // rarefaction
+    middle = ahead(v - a);  // its head
+    if (middle && !surely_below(star.u, a, star.p, s.c[4])) {
+      const T tail = tail_speed_for_sign(star.u, a, fdiv(star.p, s.c[4]), g);
+      if (rt ? tail < T(0) : tail > T(0)) return sample_rarefaction_fan(s, a, v, n, g);
     }
-    // right rarefaction
-    if (v_r - (-a_r) > T(0)) {
-      if (tail_speed_for_sign(star.u, -a_r, fdiv(star.p, right.c[4]), g) < T(0))
-        return sample_rarefaction_fan(right, -a_r, v_r, n, g);
-      return sample_middle_state(star.rho_r, star.u, star.p, right, v_r, n);
-    }
-    return right;
-  } else if (star.p > left.c[4]) {  // left shock
-    if (shock_speed(v_l, a_l, fdiv(star.p, left.c[4]), g) < T(0))
-      return sample_middle_state(star.rho_l, star.u, star.p, left, v_l, n);
-    return left;
   }
-  // left rarefaction
-  if (v_l - a_l < T(0)) {
-    if (tail_speed_for_sign(star.u, a_l, fdiv(star.p, left.c[4]), g) > T(0))
-      return sample_rarefaction_fan(left, a_l, v_l, n, g);
-    return sample_middle_state(star.rho_l, star.u, star.p, left, v_l, n);
-  }
-  return left;
+  return middle ? sample_middle_state(rho, star.u, star.p, s, v, n) : s;
 }
 
 // ------------------------------------------------------------------ vacuum.rs
