@@ -591,7 +591,7 @@ constexpr bool flux_stages() {
 // Minimum resident blocks per CU (of 4 waves, one per SIMD) the compiler must fit the flux / gradient
 // kernels into (0: its choice).  Static-geometry FP32 flux: 6, where the one-chunk variants fit 6 waves
 // per SIMD (76-78 VGPRs, no spills): 3D FP32 flux -10% against 5 waves (96 VGPRs), which was itself 12%
-// faster than the compiler's choice; 7 for its AIRS variants (72 VGPRs, 12 spilled on cold paths): 3D
+// faster than the compiler's choice; 7 for its AIRS variants (72 VGPRs, 17 spilled on cold paths): 3D
 // FP32 AIRS flux -6% more, where the 1D HLLC flux of the ensemble lost 0.4% at 7.  The others: 5, which
 // the per-step-geometry variants meet (93-96 VGPRs; at 6 they spill more); the staged FP64 ones keep 4
 // (their LDS allows no more).
