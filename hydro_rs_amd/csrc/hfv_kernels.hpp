@@ -592,9 +592,10 @@ constexpr bool flux_stages() {
 // kernels into (0: its choice).  Static-geometry FP32 flux: 6, where the one-chunk variants fit 6 waves
 // per SIMD (76-78 VGPRs, no spills): 3D FP32 flux -10% against 5 waves (96 VGPRs), which was itself 12%
 // faster than the compiler's choice; 7 for its AIRS variants (72 VGPRs, 17 spilled on cold paths): 3D
-// FP32 AIRS flux -6% more, where the 1D HLLC flux of the ensemble lost 0.4% at 7.  The others: 5, which
-// the per-step-geometry variants meet (93-96 VGPRs; at 6 they spill more); the staged FP64 ones keep 4
-// (their LDS allows no more).
+// FP32 AIRS flux -6% more, where the 1D HLLC flux of the ensemble lost 0.4% at 7.  The others: 4, which
+// the staged FP64 ones' LDS sets anyway; the per-step-geometry ones at 5 (96 VGPRs) spilled 40 to 250 registers
+// in the loop of every face: KH 48^3 steered (AIRS, FP64) 85.5 -> 68.3 us, 125^2 steered vortex (HLLC, FP32 flux)
+// 13.3 -> 11.7.
 #ifndef HFV_FLUX_WAVES_F32
 #define HFV_FLUX_WAVES_F32 6
 #endif
@@ -602,7 +603,7 @@ constexpr bool flux_stages() {
 #define HFV_FLUX_WAVES_F32_AIRS 7
 #endif
 #ifndef HFV_FLUX_WAVES
-#define HFV_FLUX_WAVES 5
+#define HFV_FLUX_WAVES 4
 #endif
 // CSR entries of a cell whose loads the per-step-geometry gradient sweeps issue together: 4 against a
 // two-entry software pipeline, KH 128^3 gradient phase -8% (FP64) / -9% (FP32 flux), ensemble -5%; 8
