@@ -1553,6 +1553,7 @@ int hfv_compute_fluxes(hfv_ctx* c, const hfv_timestep_info* info) {
   TRY(begin_phase_step(c, info, false));
   Batch B = c->batch_args();
   launch_mask(c, B, 2);
+  hipLaunchKernelGGL(k_step_taken, dim3(1), dim3(1), 0, c->stream, B, 0);
   c->fr_dirty = true;
   pack_fr_if_dirty(c);
   launch_flux(c, B);

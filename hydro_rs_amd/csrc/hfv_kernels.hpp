@@ -736,6 +736,13 @@ __device__ __forceinline__ SimStep step_begin(const SimEngine& E) {
   return S;
 }
 
+// The request of a trait-level step (begin_phase_step) is in the SimStep once its mask has run.  Where the step's
+// end is another call's, or none's, it leaves the engine here, so that the next step is what that call asks for.
+__global__ void k_step_taken(Batch B, int s) {
+  B.eng[s].force = 0;
+  B.eng[s].no_pred = 0;
+}
+
 // Engine::step / queue_step / update_ti_next (engine.rs:194-268) of simulation s by one block: sums the chunk
 // partials of this step (eight loads in flight per thread), then one thread moves the engine to its next
 // sync point.  phase: a trait-level call, which ends the step whether or not it has been ended.
