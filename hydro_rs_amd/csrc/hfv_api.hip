@@ -189,6 +189,7 @@ struct hfv_ctx {
   int64_t ncg = 8, nfg = 8, live_chunks = 0;
   int cgsh = 0, fgsh = 0;     // log2 of the group sizes that the tables were dealt in
   int64_t face_items = 0;     // faces that the only simulation's face kernels cover
+  int v3sub = 0;              // log2 of k_v3_cells' blocks per cell chunk
   std::vector<BlockJob> hcjobs, hfjobs;
   BlockJob *dcjobs = nullptr, *dfjobs = nullptr;
   Partials P{};
@@ -369,15 +370,24 @@ int64_t grid_position(int64_t j, int64_t g) { return 8 * ((j / g / 8) * g + j % 
 // face count (the faces past the current mesh have no cells and are skipped).
 int64_t face_range(const hfv_ctx* c, int s) { return c->desc[s].vmesh ? c->fcap[s] : c->fused[s]; }
 
+// log2 of the blocks per cell chunk that k_v3_cells launches for `chunks` chunks of 3D moving meshes: together some
+// 4096, a few more than the chip holds at once (10 a CU by LDS), as long as a block stays at 2 cells or more.
+int v3_sub(int64_t chunks) {
+  int sub = 0;
+  while (sub < 7 && chunks << (sub + 1) <= 4096) ++sub;
+  return sub;
+}
+
 // Rebuild the block tables from the live slots (loaded, and in a batch not finished: a finished slot's
 // blocks would only exit) and upload them with the simulation descriptors.  Chunk ids (partials) stay
 // global.
 int write_jobs(hfv_ctx* c) {
   const int S = c->nslots;
   auto live = [&](int s) { return c->loaded[s] && !(c->batch && c->heng[s].done); };
-  int64_t lc = 0, lf = 0;
+  int64_t lc = 0, lf = 0, l3 = 0;  // (l3: of 3D moving meshes)
   for (int s = 0; s < S; ++s) {
     if (!live(s)) continue;
+    if (c->desc[s].vmesh == 3) l3 += (c->nused[s] + BLOCK - 1) / BLOCK;
     lc += (c->nused[s] + BLOCK - 1) / BLOCK;
     lf += (face_range(c, s) + BLOCK - 1) / BLOCK;
   }
@@ -387,6 +397,9 @@ int write_jobs(hfv_ctx* c) {
   const int cgsh = __builtin_ctzll((uint64_t)gc), fgsh = __builtin_ctzll((uint64_t)gf);
   const int64_t items = c->batch || !c->loaded[0] ? 0 : face_range(c, 0);
   if (cgsh != c->cgsh || fgsh != c->fgsh || items != c->face_items) drop_graph(c);
+  const int v3sub = v3_sub(l3);
+  if (v3sub != c->v3sub) drop_graph(c);
+  c->v3sub = v3sub;
   c->cgsh = cgsh;
   c->fgsh = fgsh;
   c->face_items = items;
@@ -1151,7 +1164,7 @@ void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
     if (c->any_vmesh2) hipLaunchKernelGGL(k_v2_cells, dim3((unsigned)(c->ncg * HFV_V2_SUB)), gb, 0, st, B, V);
     if (c->any_vmesh3) {
       hipLaunchKernelGGL(k_v3_cells_reg, dim3((unsigned)(c->ncg * HFV_V3R_SUB)), dim3(256), 0, st, B, V);
-      hipLaunchKernelGGL(k_v3_cells, dim3((unsigned)(c->ncg * HFV_V3_SUB)), dim3(64), 0, st, B, V);
+      hipLaunchKernelGGL(k_v3_cells, dim3((unsigned)(c->ncg << c->v3sub)), dim3(64), 0, st, B, V, c->v3sub);
     }
     hipLaunchKernelGGL(k_v2_faces, gc, gb, 0, st, B, V);
     hipLaunchKernelGGL(k_v2_sum<1>, gc, gb, 0, st, B, V);

@@ -192,6 +192,7 @@ struct SimStep {
   int n_down;    // 1D periodic moving meshes: faces of this step's rebuild where the generator order steps down
   int nf_tmp;    // 2D/3D moving meshes: the rebuild's provisional faces beyond their chunks' shares
   int n_over;    // 2D/3D moving meshes: CSR entries beyond their cells' buckets in this step's rebuild
+  int n_left;    // 3D moving meshes: cells that the register builder left in this step's rebuild
 };
 
 // Batch-global counters (soft events; the first hard error of any simulation).
@@ -717,6 +718,7 @@ __device__ __forceinline__ SimStep step_begin(const SimEngine& E) {
   S.n_down = 0;
   S.nf_tmp = 0;
   S.n_over = 0;
+  S.n_left = 0;
   if (E.err) {  // a hard error stops this simulation only; the batch's other simulations go on
     S.done = 1;
   } else if (E.force) {  // hfv_step: a step at ti_current with the caller's ti_old
@@ -957,7 +959,7 @@ struct V2Over {
 struct V2Bufs {
   int32_t* gcnt;   // [N + S + 1], simulation s at cell_base + s: bin counts, then bin starts (nbins + 1); zero
                    // between the steps
-  int32_t* gfill;  // same layout: placement cursors
+  int32_t* gfill;  // same layout: placement cursors, then (3D) the list of the cells the register builder left
   int32_t* gord;   // [N] at cell_base: local cell indices grouped by bin
   int32_t* gkey;   // [N] bin of each cell
   int32_t* femit;  // [N] faces a cell emits
@@ -1028,6 +1030,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_mask(Batch B, V2Bufs V, int mode)
       G.n_down = S.n_down;
       G.nf_tmp = S.nf_tmp;
       G.n_over = S.n_over;
+      G.n_left = S.n_left;
     }
     if (!S.stepping) return;
   }

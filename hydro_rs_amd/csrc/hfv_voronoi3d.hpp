@@ -318,8 +318,9 @@ __device__ __forceinline__ int32_t v3_code_of(int32_t kk) {
 
 // this lane's bins of the (2K+1)^3 block (every 64th): f(bin key, shift codes, whether it is the
 // generator's own bin unshifted)
-template <class Fn>
-__device__ __forceinline__ void v3_lane_bins(const SimDesc& D, double xi, double yi, double zi, int K, Fn&& f) {
+template <bool NEAR = false, class Fn>
+__device__ __forceinline__ void v3_lane_bins(const SimDesc& D, double xi, double yi, double zi, int K, Fn&& f,
+                                             double near2 = 0.) {
   const int lane = __lane_id();
   const bool per = D.periodic != 0;
   const int bi[3] = {v2_bin(xi, D.vw[0], D.vnb[0]), v2_bin(yi, D.vw[1], D.vnb[1]), v2_bin(zi, D.vw[2], D.vnb[2])};
@@ -347,37 +348,62 @@ __device__ __forceinline__ void v3_lane_bins(const SimDesc& D, double xi, double
         }
       }
     }
+    if (NEAR) {
+      const double x[3] = {xi, yi, zi};
+      double d2 = 0.;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const double edge = (double)(bi[a] + dd[a] + (dd[a] < 0 ? 1 : 0)) * D.vw[a];
+        const double d = fmax((dd[a] > 0 ? edge - x[a] : x[a] - edge) - 1e-6 * D.vw[a], 0.);
+        d2 += dd[a] == 0 ? 0. : d * d;
+      }
+      skip = skip || d2 >= near2;
+    }
     if (skip) continue;
     f((b[0] * D.vnb[1] + b[1]) * D.vnb[2] + b[2], sc[0], sc[1], sc[2], dd[0] == 0 && dd[1] == 0 && dd[2] == 0);
   }
 }
 
-// this lane's candidates of the (2K+1)^3 block: f(cand) for each
-template <class Fn>
+// this lane's candidates of the (2K+1)^3 block, NEAR: of its bins closer than sqrt(near2): f(cand) for each, in order,
+// four candidates' loads in flight (a dense bin is one lane's chain)
+template <bool NEAR = false, class Fn>
 __device__ __forceinline__ void v3_lane_candidates(const Batch& B, const SimDesc& D, const V2Bufs& V, int s, int32_t i,
-                                                   double xi, double yi, double zi, int K, Fn&& f) {
+                                                   double xi, double yi, double zi, int K, Fn&& f, double near2 = 0.) {
   const int64_t N = B.C.n, cb = D.cell_base;
   const double* L = B.C.loc;
   const int32_t* gst = V.gcnt + cb + s;
   const int32_t* gord = V.gord + cb;
-  v3_lane_bins(D, xi, yi, zi, K, [&](int key, int s0, int s1, int s2, bool) {
+  v3_lane_bins<NEAR>(D, xi, yi, zi, K, [&](int key, int s0, int s1, int s2, bool) {
     const int32_t kk = ((s0 & 0xFF) << 16) | ((s1 & 0xFF) << 8) | (s2 & 0xFF);  // the host's memcmp order
     const int32_t code = v3_code_of(kk);
-    for (int32_t q = gst[key]; q < gst[key + 1]; ++q) {
-      const int32_t j = gord[q];
-      if (j == i && s0 == 0 && s1 == 0 && s2 == 0) continue;
-      const int64_t gj = cb + j;
-      V3Cand c;
-      c.rx = (L[gj] + (double)s0 * D.cfg.box[0]) - xi;
-      c.ry = (L[N + gj] + (double)s1 * D.cfg.box[1]) - yi;
-      c.rz = (L[2 * N + gj] + (double)s2 * D.cfg.box[2]) - zi;
-      c.d2 = v3dot(c.rx, c.ry, c.rz, c.rx, c.ry, c.rz);
-      c.j = j;
-      c.k = kk;
-      c.code = code;
-      f(c);
+    const int32_t g0 = gst[key], g1 = gst[key + 1];
+    for (int32_t q0 = g0; q0 < g1; q0 += 4) {
+      int32_t jj[4];
+      double x[4], y[4], z[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) jj[u] = q0 + u < g1 ? gord[q0 + u] : -1;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t gj = cb + (jj[u] < 0 ? 0 : jj[u]);
+        x[u] = L[gj];
+        y[u] = L[N + gj];
+        z[u] = L[2 * N + gj];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (jj[u] < 0 || (jj[u] == i && s0 == 0 && s1 == 0 && s2 == 0)) continue;
+        V3Cand c;
+        c.rx = (x[u] + (double)s0 * D.cfg.box[0]) - xi;
+        c.ry = (y[u] + (double)s1 * D.cfg.box[1]) - yi;
+        c.rz = (z[u] + (double)s2 * D.cfg.box[2]) - zi;
+        c.d2 = v3dot(c.rx, c.ry, c.rz, c.rx, c.ry, c.rz);
+        c.j = jj[u];
+        c.k = kk;
+        c.code = code;
+        f(c);
+      }
     }
-  });
+  }, near2);
 }
 
 // Ranks the n candidates in LDS by (squared distance, index, image code): ord[rank] = candidate.
@@ -498,12 +524,19 @@ __device__ __forceinline__ int v3_band_bin(double d2, double lo, double step) {
   return k;
 }
 
+// The squared-distance histogram of a block (V3Build::hist): bin k from lo + k step, the last one open; next = the
+// first bin that no band has taken (64: none left to read).
+struct V3Hist {
+  double lo, step;
+  int next;
+};
+
 // A block of more than HFV_V3_CAP candidates, taken in bands of squared distance: the candidates of the
-// next band [lo, hi) (hi chosen from a histogram so that at most HFV_V3_CAP fall in it; +inf for the
-// last) gathered into LDS and ranked.  Returns their count, or -1 where even a narrow band near lo holds
-// more than HFV_V3_CAP.
+// next band [lo, hi) (hi chosen from the histogram so that at most HFV_V3_CAP fall in it; +inf for the
+// last) gathered into LDS and ranked.  A histogram serves until one of its bins holds too many, so most bands scan
+// the block once.  Returns their count, or -1 where even a narrow band near lo holds more than HFV_V3_CAP.
 __device__ int v3_band(const Batch& B, const SimDesc& D, const V2Bufs& V, int s, int32_t i, double xi, double yi,
-                       double zi, int K, V3Cell& C, double lo, double& hi) {
+                       double zi, int K, V3Cell& C, V3Hist& H, double lo, double& hi) {
   const int lane = __lane_id();
   V3Build& Q = C.u.b;
   double dmax = 0.;  // beyond every candidate of the block
@@ -514,29 +547,36 @@ __device__ int v3_band(const Batch& B, const SimDesc& D, const V2Bufs& V, int s,
   }
   if (!(dmax > lo)) dmax = 2. * lo + 1.;
   int b = -1;
-  for (int zoom = 0; zoom < 4 && b < 0; ++zoom) {
-    const double step = (dmax - lo) / 64.;
-    Q.hist[lane] = 0u;
-    wave_sync();
-    v3_lane_candidates(B, D, V, s, i, xi, yi, zi, K, [&](const V3Cand& c) {
-      if (c.d2 >= lo) atomicAdd(&Q.hist[v3_band_bin(c.d2, lo, step)], 1u);
-    });
-    wave_sync();
-    int incl = (int)Q.hist[lane];
+  for (int zoom = 0; zoom < 5 && b < 0; ++zoom) {
+    if (zoom > 0 || H.next > 63) {
+      if (zoom == 0) continue;
+      H.lo = lo;
+      H.step = (dmax - lo) / 64.;
+      H.next = 0;
+      Q.hist[lane] = 0u;
+      wave_sync();
+      v3_lane_candidates(B, D, V, s, i, xi, yi, zi, K, [&](const V3Cand& c) {
+        if (c.d2 >= lo) atomicAdd(&Q.hist[v3_band_bin(c.d2, lo, H.step)], 1u);
+      });
+      wave_sync();
+    }
+    int incl = lane < H.next ? 0 : (int)Q.hist[lane];
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const int t = __shfl_up(incl, o, 64);
       if (lane >= o) incl += t;
     }
-    b = __popcll(__ballot(incl <= HFV_V3_CAP)) - 1;  // the longest prefix of bins that fits
-    if (b >= 0) hi = b == 63 ? (double)INFINITY : lo + (double)(b + 1) * step;
+    b = __popcll(__ballot(incl <= HFV_V3_CAP)) - 1;  // the longest run of bins that fits
+    if (b < H.next) b = -1;
+    if (b >= 0) hi = b == 63 ? (double)INFINITY : H.lo + (double)(b + 1) * H.step;
     if (b >= 0 && !(hi > lo)) b = -1;  // (a band too narrow for the doubles)
-    dmax = lo + step;  // else: the first bin alone holds too many; split it
+    if (zoom > 0) dmax = lo + H.step;  // else: the first bin alone holds too many; split it
   }
   if (b < 0) return -1;
+  H.next = b + 1;
   if (lane == 0) Q.nband = 0u;
   wave_sync();
-  v3_lane_candidates(B, D, V, s, i, xi, yi, zi, K, [&](const V3Cand& c) {
+  v3_lane_candidates<true>(B, D, V, s, i, xi, yi, zi, K, [&](const V3Cand& c) {
     if (!(c.d2 >= lo && c.d2 < hi)) return;
     const uint32_t at = atomicAdd(&Q.nband, 1u);  // (any order: the rank orders them)
     if (at >= HFV_V3_CAP) return;                 // (cannot happen: the histogram counted them)
@@ -548,7 +588,7 @@ __device__ int v3_band(const Batch& B, const SimDesc& D, const V2Bufs& V, int s,
     Q.rx[at] = c.rx;
     Q.ry[at] = c.ry;
     Q.rz[at] = c.rz;
-  });
+  }, hi);
   wave_sync();
   const int n = __builtin_amdgcn_readfirstlane((int)min(Q.nband, (uint32_t)HFV_V3_CAP));
   v3_rank(C, n);
@@ -621,7 +661,8 @@ __device__ int v3_build(const Batch& B, const SimDesc& D, const V2Bufs& V, int s
   const V3Build& Q = C.u.b;
   int n = v3_gather(B, D, V, s, i, xi, yi, zi, K, C);
   double blo = 0., bhi = (double)INFINITY;
-  if (n < 0) n = v3_band(B, D, V, s, i, xi, yi, zi, K, C, blo, bhi);
+  V3Hist H{0., 0., 64};
+  if (n < 0) n = v3_band(B, D, V, s, i, xi, yi, zi, K, C, H, blo, bhi);
   while (n >= 0) {
     bool stop = false;
     for (int q = 0; q < n; ++q) {
@@ -635,7 +676,7 @@ __device__ int v3_build(const Batch& B, const SimDesc& D, const V2Bufs& V, int s
     }
     if (stop || bhi == (double)INFINITY) break;
     blo = bhi;
-    n = v3_band(B, D, V, s, i, xi, yi, zi, K, C, blo, bhi);
+    n = v3_band(B, D, V, s, i, xi, yi, zi, K, C, H, blo, bhi);
   }
   if (n < 0) {  // a band too dense for the LDS: from blo on, the next one is a wave minimum over a rescan
     bool have_last = false;
@@ -838,8 +879,8 @@ __device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimS
 // the next free lanes, and those become the new vertices: kept vertices stay where they are (their order is
 // the host's), and close up only when the lanes run out.  Candidates come in bands of squared distance that
 // hold about 45 generators each (the first is enough for most cells), so that a band is ranked with one key a
-// lane.  A cell that outgrows this (64 live vertices, 64 candidates in a band, a face of more than 12 vertices)
-// is left to k_v3_cells.
+// lane.  A cell that outgrows this (64 live vertices, 64 candidates in a band that was narrowed already, six bands, a
+// face of more than 12 vertices) is left to k_v3_cells (on the KH lattice of 48^3 24 cells a rebuild, all by a face).
 // What bounds it: instruction issue, FP64 and integer alike at 4 cycles a wave (about 250 instructions a cutting
 // clip, 16 of them a cell).  7 KB of LDS and 128 VGPRs let 16 waves a CU hide each other's latencies, where
 // the LDS cell has 15 KB (10 waves) and spends 66k of its 126k cycles a cell on clips (LDS round trips), 30k on
@@ -847,8 +888,8 @@ __device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimS
 // 16.3 -> 12.2 ms, the rebuild 1.73 -> 1.25 ms a step.
 #define HFV_V3R_CAP 64  // candidates of a band: one a lane
 #define HFV_V3R_FAN 12  // vertices of a face
+#define HFV_V3R_BANDS 6 // bands tried
 #define HFV_V3R_TRI 96  // fan triangles of a cell
-#define HFV_V3_LEFT (-1)  // femit mark: the cell is left to k_v3_cells
 
 struct V3RCands {
   V3Key key[HFV_V3R_CAP];
@@ -1018,7 +1059,8 @@ __device__ __forceinline__ int v3r_clip(V3RCell& C, V3RVerts& T, int& np, double
   return 1;
 }
 
-// The block's candidates of squared distance in [lo, hi) into LDS and ranked: their count, -1 beyond HFV_V3R_CAP.
+// The block's candidates of squared distance in [lo, hi) into LDS and ranked: their count (beyond HFV_V3R_CAP: the
+// count only).
 __device__ __forceinline__ int v3r_band(const Batch& B, const SimDesc& D, const V2Bufs& V, int s, int32_t i, double xi,
                                         double yi, double zi, int K, V3RCell& C, double lo, double hi) {
   const int lane = __lane_id();
@@ -1030,7 +1072,7 @@ __device__ __forceinline__ int v3r_band(const Batch& B, const SimDesc& D, const 
   wave_sync();
   if (lane == 0) Q.n = 0;
   wave_sync();
-  v3_lane_bins(D, xi, yi, zi, K, [&](int key, int s0, int s1, int s2, bool) {
+  v3_lane_bins<true>(D, xi, yi, zi, K, [&](int key, int s0, int s1, int s2, bool) {
     const int32_t kk = ((s0 & 0xFF) << 16) | ((s1 & 0xFF) << 8) | (s2 & 0xFF);  // the host's memcmp order
     const int32_t g0 = gst[key], g1 = gst[key + 1];
     for (int32_t q0 = g0; q0 < g1; q0 += 2) {  // (two candidates' loads in flight)
@@ -1064,10 +1106,10 @@ __device__ __forceinline__ int v3r_band(const Batch& B, const SimDesc& D, const 
         Q.rz[at] = rz;
       }
     }
-  });
+  }, hi);
   wave_sync();
   const int n = __builtin_amdgcn_readfirstlane(Q.n);
-  if (n > HFV_V3R_CAP) return -1;
+  if (n > HFV_V3R_CAP) return n;
   // the rank of this lane's candidate: the number of keys below it, by the squared distance (a non-negative
   // double orders as its bits), by the whole key where two squared distances are equal
   const V3Key own = Q.key[lane < n ? lane : 0];
@@ -1135,15 +1177,33 @@ __device__ __forceinline__ int v3r_build(const Batch& B, const SimDesc& D, const
   T.top = 8;
   np = 6;
   const V3RCands& Q = C.u.q;
-  // bands of equal volume: radii 2.2 mean bin widths times the cube roots of 1, 2, 3, 4, then all the rest
+  // Bands of squared distance that hold some 45 candidates each: the volume v of their balls is counted in units of
+  // the first band's, of radius 2.2 mean bin widths (44.6 bins), and the next band's follows from what the last one
+  // held.  In a dense place the generator's own bin tells the first one (a bin holds 8 of the mean density's
+  // generators once in 10^5), and a band that holds more than the lanes is narrowed, once: a cell that calls for
+  // more has a clump beside it and hundreds of candidates, which k_v3_cells takes 192 at a time.
   const double t0 = 4.84 * ((w0 * w0 + w1 * w1 + w2 * w2) / 3.);
+  const float far = 1.7320508f * (float)(K + 1) / 2.2f, vend = far * far * far;  // (the block lies within)
+  int own;
+  {
+    const int key = (v2_bin(xi, w0, D.vnb[0]) * D.vnb[1] + v2_bin(yi, w1, D.vnb[1])) * D.vnb[2] + v2_bin(zi, w2, D.vnb[2]);
+    const int32_t* g = V.gcnt + D.cell_base + s + key;
+    own = __builtin_amdgcn_readfirstlane(g[1] - g[0]);
+  }
+  float v = 0.f, dv = own >= 8 ? 1.f / (float)own : 1.f;
   double blo = 0.;
-  bool stop = false;
-  for (int band = 0; band < 5 && !stop; ++band) {
-    const double bhi = band == 0 ? t0 : band == 1 ? 1.5874 * t0 : band == 2 ? 2.0801 * t0 : band == 3 ? 2.5198 * t0
-                                                                                                   : (double)INFINITY;
+  int narrowed = 0;
+  for (int pass = 0; blo < (double)INFINITY; ++pass) {
+    if (pass == HFV_V3R_BANDS) return 2;
+    const float vhi = v + dv;
+    const double bhi = vhi < vend ? fmax(blo, t0 * (double)cbrtf(vhi * vhi)) : (double)INFINITY;
     const int n = v3r_band(B, D, V, s, i, xi, yi, zi, K, C, blo, bhi);
-    if (n < 0) return 2;
+    if (n > HFV_V3R_CAP) {
+      if (++narrowed == 2) return 2;
+      dv = (vhi < vend ? dv : vend - v) * 45.f / (float)n;
+      continue;
+    }
+    bool stop = false;
     for (int q = 0; q < n; ++q) {
       const int a = __builtin_amdgcn_readfirstlane(Q.ord[q]);
       const V3Key key = Q.key[a];
@@ -1154,8 +1214,10 @@ __device__ __forceinline__ int v3r_build(const Batch& B, const SimDesc& D, const
       if (v3r_clip(C, T, np, Q.rx[a], Q.ry[a], Q.rz[a], 0.5 * key.d2, key.j, v3_code_of(key.k)) < 0) return 2;
     }
     // every later candidate is at least this band's end away
-    if (!__ballot(T.q >= 0.25 * bhi)) stop = true;
+    if (stop || !__ballot(T.q >= 0.25 * bhi)) break;
     blo = bhi;
+    v = vhi;
+    dv *= fminf(45.f / (float)(n + 1), 8.f);
   }
   r2 = wave_max_nonneg(T.q);
   // completeness: every unvisited generator lies farther than K bin widths
@@ -1354,44 +1416,48 @@ __global__ void __launch_bounds__(256, 4) k_v3_cells_reg(Batch B, V2Bufs V) {
   const double xi = B.C.loc[gi], yi = B.C.loc[N + gi], zi = B.C.loc[2 * N + gi];
   const int kmax = max(6, max(D.vnb[0], max(D.vnb[1], D.vnb[2])));
   V3RVerts T;
-  int np = 0, r = 1;
+  int np = 0, r = 1, K = 2;
   double r2 = 0.;
-  for (int K = 2; K <= kmax && r == 1; ++K) {
+  for (; K <= kmax; ++K) {
     r = v3r_build(B, D, V, s, i, xi, yi, zi, K, C, T, np, r2);
     if (r == 0) r = v3r_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, C, T, np, r2);
+    if (r != 1 || K == 3) break;  // (beyond 7 x 7 x 7 bins the LDS cell, whose candidate list is longer)
   }
-  if (r != 0 && lane == 0) V.femit[gi] = HFV_V3_LEFT;
+  if (r != 0 && lane == 0) {
+    V.femit[gi] = K + (r == 1 ? 1 : 0);  // the K to go on with: smaller ones are known to be too small
+    V.gfill[cb + s + atomicAdd(&S.n_left, 1)] = i;
+  }
 }
 
-// The cells that k_v3_cells_reg left.  Grid: HFV_V3_SUB one-wavefront blocks per cell chunk, each looking
-// through HFV_BLOCK / HFV_V3_SUB cells and building those marked, one after another (a block per cell, nearly
-// all of which only look, took 75 us on KH 48^3).
-#define HFV_V3_SUB 8
-__global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V) {
+// The cells that k_v3_cells_reg left, from the list of their simulation (in gfill, whose placement cursors are
+// used up): its 1 << sub one-wavefront blocks per cell chunk take entries in turn, so that they have equal shares
+// wherever the cells lie.  Blocks that looked through 32 cells each and built those left among them had a clump's
+// cells to build one after another.  With fully active steps, a step of clumped generators (times for a wave per
+// cell, those blocks, the list): 2000 cells, three quarters of them in a cube of 0.4: 2.70, 21.3, 2.20 ms; 8000
+// alike: 5.51, 33.1, 3.41; 64,000, half of them in a cube of 0.5: 3.93, 10.35, 3.66; 64,000 uniform: 3.90, 3.10, 2.77;
+// the KH lattice of 48^3: 2.89, 1.97, 1.95.
+__global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V, int sub) {
   __shared__ V3Cell C;
-  const BlockJob J = B.cjobs[blockIdx.x / HFV_V3_SUB];
+  const BlockJob J = B.cjobs[blockIdx.x >> sub];
   if (J.sim < 0) return;
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
   SimStep& S = B.st[s];
   if (D.vmesh != 3 || !S.stepping) return;
-  constexpr int CELLS = HFV_BLOCK / HFV_V3_SUB;
-  static_assert(CELLS <= 64, "a lane per cell looked at");
-  const int64_t g0 = (int64_t)J.lo + (blockIdx.x % HFV_V3_SUB) * CELLS;
   const int lane = __lane_id();
   const int64_t N = B.C.n, cb = D.cell_base;
   const int kmax = max(6, max(D.vnb[0], max(D.vnb[1], D.vnb[2])));
-  uint64_t todo = __ballot(lane < CELLS && g0 + lane < J.hi && V.femit[g0 + lane] == HFV_V3_LEFT);
-  for (; todo; todo &= todo - 1) {
-    const int64_t gi = g0 + __builtin_ctzll(todo);
-    const int32_t i = (int32_t)(gi - cb);
+  const int32_t n = S.n_left, step = (D.cchunk1 - D.cchunk0) << sub;
+  for (int32_t q = ((J.chunk - D.cchunk0) << sub) + (int32_t)(blockIdx.x & ((1u << sub) - 1u)); q < n; q += step) {
+    const int32_t i = V.gfill[cb + s + q];
+    const int64_t gi = cb + i;
     const double xi = B.C.loc[gi], yi = B.C.loc[N + gi], zi = B.C.loc[2 * N + gi];
     int np = 0, nt = 0, r = 1;
     double r2 = 0.;
     wave_sync();
-    for (int K = 2; K <= kmax && r == 1; ++K) {
+    for (int K = __builtin_amdgcn_readfirstlane(V.femit[gi]); K <= kmax && r == 1; ++K) {
       r = v3_build(B, D, V, s, i, xi, yi, zi, K, C, np, nt, r2);
-      if (r == 0) r = v3_finish(B, V, D, S, J.chunk, gi, i, xi, yi, zi, C, np, nt, r2);
+      if (r == 0) r = v3_finish(B, V, D, S, D.cchunk0 + i / HFV_BLOCK, gi, i, xi, yi, zi, C, np, nt, r2);
     }
     if (r != 0 && lane == 0) {
       V.femit[gi] = 0;
