@@ -948,12 +948,12 @@ struct V2Face {
   int32_t nb, code;
 };
 
-// CSR entries a cell's bucket holds between k_v2_faces and k_v2_conn (further ones go to a list that the
-// cells concerned search): a random 3D mesh has 15.5 faces a cell, one cell in a hundred has more than 24
+// CSR entries a cell's bucket holds between k_v2_faces and k_v2_conn (further ones are chained in a list of the
+// simulation): a random 3D mesh has 15.5 faces a cell, one cell in a hundred has more than 24
 #define HFV_BUCKET 24
-// An entry beyond its cell's bucket.
+// An entry beyond its cell's bucket, and the next one of the cell (-1: none).
 struct V2Over {
-  int32_t cell, conn, nbr;
+  int32_t conn, nbr, next;
 };
 
 struct V2Bufs {
@@ -961,7 +961,7 @@ struct V2Bufs {
                    // between the steps
   int32_t* gfill;  // same layout: placement cursors, then (3D) the list of the cells the register builder left
   int32_t* gord;   // [N] at cell_base: local cell indices grouped by bin
-  int32_t* gkey;   // [N] bin of each cell
+  int32_t* gkey;   // [N] bin of each cell, then the first of its entries in over (-1: none)
   int32_t* femit;  // [N] faces a cell emits
   int32_t* vst;    // [N] start of a cell's faces in vf
   int32_t* ccnt;   // [N] CSR entries per cell

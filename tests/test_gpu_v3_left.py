@@ -49,6 +49,21 @@ def test_clumped_mesh_equals_host(n, share, width, boundary):
     dev.close()
 
 
+def test_cells_of_many_entries_equal_host():
+    """Random generators: one cell in a hundred has more CSR entries than its bucket holds, chained behind it."""
+    print("[v3 left] chained entries", flush=True)
+    prob = _clump(20000, 0.0, 1.0, fvs.PERIODIC)
+    many = prob.mesh.as_dict()["count"] > 24
+    assert 0 < many.sum() < prob.n // 20
+    dev = ics.build_device_sim(prob)
+    assert dev.run(1) == 1
+    loc = dev.get_state(["loc"])["loc"].reshape(3, prob.n).T.copy()
+    want, got = VoronoiMesh(3, prob.cfg.box, True, loc).as_dict(), dev.get_mesh()
+    for k in ("n_faces", "left", "right", "offset", "count", "conn"):
+        assert np.array_equal(got[k], want[k]), k
+    dev.close()
+
+
 def test_clumped_batch_members_equal_alone():
     print("[v3 left] batch", flush=True)
     probs = [_clump(1000, 0.5, 0.2, fvs.PERIODIC), ics.sedov_2d(side=16, t_end=0.01),
