@@ -189,6 +189,7 @@ struct hfv_ctx {
   int64_t ncg = 8, nfg = 8, live_chunks = 0;
   int cgsh = 0, fgsh = 0;     // log2 of the group sizes that the tables were dealt in
   int64_t face_items = 0;     // faces that the only simulation's face kernels cover
+  bool vscan = false;         // the rebuild's chunk sums are scanned (kScanChunks)
   int v3sub = 0;              // log2 of k_v3_cells' blocks per cell chunk
   std::vector<BlockJob> hcjobs, hfjobs;
   BlockJob *dcjobs = nullptr, *dfjobs = nullptr;
@@ -305,11 +306,10 @@ int ensure_v2(hfv_ctx* c) {
   v.vf = dalloc<V2Face>(c, 2 * c->nf);
   v.bkt = dalloc<uint64_t>(c, HFV_BUCKET * c->n);
   v.over = dalloc<V2Over>(c, c->nconn);
-  v.part0 = dalloc<int32_t>(c, c->ncchunk);
-  v.part1 = dalloc<int32_t>(c, c->ncchunk);
-  v.part2 = dalloc<int32_t>(c, c->ncchunk);
+  for (int32_t*& p : v.part) p = dalloc<int32_t>(c, c->ncchunk);
+  v.ptot = dalloc<int32_t>(c, 3 * c->nslots);
   if (!v.gcnt || !v.gfill || !v.femit || !v.ccnt || !v.gord || !v.gkey || !v.vst || !v.vf || !v.bkt || !v.over ||
-      !v.part0 || !v.part1 || !v.part2)
+      !v.part[0] || !v.part[1] || !v.part[2] || !v.ptot)
     return set_err(HFV_ERR_HIP, "out of device memory (rebuild buffers)");
   HIP_OK(hipMemsetAsync(v.gcnt, 0, sizeof(int32_t) * ns, c->stream));
   HIP_OK(hipMemsetAsync(v.vst, 0, sizeof(int32_t) * c->n, c->stream));
@@ -370,6 +370,11 @@ int64_t grid_position(int64_t j, int64_t g) { return 8 * ((j / g / 8) * g + j % 
 // face count (the faces past the current mesh have no cells and are skipped).
 int64_t face_range(const hfv_ctx* c, int s) { return c->desc[s].vmesh ? c->fcap[s] : c->fused[s]; }
 
+// Chunks from which on the rebuild's chunk sums are scanned by launches of their own.  On random 2D generators the
+// three kernels that need the sums before a chunk took, reading all of them / after the scans: 122 / 117 us on
+// 262,144 (1024 chunks; the scans 14), 498 / 457 on 10^6 (3906; the scans 20), 2131 / 1676 on 4 x 10^6 (the scans 54).
+constexpr int64_t kScanChunks = 2048;
+
 // log2 of the blocks per cell chunk that k_v3_cells launches for `chunks` chunks of 3D moving meshes: together some
 // 4096, a few more than the chip holds at once (10 a CU by LDS), as long as a block stays at 2 cells or more.
 int v3_sub(int64_t chunks) {
@@ -384,9 +389,10 @@ int v3_sub(int64_t chunks) {
 int write_jobs(hfv_ctx* c) {
   const int S = c->nslots;
   auto live = [&](int s) { return c->loaded[s] && !(c->batch && c->heng[s].done); };
-  int64_t lc = 0, lf = 0, l3 = 0;  // (l3: of 3D moving meshes)
+  int64_t lc = 0, lf = 0, l3 = 0, lv = 0;  // (l3: of 3D moving meshes, lv: of the largest moving mesh)
   for (int s = 0; s < S; ++s) {
     if (!live(s)) continue;
+    if (c->desc[s].vmesh) lv = std::max<int64_t>(lv, (c->nused[s] + BLOCK - 1) / BLOCK);
     if (c->desc[s].vmesh == 3) l3 += (c->nused[s] + BLOCK - 1) / BLOCK;
     lc += (c->nused[s] + BLOCK - 1) / BLOCK;
     lf += (face_range(c, s) + BLOCK - 1) / BLOCK;
@@ -398,8 +404,10 @@ int write_jobs(hfv_ctx* c) {
   const int64_t items = c->batch || !c->loaded[0] ? 0 : face_range(c, 0);
   if (cgsh != c->cgsh || fgsh != c->fgsh || items != c->face_items) drop_graph(c);
   const int v3sub = v3_sub(l3);
-  if (v3sub != c->v3sub) drop_graph(c);
+  const bool vscan = lv > kScanChunks;
+  if (v3sub != c->v3sub || vscan != c->vscan) drop_graph(c);
   c->v3sub = v3sub;
+  c->vscan = vscan;
   c->cgsh = cgsh;
   c->fgsh = fgsh;
   c->face_items = items;
@@ -1157,8 +1165,13 @@ void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
     hipLaunchKernelGGL(k_mesh1d_cells, gc, gb, 0, st, B);
   }
   if (c->any_vmesh) {
-    const V2Bufs& V = c->v2;
+    V2Bufs V = c->v2;
+    V.scanned = c->vscan ? 1 : 0;
+    auto prefix = [&](int k) {
+      if (c->vscan) hipLaunchKernelGGL(k_v2_prefix, dim3((unsigned)c->nslots), dim3(HFV_PREFIX_BLOCK), 0, st, B, V, k);
+    };
     hipLaunchKernelGGL(k_v2_sum<0>, gc, gb, 0, st, B, V);
+    prefix(0);
     hipLaunchKernelGGL(k_v2_bins, gc, gb, 0, st, B, V);
     hipLaunchKernelGGL(k_v2_place, gc, gb, 0, st, B, V);
     if (c->any_vmesh2) hipLaunchKernelGGL(k_v2_cells, dim3((unsigned)(c->ncg * HFV_V2_SUB)), gb, 0, st, B, V);
@@ -1166,8 +1179,10 @@ void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
       hipLaunchKernelGGL(k_v3_cells_reg, dim3((unsigned)(c->ncg * HFV_V3R_SUB)), dim3(256), 0, st, B, V);
       hipLaunchKernelGGL(k_v3_cells, dim3((unsigned)(c->ncg << c->v3sub)), dim3(64), 0, st, B, V, c->v3sub);
     }
+    prefix(1);
     hipLaunchKernelGGL(k_v2_faces, gc, gb, 0, st, B, V);
     hipLaunchKernelGGL(k_v2_sum<1>, gc, gb, 0, st, B, V);
+    prefix(2);
     hipLaunchKernelGGL(k_v2_conn, gc, gb, 0, st, B, V);
   }
 }

@@ -968,9 +968,11 @@ struct V2Bufs {
   V2Face* vf;      // [2 F] faces in provisional order: shares of the chunks at face_base, the rest at F + face_base
   uint64_t* bkt;   // [HFV_BUCKET][N] entries of a cell: (CSR value << 32) | neighbour
   V2Over* over;    // [CSR capacity] at conn_base: entries beyond their cells' buckets
-  int32_t* part0;  // [cell chunks] sums of gcnt over the chunk's bins
-  int32_t* part1;  // [cell chunks] sums of femit over the chunk's cells (their cursors while they are built)
-  int32_t* part2;  // [cell chunks] sums of ccnt
+  // [cell chunks] sums over the chunk's bins of gcnt, over its cells of femit (their cursors while they are built)
+  // and of ccnt
+  int32_t* part[3];
+  int32_t* ptot;   // [S][3] the totals where part is scanned
+  int scanned;     // part holds the sums of the chunks before (k_v2_prefix)
 };
 
 __device__ __forceinline__ int v2_bin(double x, double w, int nb) {

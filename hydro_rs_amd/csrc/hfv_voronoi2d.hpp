@@ -33,7 +33,7 @@
 
 namespace hfv {
 
-#define HFV_SCAN_BLOCK 1024
+#define HFV_PREFIX_BLOCK 1024
 // A clip removes the vertices beyond a plane by more than this fraction of its offset (the host
 // tessellator's threshold): vertices on it test as beyond by a rounding error on exact lattices.
 #define HFV_CLIP_TOL 1e-12
@@ -71,10 +71,16 @@ __device__ __forceinline__ int32_t block_excl_scan(int32_t v, int32_t* total) {
   return before + x - v;
 }
 
-// The sum of the simulation's chunk sums before chunk `chunk`, and of all of them (every thread gets both).
-// Each block reads every chunk sum: at most a few thousand words that the L2 holds, where a launch of its
-// own to scan them costs 4-5 us.
-__device__ __forceinline__ int32_t chunks_before(const int32_t* part, const SimDesc& D, int32_t chunk, int32_t* total) {
+// The sum of the simulation's chunk sums (array k of V.part) before chunk `chunk`, and of all of them (every thread
+// gets both).  Each block reads every chunk sum: at most a few thousand words that the L2 holds, where a launch of
+// its own to scan them costs 4-5 us.  Meshes of more chunks have them scanned (k_v2_prefix).
+__device__ __forceinline__ int32_t chunks_before(const V2Bufs& V, int k, const SimDesc& D, int s, int32_t chunk,
+                                                 int32_t* total) {
+  const int32_t* part = V.part[k];
+  if (V.scanned) {
+    *total = V.ptot[3 * s + k];
+    return part[chunk];
+  }
   __shared__ int32_t wb[HFV_BLOCK / 64], wt[HFV_BLOCK / 64];
   int32_t b = 0, t = 0;
   for (int32_t c = D.cchunk0 + (int32_t)threadIdx.x; c < D.cchunk1; c += HFV_BLOCK) {
@@ -117,7 +123,39 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_sum(Batch B, V2Bufs V) {
   const int64_t len = CSR ? D.n : (int64_t)D.vnb[0] * D.vnb[1] * D.vnb[2];
   const int32_t* a = CSR ? V.ccnt + D.cell_base : V.gcnt + D.cell_base + s;
   const uint32_t t = block_sum_u32(k < len ? (uint32_t)a[k] : 0u);
-  if (threadIdx.x == 0) (CSR ? V.part2 : V.part0)[J.chunk] = (int32_t)t;
+  if (threadIdx.x == 0) V.part[CSR ? 2 : 0][J.chunk] = (int32_t)t;
+}
+
+// The chunk sums (array k) of a simulation, scanned in place: one block per simulation.
+__global__ void __launch_bounds__(HFV_PREFIX_BLOCK) k_v2_prefix(Batch B, V2Bufs V, int k) {
+  const int s = blockIdx.x;
+  const SimDesc& D = B.sims[s];
+  if (!D.vmesh || !B.st[s].stepping) return;
+  __shared__ int32_t ws[HFV_PREFIX_BLOCK / 64];
+  int32_t* part = V.part[k];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int32_t carry = 0;
+  for (int32_t c0 = D.cchunk0; c0 < D.cchunk1; c0 += HFV_PREFIX_BLOCK) {
+    const int32_t c = c0 + (int32_t)threadIdx.x;
+    const int32_t v = c < D.cchunk1 ? part[c] : 0;
+    int32_t x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int32_t y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) ws[wid] = x;
+    __syncthreads();
+    int32_t before = 0, tot = 0;
+    for (int w = 0; w < HFV_PREFIX_BLOCK / 64; ++w) {
+      if (w < wid) before += ws[w];
+      tot += ws[w];
+    }
+    if (c < D.cchunk1) part[c] = carry + before + x - v;
+    carry += tot;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) V.ptot[3 * s + k] = carry;
 }
 
 // Bin starts and placement cursors; the chunk sums of the emitted faces restart at zero.
@@ -127,13 +165,13 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_bins(Batch B, V2Bufs V) {
   const int s = J.sim;
   const SimDesc& D = B.sims[s];
   if (!D.vmesh || !B.st[s].stepping) return;
-  if (threadIdx.x == 0) V.part1[J.chunk] = 0;
+  if (threadIdx.x == 0) V.part[1][J.chunk] = 0;
   const int64_t nbins = (int64_t)D.vnb[0] * D.vnb[1] * D.vnb[2];  // <= n
   const int64_t k = (int64_t)J.lo - D.cell_base + threadIdx.x;
   int32_t* a = V.gcnt + D.cell_base + s;
   const int32_t v = k < nbins ? a[k] : 0;
   int32_t all, tot;
-  const int32_t base = chunks_before(V.part0, D, J.chunk, &all);
+  const int32_t base = chunks_before(V, 0, D, s, J.chunk, &all);
   const int32_t x = base + block_excl_scan(v, &tot);
   if (k < nbins) {
     a[k] = x;
@@ -191,7 +229,7 @@ __device__ __forceinline__ bool v2_emits(const Batch& B, int64_t cb, int32_t nb,
 __device__ __forceinline__ int32_t v_place_faces(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int chunk,
                                                  int cnt) {
   const int32_t share = (int32_t)(D.face_cap / (D.cchunk1 - D.cchunk0));
-  const int32_t p = atomicAdd(&V.part1[chunk], cnt);
+  const int32_t p = atomicAdd(&V.part[1][chunk], cnt);
   if (p + cnt <= share) return (int32_t)(D.face_base + (int64_t)(chunk - D.cchunk0) * share + p);
   const int32_t o = atomicAdd(&S.nf_tmp, cnt);
   return (int64_t)o + cnt <= D.face_cap ? (int32_t)(B.F.nf + D.face_base + o) : -1;
@@ -876,7 +914,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
   const int64_t gi0 = (int64_t)J.lo + threadIdx.x;
   const bool in = gi0 < J.hi;
   int32_t all, tot;
-  const int32_t base = chunks_before(V.part1, D, J.chunk, &all);
+  const int32_t base = chunks_before(V, 1, D, s, J.chunk, &all);
   offs[threadIdx.x] = block_excl_scan(in ? V.femit[gi0] : 0, &tot);
   starts[threadIdx.x] = in ? V.vst[gi0] : 0;
   const bool full = all > D.face_cap;
@@ -940,7 +978,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_conn(Batch B, V2Bufs V) {
   if (bin < (int64_t)D.vnb[0] * D.vnb[1] * D.vnb[2]) V.gcnt[D.cell_base + s + bin] = 0;
   const int m = in ? V.ccnt[gi] : 0;
   int32_t all, tot;
-  const int32_t base = chunks_before(V.part2, D, J.chunk, &all);
+  const int32_t base = chunks_before(V, 2, D, s, J.chunk, &all);
   const int32_t x = base + block_excl_scan(m, &tot);
   const bool full = all > D.conn_cap;
   const bool bad = full || S.err != 0;
