@@ -303,12 +303,11 @@ int ensure_v2(hfv_ctx* c) {
   v.gord = dalloc<int32_t>(c, c->n);
   v.gkey = dalloc<int32_t>(c, c->n);
   v.vst = dalloc<int32_t>(c, c->n);
-  v.vf = dalloc<V2Face>(c, 2 * c->nf);
+  v.vf = dalloc<V2Face>(c, c->nf);
   v.bkt = dalloc<uint64_t>(c, HFV_BUCKET * c->n);
-  v.over = dalloc<V2Over>(c, c->nconn);
   for (int32_t*& p : v.part) p = dalloc<int32_t>(c, c->ncchunk);
   v.ptot = dalloc<int32_t>(c, 3 * c->nslots);
-  if (!v.gcnt || !v.gfill || !v.femit || !v.ccnt || !v.gord || !v.gkey || !v.vst || !v.vf || !v.bkt || !v.over ||
+  if (!v.gcnt || !v.gfill || !v.femit || !v.ccnt || !v.gord || !v.gkey || !v.vst || !v.vf || !v.bkt ||
       !v.part[0] || !v.part[1] || !v.part[2] || !v.ptot)
     return set_err(HFV_ERR_HIP, "out of device memory (rebuild buffers)");
   HIP_OK(hipMemsetAsync(v.gcnt, 0, sizeof(int32_t) * ns, c->stream));
@@ -537,13 +536,14 @@ int alloc_batch(hfv_ctx* c) {
   F.nloc = dalloc<uint16_t>(c, nk);
   C.minv = dalloc<double>(c, 6 * n);
   // sliced gradient geometry: a slot's slices hold the longest of their 64 cells' CSR rows each; a mesh
-  // whose slices need more than this evaluates its gradient geometry per step
+  // whose slices need more than this evaluates its gradient geometry per step.  None in a context whose only mesh
+  // moves: their 45 bytes an entry are twice what the rebuild's buffers (ensure_v2) take.
   c->sebase.assign(S, 0);
   c->secap.assign(S, 0);
   int64_t nse = 0;
   for (int s = 0; s < S; ++s) {
     c->sebase[s] = nse;
-    c->secap[s] = (c->kcap[s] + c->kcap[s] / 2 + 64 * 8) / 64 * 64;
+    c->secap[s] = c->batch || c->params[s].motion == HFV_FIXED ? (c->kcap[s] + c->kcap[s] / 2 + 64 * 8) / 64 * 64 : 0;
     nse += c->secap[s];
   }
   F.nse = nse;

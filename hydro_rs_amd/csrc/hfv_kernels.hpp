@@ -948,13 +948,17 @@ struct V2Face {
   int32_t nb, code;
 };
 
+static_assert(sizeof(V2Face) == 8 * sizeof(double), "a face takes a flux record's place");
+
 // CSR entries a cell's bucket holds between k_v2_faces and k_v2_conn (further ones are chained in a list of the
 // simulation): a random 3D mesh has 15.5 faces a cell, one cell in a hundred has more than 24
 #define HFV_BUCKET 24
-// An entry beyond its cell's bucket, and the next one of the cell (-1: none).
+// An entry beyond its cell's bucket, and the next one of the cell (-1: none).  A simulation's list (two entries a
+// face at most) has the place of its faces' static geometry (F.fs), which moving meshes have not.
 struct V2Over {
   int32_t conn, nbr, next;
 };
+static_assert(2 * sizeof(V2Over) <= 4 * sizeof(double), "both entries of a face in its static geometry's place");
 
 struct V2Bufs {
   int32_t* gcnt;   // [N + S + 1], simulation s at cell_base + s: bin counts, then bin starts (nbins + 1); zero
@@ -965,9 +969,10 @@ struct V2Bufs {
   int32_t* femit;  // [N] faces a cell emits
   int32_t* vst;    // [N] start of a cell's faces in vf
   int32_t* ccnt;   // [N] CSR entries per cell
-  V2Face* vf;      // [2 F] faces in provisional order: shares of the chunks at face_base, the rest at F + face_base
+  // [F] faces in provisional order, the chunks' shares at face_base.  Faces beyond their chunk's share go to the place
+  // of the simulation's flux records (F.rec), dead between the accumulation and the next fluxes.
+  V2Face* vf;
   uint64_t* bkt;   // [HFV_BUCKET][N] entries of a cell: (CSR value << 32) | neighbour
-  V2Over* over;    // [CSR capacity] at conn_base: entries beyond their cells' buckets
   // [cell chunks] sums over the chunk's bins of gcnt, over its cells of femit (their cursors while they are built)
   // and of ccnt
   int32_t* part[3];

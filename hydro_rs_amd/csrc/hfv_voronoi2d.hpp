@@ -222,10 +222,10 @@ __device__ __forceinline__ bool v2_emits(const Batch& B, int64_t cb, int32_t nb,
   return nb < 0 || nb > i || !B.C.act[cb + nb];
 }
 
-// Place of a cell's cnt emitted faces in the provisional order (an index into vf): after those that its chunk
-// has placed, in the chunk's share of the simulation's face capacity, or in the common second half where the
-// chunk's share is full.  -1 beyond the capacity.  (One cursor for the whole simulation instead is an atomic
-// on one address per cell, about 20 ns each: it alone bounded the 3D cell kernel.)
+// Place of a cell's cnt emitted faces in the provisional order: after those that its chunk has placed, in the
+// chunk's share of the simulation's face capacity, or where the share is full in the common overflow (from F.nf on:
+// v_faces_at).  -1 beyond the capacity.  (One cursor for the whole simulation instead is an atomic on one address
+// per cell, about 20 ns each: it alone bounded the 3D cell kernel.)
 __device__ __forceinline__ int32_t v_place_faces(const Batch& B, const V2Bufs& V, const SimDesc& D, SimStep& S, int chunk,
                                                  int cnt) {
   const int32_t share = (int32_t)(D.face_cap / (D.cchunk1 - D.cchunk0));
@@ -234,6 +234,11 @@ __device__ __forceinline__ int32_t v_place_faces(const Batch& B, const V2Bufs& V
   const int32_t o = atomicAdd(&S.nf_tmp, cnt);
   return (int64_t)o + cnt <= D.face_cap ? (int32_t)(B.F.nf + D.face_base + o) : -1;
 }
+
+__device__ __forceinline__ V2Face* v_faces_at(const Batch& B, const V2Bufs& V, int32_t start) {
+  return start < B.F.nf ? V.vf + start : (V2Face*)B.F.rec + (start - B.F.nf);
+}
+__device__ __forceinline__ V2Over* v_over(const Batch& B, const SimDesc& D) { return (V2Over*)(B.F.fs + 4 * D.face_base); }
 
 // The finished cell: area and centroid summed over the edges in order (the host tessellator's
 // Cell2::finish), the emitted faces appended to vf in edge order, and the cell's geometry
@@ -265,7 +270,7 @@ __device__ void v2_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, Sim
   }
   V.vst[gi] = start;
   V.femit[gi] = cnt;
-  V2Face* out = V.vf + start;
+  V2Face* out = v_faces_at(B, V, start);
   int q = 0;
   for (int k = 0; k < m; ++k) {
     const int km = k == 0 ? m - 1 : k - 1;
@@ -827,7 +832,7 @@ __device__ __forceinline__ void v2_reg_finish(const Batch& B, const V2Bufs& V, c
     f.nz = 0.;
     f.nb = P.nb < 0 ? -1 : P.nb;
     f.code = P.code;
-    V.vf[start + __popc(em & ((1u << lane) - 1u))] = f;
+    v_faces_at(B, V, start)[__popc(em & ((1u << lane) - 1u))] = f;
   }
   if (lane != 0) return;
   V.vst[gi] = start;
@@ -936,7 +941,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
       if (offs[lo + h] <= t) lo += h;
     const int64_t gi = (int64_t)J.lo + lo;
     const int64_t f = D.face_base + base + t;
-    const V2Face r = V.vf[starts[lo] + (t - offs[lo])];
+    const V2Face r = v_faces_at(B, V, starts[lo])[t - offs[lo]];
     F.area[f] = r.area;
     F.nrm[f] = r.nx;
     F.nrm[NF + f] = r.ny;
@@ -955,7 +960,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
         return;
       }
       const int32_t o = atomicAdd(&S.n_over, 1);
-      if (o < D.conn_cap) V.over[D.conn_base + o] = V2Over{conn, nbr, atomicExch(&V.gkey[cell], o)};  // (more: refused)
+      if (o < 2 * D.face_cap) v_over(B, D)[o] = V2Over{conn, nbr, atomicExch(&V.gkey[cell], o)};
     };
     put((int32_t)gi, (int32_t)(f << 1), right);
     if (right >= 0) put(right, (int32_t)((f << 1) | 1), (int32_t)gi);
@@ -1033,7 +1038,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_conn(Batch B, V2Bufs V) {
     insert(at, (int32_t)(w >> 32), (int32_t)(uint32_t)w);
   }
   for (int32_t o = V.gkey[gi]; o >= 0;) {
-    const V2Over w = V.over[D.conn_base + o];
+    const V2Over w = v_over(B, D)[o];
     insert(at++, w.conn, w.nbr);
     o = w.next;
   }

@@ -847,7 +847,7 @@ __device__ int v3_finish(const Batch& B, const V2Bufs& V, const SimDesc& D, SimS
     f.nz = inv * C.pz[p];
     f.nb = pnb < 0 ? -1 : pnb;
     f.code = C.pcode[p];
-    V.vf[start + __popcll(me & ((1ull << lane) - 1ull))] = f;
+    v_faces_at(B, V, start)[__popcll(me & ((1ull << lane) - 1ull))] = f;
   }
   wave_sync();
   if (lane != 0) return 0;
@@ -1369,7 +1369,7 @@ __device__ __forceinline__ int v3r_finish(const Batch& B, const V2Bufs& V, const
     o.nz = inv * C.pz[p];
     o.nb = pnb < 0 ? -1 : pnb;
     o.code = C.pcode[p];
-    V.vf[start + __popcll(me & ((1ull << lane) - 1ull))] = o;
+    v_faces_at(B, V, start)[__popcll(me & ((1ull << lane) - 1ull))] = o;
   }
   wave_sync();
   // the cell's volume and centroid: the tetrahedron terms added in the host's order, one sum a lane
