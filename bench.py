@@ -175,7 +175,7 @@ def summarize_pmc(fetch_dir, write_dir, copy_fetch_dir, copy_write_dir, label, c
     for k, v in sorted(table.items(), key=lambda kv: -kv[1]["traffic_bytes"]):
         lines.append(f"| `{k}` | {v['dispatches']} | {v['fetch_bytes'] / 1e6:.1f} | {v['write_bytes'] / 1e6:.1f} | "
                      f"{v['traffic_bytes'] / 1e6:.1f} |")
-    lines += ["", "TRAFFIC_JSON " + json.dumps({"label": label, "kernels": table})]
+    lines += ["", "TRAFFIC_JSON " + json.dumps({"label": label, "kernels_id": kernels_id(), "kernels": table})]
     out = os.path.join(PROFILES, f"{label}_pmc.md")
     open(out, "w").write("\n".join(lines) + "\n")
     return out
@@ -221,14 +221,28 @@ def summarize_trace(stats_csv, label, command, note="", trace_csv=None, window=0
     return out
 
 
+def kernels_id():
+    """Identity of the device sources apart from their comments and white space: what a profile is of."""
+    import glob
+    import hashlib
+    import re
+
+    h = hashlib.sha256()
+    for path in sorted(glob.glob(os.path.join(ROOT, "hydro_rs_amd", "csrc", "*.h*"))):
+        h.update("".join(re.sub(r"//.*", "", open(path).read()).split()).encode())
+    return h.hexdigest()[:16]
+
+
 def traffic_for(label, kernel_name):
-    """HBM bytes per dispatch of kernel_name from profiles/<label>_pmc.md (None when not profiled)."""
+    """HBM bytes per dispatch of kernel_name from profiles/<label>_pmc.md (None when not profiled, or when the record is
+    of other kernels than the present ones)."""
     path = os.path.join(PROFILES, f"{label}_pmc.md")
     if not os.path.exists(path):
         return None
     for line in open(path):
         if line.startswith("TRAFFIC_JSON "):
-            rec = json.loads(line[len("TRAFFIC_JSON "):]).get("kernels", {}).get(kernel_name)
+            doc = json.loads(line[len("TRAFFIC_JSON "):])
+            rec = doc["kernels"].get(kernel_name) if doc.get("kernels_id") == kernels_id() else None
             return rec["traffic_bytes"] if rec else None
     return None
 
@@ -239,7 +253,7 @@ def flux_kernel_name(fp32, solver, static_geometry=True, fpt=1):
             f"{'true' if static_geometry else 'false'}, {fpt or 1}>(hfv::Batch)")
 
 
-SLOT_KERNELS = {"apply_c2p": ["hfv::k_apply(hfv::Batch, int)"], "mask_predict": ["void hfv::k_mask<false>(hfv::Batch, int)"],
+SLOT_KERNELS = {"apply_c2p": ["hfv::k_apply(hfv::Batch, int)"], "mask_predict": ["void hfv::k_mask<false>(hfv::Batch, hfv::V2Bufs, int)"],
                 "wakeup": ["hfv::k_sync_min(hfv::Batch)"], "limit_kick": ["hfv::k_limit(hfv::Batch, int)"]}
 
 
