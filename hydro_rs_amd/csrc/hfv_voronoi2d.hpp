@@ -207,7 +207,6 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_place(Batch B, V2Bufs V) {
 #define HFV_V2_TEAM 16
 #define HFV_V2_TLW 48
 #define HFV_V2_CAP 96           // 3 blocks a CU; a 9 x 9-bin block (K = 4) at one generator per bin mostly fits
-#define HFV_V2_OWN (HFV_V2_CAP / HFV_V2_TEAM)
 #define HFV_V2_SUB HFV_V2_TEAM  // blocks per cell chunk
 
 template <int TL>
@@ -935,7 +934,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
   if (bad) return;
   const Faces& F = B.F;
   for (int32_t t = threadIdx.x; t < tot; t += HFV_BLOCK) {
-    int lo = 0;  // the last cell whose offset is <= t (later cells of the same offset emit nothing)
+    int lo = 0;  // the last cell whose offset is <= t (earlier cells of the same offset emit nothing)
 #pragma unroll
     for (int h = HFV_BLOCK / 2; h > 0; h >>= 1)
       if (offs[lo + h] <= t) lo += h;

@@ -333,8 +333,10 @@ typedef struct {
 } hfv_tune_class;
 int hfv_autotune(hfv_ctx* ctx, int launches, int rounds, hfv_tune_class* out, int max_out, int* n_out);
 /* The same choices for one slot by hand: staged 1/0 (-1: by dimension, on for 2D and 3D, the
- * default), static_grad and gstaged 1/0 (-1: by dimension, on for 3D, the default).  They take effect for static-geometry
- * simulations only; hfv_get_tuning reports what a slot currently runs. */
+ * default), static_grad and gstaged 1/0 (-1: by dimension, on for 3D, the default).  They take effect for
+ * static-geometry simulations only, and static_grad = 1 only where the mesh fits its slot's precomputed geometry
+ * (1.5 entries for each CSR entry of the slot's capacity: every 64 cells take 64 times their longest CSR row);
+ * hfv_get_tuning reports what a slot currently runs. */
 int hfv_set_tuning(hfv_ctx* ctx, int slot, int staged, int static_grad, int gstaged);
 int hfv_get_tuning(hfv_ctx* ctx, int slot, int* staged, int* static_grad, int* gstaged);
 /* The flux kernel's launch shape for the whole context: face chunks per thread block, i.e. faces per
