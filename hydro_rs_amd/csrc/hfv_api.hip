@@ -1165,14 +1165,13 @@ void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
     hipLaunchKernelGGL(k_mesh1d_cells, gc, gb, 0, st, B);
   }
   if (c->any_vmesh) {
-    V2Bufs V = c->v2;
-    V.scanned = c->vscan ? 1 : 0;
+    const V2Bufs& V = c->v2;
     auto prefix = [&](int k) {
       if (c->vscan) hipLaunchKernelGGL(k_v2_prefix, dim3((unsigned)c->nslots), dim3(HFV_PREFIX_BLOCK), 0, st, B, V, k);
     };
     hipLaunchKernelGGL(k_v2_sum<0>, gc, gb, 0, st, B, V);
     prefix(0);
-    hipLaunchKernelGGL(k_v2_bins, gc, gb, 0, st, B, V);
+    hipLaunchKernelGGL(c->vscan ? k_v2_bins<true> : k_v2_bins<false>, gc, gb, 0, st, B, V);
     hipLaunchKernelGGL(k_v2_place, gc, gb, 0, st, B, V);
     if (c->any_vmesh2) hipLaunchKernelGGL(k_v2_cells, dim3((unsigned)(c->ncg * HFV_V2_SUB)), gb, 0, st, B, V);
     if (c->any_vmesh3) {
@@ -1180,10 +1179,10 @@ void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
       hipLaunchKernelGGL(k_v3_cells, dim3((unsigned)(c->ncg << c->v3sub)), dim3(64), 0, st, B, V, c->v3sub);
     }
     prefix(1);
-    hipLaunchKernelGGL(k_v2_faces, gc, gb, 0, st, B, V);
+    hipLaunchKernelGGL(c->vscan ? k_v2_faces<true> : k_v2_faces<false>, gc, gb, 0, st, B, V);
     hipLaunchKernelGGL(k_v2_sum<1>, gc, gb, 0, st, B, V);
     prefix(2);
-    hipLaunchKernelGGL(k_v2_conn, gc, gb, 0, st, B, V);
+    hipLaunchKernelGGL(c->vscan ? k_v2_conn<true> : k_v2_conn<false>, gc, gb, 0, st, B, V);
   }
 }
 

@@ -974,10 +974,9 @@ struct V2Bufs {
   V2Face* vf;
   uint64_t* bkt;   // [HFV_BUCKET][N] entries of a cell: (CSR value << 32) | neighbour
   // [cell chunks] sums over the chunk's bins of gcnt, over its cells of femit (their cursors while they are built)
-  // and of ccnt
+  // and of ccnt; of large meshes (SCANNED), once k_v2_prefix has run, those of the chunks before
   int32_t* part[3];
   int32_t* ptot;   // [S][3] the totals where part is scanned
-  int scanned;     // part holds the sums of the chunks before (k_v2_prefix)
 };
 
 __device__ __forceinline__ int v2_bin(double x, double w, int nb) {

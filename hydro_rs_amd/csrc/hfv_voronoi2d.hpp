@@ -74,10 +74,11 @@ __device__ __forceinline__ int32_t block_excl_scan(int32_t v, int32_t* total) {
 // The sum of the simulation's chunk sums (array k of V.part) before chunk `chunk`, and of all of them (every thread
 // gets both).  Each block reads every chunk sum: at most a few thousand words that the L2 holds, where a launch of
 // its own to scan them costs 4-5 us.  Meshes of more chunks have them scanned (k_v2_prefix).
+template <bool SCANNED>
 __device__ __forceinline__ int32_t chunks_before(const V2Bufs& V, int k, const SimDesc& D, int s, int32_t chunk,
                                                  int32_t* total) {
   const int32_t* part = V.part[k];
-  if (V.scanned) {
+  if (SCANNED) {
     *total = V.ptot[3 * s + k];
     return part[chunk];
   }
@@ -159,6 +160,7 @@ __global__ void __launch_bounds__(HFV_PREFIX_BLOCK) k_v2_prefix(Batch B, V2Bufs 
 }
 
 // Bin starts and placement cursors; the chunk sums of the emitted faces restart at zero.
+template <bool SCANNED>
 __global__ void __launch_bounds__(HFV_BLOCK) k_v2_bins(Batch B, V2Bufs V) {
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
@@ -171,7 +173,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_bins(Batch B, V2Bufs V) {
   int32_t* a = V.gcnt + D.cell_base + s;
   const int32_t v = k < nbins ? a[k] : 0;
   int32_t all, tot;
-  const int32_t base = chunks_before(V, 0, D, s, J.chunk, &all);
+  const int32_t base = chunks_before<SCANNED>(V, 0, D, s, J.chunk, &all);
   const int32_t x = base + block_excl_scan(v, &tot);
   if (k < nbins) {
     a[k] = x;
@@ -189,6 +191,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_place(Batch B, V2Bufs V) {
   const int64_t gi = (int64_t)J.lo + threadIdx.x;
   if (gi >= J.hi) return;
   const int32_t p = atomicAdd(&V.gfill[D.cell_base + s + V.gkey[gi]], 1);
+  V.gkey[gi] = -1;  // (no chained entries yet)
   V.gord[D.cell_base + p] = (int32_t)(gi - D.cell_base);
 }
 
@@ -235,7 +238,8 @@ __device__ __forceinline__ int32_t v_place_faces(const Batch& B, const V2Bufs& V
 }
 
 __device__ __forceinline__ V2Face* v_faces_at(const Batch& B, const V2Bufs& V, int32_t start) {
-  return start < B.F.nf ? V.vf + start : (V2Face*)B.F.rec + (start - B.F.nf);
+  const int32_t nf = (int32_t)B.F.nf;  // (below 2^30: CSR values hold a face and a side)
+  return start < nf ? V.vf + (uint32_t)start : (V2Face*)B.F.rec + (uint32_t)(start - nf);
 }
 __device__ __forceinline__ V2Over* v_over(const Batch& B, const SimDesc& D) { return (V2Over*)(B.F.fs + 4 * D.face_base); }
 
@@ -865,10 +869,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_cells(Batch B, V2Bufs V) {
   if (gi >= J.hi) return;  // whole teams; no block barrier follows
   const int64_t N = B.C.n, cb = D.cell_base;
   const int32_t i = (int32_t)(gi - cb);
-  if (lane == 0) {
-    V.ccnt[gi] = 0;
-    V.gkey[gi] = -1;
-  }
+  if (lane == 0) V.ccnt[gi] = 0;
   if (!B.C.act[gi]) {  // unbuilt in a partial build
     if (lane == 0) V.femit[gi] = 0;
     return;
@@ -906,6 +907,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_cells(Batch B, V2Bufs V) {
 // The faces of a chunk's cells, in cell order after the faces of the chunks before: face arrays, and the
 // entries of both cells into their buckets.  The block's threads take its faces in turn, whichever cell
 // emitted them (a binary search of the cells' offsets in LDS).
+template <bool SCANNED>
 __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
   __shared__ int32_t offs[HFV_BLOCK], starts[HFV_BLOCK];
   const BlockJob J = B.cjobs[blockIdx.x];
@@ -918,7 +920,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
   const int64_t gi0 = (int64_t)J.lo + threadIdx.x;
   const bool in = gi0 < J.hi;
   int32_t all, tot;
-  const int32_t base = chunks_before(V, 1, D, s, J.chunk, &all);
+  const int32_t base = chunks_before<SCANNED>(V, 1, D, s, J.chunk, &all);
   offs[threadIdx.x] = block_excl_scan(in ? V.femit[gi0] : 0, &tot);
   starts[threadIdx.x] = in ? V.vst[gi0] : 0;
   const bool full = all > D.face_cap;
@@ -968,6 +970,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
 
 // CSR offsets, and every cell's entries in ascending face order (then side): CSR values are distinct and
 // non-negative, so the packed words order as they do.  The bin counts restart at zero.
+template <bool SCANNED>
 __global__ void __launch_bounds__(HFV_BLOCK) k_v2_conn(Batch B, V2Bufs V) {
   __shared__ uint64_t ent[HFV_BUCKET][HFV_BLOCK];  // [slot][thread]
   const BlockJob J = B.cjobs[blockIdx.x];
@@ -982,7 +985,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_conn(Batch B, V2Bufs V) {
   if (bin < (int64_t)D.vnb[0] * D.vnb[1] * D.vnb[2]) V.gcnt[D.cell_base + s + bin] = 0;
   const int m = in ? V.ccnt[gi] : 0;
   int32_t all, tot;
-  const int32_t base = chunks_before(V, 2, D, s, J.chunk, &all);
+  const int32_t base = chunks_before<SCANNED>(V, 2, D, s, J.chunk, &all);
   const int32_t x = base + block_excl_scan(m, &tot);
   const bool full = all > D.conn_cap;
   const bool bad = full || S.err != 0;

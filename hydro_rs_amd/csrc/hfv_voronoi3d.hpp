@@ -1405,10 +1405,7 @@ __global__ void __launch_bounds__(256, 4) k_v3_cells_reg(Batch B, V2Bufs V) {
   const int64_t gi = (int64_t)J.lo + (blockIdx.x % HFV_V3R_SUB) * 4 + wave;
   if (gi >= J.hi) return;  // (no block barrier follows)
   const int lane = __lane_id();
-  if (lane == 0) {
-    V.ccnt[gi] = 0;
-    V.gkey[gi] = -1;
-  }
+  if (lane == 0) V.ccnt[gi] = 0;
   if (!B.C.act[gi]) {  // unbuilt in a partial build
     if (lane == 0) V.femit[gi] = 0;
     return;
