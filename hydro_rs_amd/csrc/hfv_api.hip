@@ -190,7 +190,9 @@ struct hfv_ctx {
   int cgsh = 0, fgsh = 0;     // log2 of the group sizes that the tables were dealt in
   int64_t face_items = 0;     // faces that the only simulation's face kernels cover
   bool vscan = false;         // the rebuild's chunk sums are scanned (kScanChunks)
-  int v3sub = 0;              // log2 of k_v3_cells' blocks per cell chunk
+  std::vector<int32_t> hv3;   // live slots with a 3D moving mesh, and k_v3_cells' blocks for each
+  int32_t* dv3 = nullptr;
+  int v3per = 0;
   std::vector<BlockJob> hcjobs, hfjobs;
   BlockJob *dcjobs = nullptr, *dfjobs = nullptr;
   Partials P{};
@@ -374,25 +376,22 @@ int64_t face_range(const hfv_ctx* c, int s) { return c->desc[s].vmesh ? c->fcap[
 // 262,144 (1024 chunks; the scans 14), 498 / 457 on 10^6 (3906; the scans 20), 2131 / 1676 on 4 x 10^6 (the scans 54).
 constexpr int64_t kScanChunks = 2048;
 
-// log2 of the blocks per cell chunk that k_v3_cells launches for `chunks` chunks of 3D moving meshes: together some
-// 4096, a few more than the chip holds at once (10 a CU by LDS), as long as a block stays at 2 cells or more.
-int v3_sub(int64_t chunks) {
-  int sub = 0;
-  while (sub < 7 && chunks << (sub + 1) <= 4096) ++sub;
-  return sub;
-}
-
 // Rebuild the block tables from the live slots (loaded, and in a batch not finished: a finished slot's
 // blocks would only exit) and upload them with the simulation descriptors.  Chunk ids (partials) stay
 // global.
 int write_jobs(hfv_ctx* c) {
   const int S = c->nslots;
   auto live = [&](int s) { return c->loaded[s] && !(c->batch && c->heng[s].done); };
-  int64_t lc = 0, lf = 0, l3 = 0, lv = 0;  // (l3: of 3D moving meshes, lv: of the largest moving mesh)
+  int64_t lc = 0, lf = 0, lv = 0, lv3 = 0;  // (lv, lv3: of the largest moving mesh, the largest 3D one)
+  const size_t n3 = c->hv3.size();
+  c->hv3.clear();
   for (int s = 0; s < S; ++s) {
     if (!live(s)) continue;
     if (c->desc[s].vmesh) lv = std::max<int64_t>(lv, (c->nused[s] + BLOCK - 1) / BLOCK);
-    if (c->desc[s].vmesh == 3) l3 += (c->nused[s] + BLOCK - 1) / BLOCK;
+    if (c->desc[s].vmesh == 3) {
+      lv3 = std::max<int64_t>(lv3, (c->nused[s] + BLOCK - 1) / BLOCK);
+      c->hv3.push_back(s);
+    }
     lc += (c->nused[s] + BLOCK - 1) / BLOCK;
     lf += (face_range(c, s) + BLOCK - 1) / BLOCK;
   }
@@ -402,10 +401,12 @@ int write_jobs(hfv_ctx* c) {
   const int cgsh = __builtin_ctzll((uint64_t)gc), fgsh = __builtin_ctzll((uint64_t)gf);
   const int64_t items = c->batch || !c->loaded[0] ? 0 : face_range(c, 0);
   if (cgsh != c->cgsh || fgsh != c->fgsh || items != c->face_items) drop_graph(c);
-  const int v3sub = v3_sub(l3);
+  // k_v3_cells: together some 4096 one-wave blocks, a few more than the chip holds at once (10 a CU by LDS), as long
+  // as a block stays at 2 cells or more
+  const int v3per = c->hv3.empty() ? 0 : (int)std::min<int64_t>(std::max<int64_t>(4096 / (int64_t)c->hv3.size(), 32), 128 * lv3);
   const bool vscan = lv > kScanChunks;
-  if (v3sub != c->v3sub || vscan != c->vscan) drop_graph(c);
-  c->v3sub = v3sub;
+  if (v3per != c->v3per || n3 != c->hv3.size() || vscan != c->vscan) drop_graph(c);
+  c->v3per = v3per;
   c->vscan = vscan;
   c->cgsh = cgsh;
   c->fgsh = fgsh;
@@ -441,6 +442,8 @@ int write_jobs(hfv_ctx* c) {
   hipStream_t st = c->stream;
   HIP_OK(hipMemcpyAsync(c->dcjobs, c->hcjobs.data(), sizeof(BlockJob) * c->ncpos, hipMemcpyHostToDevice, st));
   HIP_OK(hipMemcpyAsync(c->dfjobs, c->hfjobs.data(), sizeof(BlockJob) * c->nfpos, hipMemcpyHostToDevice, st));
+  if (!c->hv3.empty())
+    HIP_OK(hipMemcpyAsync(c->dv3, c->hv3.data(), sizeof(int32_t) * c->hv3.size(), hipMemcpyHostToDevice, st));
   HIP_OK(hipMemcpyAsync(c->ddesc, c->desc.data(), sizeof(SimDesc) * S, hipMemcpyHostToDevice, st));
   HIP_OK(hipStreamSynchronize(st));
   return HFV_OK;
@@ -565,6 +568,8 @@ int alloc_batch(hfv_ctx* c) {
   c->ddesc = dalloc<SimDesc>(c, S);
   c->deng = dalloc<SimEngine>(c, S);
   c->dst = dalloc<SimStep>(c, S);
+  c->dv3 = dalloc<int32_t>(c, S);
+  c->hv3.clear();
   for (void* p : c->bufs)
     if (!p) return set_err(HFV_ERR_HIP, "hipMalloc failed");
   hipStream_t st = c->stream;
@@ -1176,7 +1181,8 @@ void enqueue_rebuild(hfv_ctx* c, const Batch& B) {
     if (c->any_vmesh2) hipLaunchKernelGGL(k_v2_cells, dim3((unsigned)(c->ncg * HFV_V2_SUB)), gb, 0, st, B, V);
     if (c->any_vmesh3) {
       hipLaunchKernelGGL(k_v3_cells_reg, dim3((unsigned)(c->ncg * HFV_V3R_SUB)), dim3(256), 0, st, B, V);
-      hipLaunchKernelGGL(k_v3_cells, dim3((unsigned)(c->ncg << c->v3sub)), dim3(64), 0, st, B, V, c->v3sub);
+      if (c->v3per)
+        hipLaunchKernelGGL(k_v3_cells, dim3((unsigned)(c->hv3.size() * c->v3per)), dim3(64), 0, st, B, V, c->dv3, c->v3per);
     }
     prefix(1);
     hipLaunchKernelGGL(c->vscan ? k_v2_faces<true> : k_v2_faces<false>, gc, gb, 0, st, B, V);

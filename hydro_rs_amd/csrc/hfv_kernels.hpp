@@ -970,7 +970,9 @@ struct V2Bufs {
   int32_t* vst;    // [N] start of a cell's faces in vf
   int32_t* ccnt;   // [N] CSR entries per cell
   // [F] faces in provisional order, the chunks' shares at face_base.  Faces beyond their chunk's share go to the place
-  // of the simulation's flux records (F.rec), dead between the accumulation and the next fluxes.
+  // of the simulation's flux records (F.rec), dead between the accumulation and the next fluxes in every
+  // simulation of the batch, as all step in the same launches.  (FP32 records are half as long, so that this may be
+  // another slot's; the host reads those of slot 0 only, which lie before every other slot's place.)
   V2Face* vf;
   uint64_t* bkt;   // [HFV_BUCKET][N] entries of a cell: (CSR value << 32) | neighbour
   // [cell chunks] sums over the chunk's bins of gcnt, over its cells of femit (their cursors while they are built)

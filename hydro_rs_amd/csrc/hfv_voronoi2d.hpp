@@ -25,9 +25,9 @@
 //   k_v2_sum<1>, k_v2_conn      CSR offsets; the entries in ascending face order
 // Each prefix sum over cells (or bins) is two levels: a kernel before leaves the sums of the chunks of
 // HFV_BLOCK elements, and every block of the kernel that needs the sum adds up the chunks before its own
-// (chunks_before; on large meshes k_v2_prefix has scanned them) and scans its chunk.  The rebuild was 18 launches of 4-5 us each (counts, sums,
-// scans, fill and sort apart) and is 7 in 2D: a 125^2 vortex with steered generators 218 -> 202 us a step,
-// a Sedov 256^2 run to t = 0.004 121 -> 111.5 ms.
+// (chunks_before; on large meshes k_v2_prefix has scanned them) and scans its chunk.  The rebuild was 18
+// launches of 4-5 us each (counts, sums, scans, fill and sort apart) and is 7 in 2D: a 125^2 vortex with
+// steered generators 218 -> 202 us a step, a Sedov 256^2 run to t = 0.004 121 -> 111.5 ms.
 // Inactive cells keep their geometry and get new CSR ranges (the reference's note at space.rs:233-235).
 #pragma once
 

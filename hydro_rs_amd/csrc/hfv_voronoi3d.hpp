@@ -1430,25 +1430,23 @@ __global__ void __launch_bounds__(256, 4) k_v3_cells_reg(Batch B, V2Bufs V) {
 }
 
 // The cells that k_v3_cells_reg left, from the list of their simulation (in gfill, whose placement cursors are
-// used up): its 1 << sub one-wavefront blocks per cell chunk take entries in turn, so that they have equal shares
-// wherever the cells lie.  Blocks that looked through 32 cells each and built those left among them had a clump's
+// used up): the `per` one-wavefront blocks of each of the slots take its entries in turn, so that they have equal
+// shares wherever the cells lie.  Blocks that looked through 32 cells each and built those left among them had a clump's
 // cells to build one after another.  With fully active steps, a step of clumped generators (times for a wave per
 // cell, those blocks, the list): 2000 cells, three quarters of them in a cube of 0.4: 2.70, 21.3, 2.20 ms; 8000
 // alike: 5.51, 33.1, 3.41; 64,000, half of them in a cube of 0.5: 3.93, 10.35, 3.66; 64,000 uniform: 3.90, 3.10, 2.77;
 // the KH lattice of 48^3: 2.89, 1.97, 1.95.
-__global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V, int sub) {
+__global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V, const int32_t* slots, int per) {
   __shared__ V3Cell C;
-  const BlockJob J = B.cjobs[blockIdx.x >> sub];
-  if (J.sim < 0) return;
-  const int s = J.sim;
+  const int s = slots[blockIdx.x / (uint32_t)per];
   const SimDesc& D = B.sims[s];
   SimStep& S = B.st[s];
   if (D.vmesh != 3 || !S.stepping) return;
   const int lane = __lane_id();
   const int64_t N = B.C.n, cb = D.cell_base;
   const int kmax = max(6, max(D.vnb[0], max(D.vnb[1], D.vnb[2])));
-  const int32_t n = S.n_left, step = (D.cchunk1 - D.cchunk0) << sub;
-  for (int32_t q = ((J.chunk - D.cchunk0) << sub) + (int32_t)(blockIdx.x & ((1u << sub) - 1u)); q < n; q += step) {
+  const int32_t n = S.n_left;
+  for (int32_t q = (int32_t)(blockIdx.x % (uint32_t)per); q < n; q += per) {
     const int32_t i = V.gfill[cb + s + q];
     const int64_t gi = cb + i;
     const double xi = B.C.loc[gi], yi = B.C.loc[N + gi], zi = B.C.loc[2 * N + gi];
