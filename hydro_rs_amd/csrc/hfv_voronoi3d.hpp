@@ -1433,8 +1433,8 @@ __global__ void __launch_bounds__(256, 4) k_v3_cells_reg(Batch B, V2Bufs V) {
 // used up): the `per` one-wavefront blocks of each of the slots take its entries in turn, so that they have equal
 // shares wherever the cells lie.  Blocks that looked through 32 cells each and built those left among them had a clump's
 // cells to build one after another.  With fully active steps, a step of clumped generators (times for a wave per
-// cell, those blocks, the list): 2000 cells, three quarters of them in a cube of 0.4: 2.70, 21.3, 2.20 ms; 8000
-// alike: 5.51, 33.1, 3.41; 64,000, half of them in a cube of 0.5: 3.93, 10.35, 3.66; 64,000 uniform: 3.90, 3.10, 2.77;
+// cell, those blocks, the list): 2000 cells, three quarters of them in a cube of 0.4: 2.70, 21.3, 2.19 ms; 8000
+// alike: 5.51, 33.1, 3.37; 64,000, half of them in a cube of 0.5: 3.93, 10.35, 3.55; 64,000 uniform: 3.90, 3.10, 2.63;
 // the KH lattice of 48^3: 2.89, 1.97, 1.95.
 __global__ void __launch_bounds__(64) k_v3_cells(Batch B, V2Bufs V, const int32_t* slots, int per) {
   __shared__ V3Cell C;
