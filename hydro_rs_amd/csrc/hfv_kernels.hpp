@@ -953,10 +953,11 @@ static_assert(sizeof(V2Face) == 8 * sizeof(double), "a face takes a flux record'
 // CSR entries a cell's bucket holds between k_v2_faces and k_v2_conn (further ones are chained in a list of the
 // simulation): a random 3D mesh has 15.5 faces a cell, one cell in a hundred has more than 24
 #define HFV_BUCKET 24
-// An entry beyond its cell's bucket, and the next one of the cell (-1: none).  A simulation's list (two entries a
-// face at most) has the place of its faces' static geometry (F.fs), which moving meshes have not.
+// An entry beyond its cell's bucket, and the next one of the cell (the last one's is not read: ccnt tells).  A
+// simulation's list (two entries a face at most) has the place of its faces' static geometry (F.fs), which moving
+// meshes have not.
 struct V2Over {
-  int32_t conn, nbr, next;
+  int32_t cell, conn, nbr, next;
 };
 static_assert(2 * sizeof(V2Over) <= 4 * sizeof(double), "both entries of a face in its static geometry's place");
 
@@ -965,7 +966,7 @@ struct V2Bufs {
                    // between the steps
   int32_t* gfill;  // same layout: placement cursors, then (3D) the list of the cells the register builder left
   int32_t* gord;   // [N] at cell_base: local cell indices grouped by bin
-  int32_t* gkey;   // [N] bin of each cell, then the first of its entries in over (-1: none)
+  int32_t* gkey;   // [N] bin of each cell, then the first of its chained entries where it has any
   int32_t* femit;  // [N] faces a cell emits
   int32_t* vst;    // [N] start of a cell's faces in vf
   int32_t* ccnt;   // [N] CSR entries per cell

@@ -111,8 +111,12 @@ __device__ __forceinline__ int32_t chunks_before(const V2Bufs& V, int k, const S
   return b;
 }
 
+// A simulation's entries beyond their cells' buckets.
+__device__ __forceinline__ V2Over* v_over(const Batch& B, const SimDesc& D) { return (V2Over*)(B.F.fs + 4 * D.face_base); }
+
 // Chunk sums of the bin counts (CSR 0) or of the cells' CSR entries (CSR 1).  (Added up by the counting
-// atomics instead, they put hundreds of atomics on one address: 10-100 us.)
+// atomics instead, they put hundreds of atomics on one address: 10-100 us.)  CSR 1 also chains the entries beyond
+// the buckets to their cells.
 template <int CSR>
 __global__ void __launch_bounds__(HFV_BLOCK) k_v2_sum(Batch B, V2Bufs V) {
   const BlockJob J = B.cjobs[blockIdx.x];
@@ -125,6 +129,11 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_sum(Batch B, V2Bufs V) {
   const int32_t* a = CSR ? V.ccnt + D.cell_base : V.gcnt + D.cell_base + s;
   const uint32_t t = block_sum_u32(k < len ? (uint32_t)a[k] : 0u);
   if (threadIdx.x == 0) V.part[CSR ? 2 : 0][J.chunk] = (int32_t)t;
+  if (CSR && k < len) {
+    const int64_t no = min((int64_t)B.st[s].n_over, 2 * D.face_cap);
+    V2Over* over = v_over(B, D);
+    for (int64_t o = k; o < no; o += len) over[o].next = atomicExch(&V.gkey[over[o].cell], (int32_t)o);
+  }
 }
 
 // The chunk sums (array k) of a simulation, scanned in place: one block per simulation.
@@ -191,7 +200,6 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_place(Batch B, V2Bufs V) {
   const int64_t gi = (int64_t)J.lo + threadIdx.x;
   if (gi >= J.hi) return;
   const int32_t p = atomicAdd(&V.gfill[D.cell_base + s + V.gkey[gi]], 1);
-  V.gkey[gi] = -1;  // (no chained entries yet)
   V.gord[D.cell_base + p] = (int32_t)(gi - D.cell_base);
 }
 
@@ -241,7 +249,6 @@ __device__ __forceinline__ V2Face* v_faces_at(const Batch& B, const V2Bufs& V, i
   const int32_t nf = (int32_t)B.F.nf;  // (below 2^30: CSR values hold a face and a side)
   return start < nf ? V.vf + (uint32_t)start : (V2Face*)B.F.rec + (uint32_t)(start - nf);
 }
-__device__ __forceinline__ V2Over* v_over(const Batch& B, const SimDesc& D) { return (V2Over*)(B.F.fs + 4 * D.face_base); }
 
 // The finished cell: area and centroid summed over the edges in order (the host tessellator's
 // Cell2::finish), the emitted faces appended to vf in edge order, and the cell's geometry
@@ -907,9 +914,12 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_cells(Batch B, V2Bufs V) {
 // The faces of a chunk's cells, in cell order after the faces of the chunks before: face arrays, and the
 // entries of both cells into their buckets.  The block's threads take its faces in turn, whichever cell
 // emitted them (a binary search of the cells' offsets in LDS).
+// (Chaining the entries beyond the buckets here, and telling the two places of provisional faces apart for each
+// face instead of each cell, this kernel took 19.3 us instead of 18.3 on a 125^2 vortex.)
 template <bool SCANNED>
 __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
-  __shared__ int32_t offs[HFV_BLOCK], starts[HFV_BLOCK];
+  __shared__ int32_t offs[HFV_BLOCK];
+  __shared__ const V2Face* starts[HFV_BLOCK];
   const BlockJob J = B.cjobs[blockIdx.x];
   if (J.sim < 0) return;
   const int s = J.sim;
@@ -922,7 +932,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
   int32_t all, tot;
   const int32_t base = chunks_before<SCANNED>(V, 1, D, s, J.chunk, &all);
   offs[threadIdx.x] = block_excl_scan(in ? V.femit[gi0] : 0, &tot);
-  starts[threadIdx.x] = in ? V.vst[gi0] : 0;
+  starts[threadIdx.x] = v_faces_at(B, V, in ? V.vst[gi0] : 0);
   const bool full = all > D.face_cap;
   const bool bad = full || S.err != 0;  // a failed cell emitted nothing: the simulation stops
   if (J.chunk == D.cchunk0 && threadIdx.x == 0) {
@@ -942,7 +952,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
       if (offs[lo + h] <= t) lo += h;
     const int64_t gi = (int64_t)J.lo + lo;
     const int64_t f = D.face_base + base + t;
-    const V2Face r = v_faces_at(B, V, starts[lo])[t - offs[lo]];
+    const V2Face r = starts[lo][t - offs[lo]];
     F.area[f] = r.area;
     F.nrm[f] = r.nx;
     F.nrm[NF + f] = r.ny;
@@ -961,7 +971,7 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_faces(Batch B, V2Bufs V) {
         return;
       }
       const int32_t o = atomicAdd(&S.n_over, 1);
-      if (o < 2 * D.face_cap) v_over(B, D)[o] = V2Over{conn, nbr, atomicExch(&V.gkey[cell], o)};
+      if (o < 2 * D.face_cap) v_over(B, D)[o] = V2Over{cell, conn, nbr, -1};
     };
     put((int32_t)gi, (int32_t)(f << 1), right);
     if (right >= 0) put(right, (int32_t)((f << 1) | 1), (int32_t)gi);
@@ -1004,7 +1014,14 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_conn(Batch B, V2Bufs V) {
   int32_t* nb = B.F.nbr;
   if (m <= HFV_BUCKET) {
     uint64_t* v = &ent[0][threadIdx.x];
-    for (int k = 0; k < m; ++k) v[k * HFV_BLOCK] = V.bkt[(int64_t)k * N + gi];
+    for (int k = 0; k < m; k += 4) {  // (four loads in flight)
+      uint64_t w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = k + u < m ? V.bkt[(int64_t)(k + u) * N + gi] : 0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (k + u < m) v[(k + u) * HFV_BLOCK] = w[u];
+    }
     for (int k = 1; k < m; ++k) {
       const uint64_t w = v[k * HFV_BLOCK];
       int j = k - 1;
@@ -1021,10 +1038,22 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_conn(Batch B, V2Bufs V) {
     }
     return;
   }
-  // more than the bucket holds: its entries and those chained behind them, sorted in place in memory (as one list of
-  // the simulation that every such cell searched, this kernel took 773 us on 262,144 random 3D generators and 5450 on
-  // 10^6; chained 224 and 639)
-  auto insert = [&](int32_t at, int32_t conn, int32_t nbr) {
+  // more than the bucket holds: its entries and those that k_v2_sum chained to it, sorted in place in memory (with every
+  // such cell searching the simulation's whole list, this kernel took 763 us on 262,144 random 3D generators and 5460
+  // on 10^6; chained 237 and 682)
+  int32_t o = 0;
+  for (int32_t at = 0; at < m; ++at) {
+    int32_t conn, nbr;
+    if (at < HFV_BUCKET) {
+      const uint64_t w = V.bkt[(int64_t)at * N + gi];
+      conn = (int32_t)(w >> 32);
+      nbr = (int32_t)(uint32_t)w;
+    } else {
+      const V2Over w = v_over(B, D)[at == HFV_BUCKET ? V.gkey[gi] : o];
+      conn = w.conn;
+      nbr = w.nbr;
+      o = w.next;
+    }
     int32_t j = e0 + at - 1;
     while (j >= e0 && c[j] > conn) {
       c[j + 1] = c[j];
@@ -1033,16 +1062,6 @@ __global__ void __launch_bounds__(HFV_BLOCK) k_v2_conn(Batch B, V2Bufs V) {
     }
     c[j + 1] = conn;
     nb[j + 1] = nbr;
-  };
-  int32_t at = 0;
-  for (; at < HFV_BUCKET; ++at) {
-    const uint64_t w = V.bkt[(int64_t)at * N + gi];
-    insert(at, (int32_t)(w >> 32), (int32_t)(uint32_t)w);
-  }
-  for (int32_t o = V.gkey[gi]; o >= 0;) {
-    const V2Over w = v_over(B, D)[o];
-    insert(at++, w.conn, w.nbr);
-    o = w.next;
   }
 }
 
